@@ -367,8 +367,8 @@ typedef struct twg_collapse_desc {
  * its "real update" (src/tetwild/EdgeCollapser.cpp:284-446) -- boundary and
  * surface point envelope of v2, isFlip and calTetQualities of the new tets,
  * getCheckQuality / isBetterOrEqualThan, isCollapsable_epsilon -- with the
- * reference's return code.  The one-ring checks run in one persistent launch
- * (tile = 16, 32 or 64 lanes per candidate, chunk = candidates per queue pop;
+ * reference's return code.  The one-ring checks run in one launch
+ * (tile = 16, 32 or 64 lanes per candidate, chunk = candidates per tile;
  * 0 = tuned or default).  Codes and new_q are identical to the CPU
  * restatement for any tile and chunk.  precision TWG_MIXED walks the envelope
  * trees with FP32 boxes (identical decisions).  new_q is complete when the

@@ -72,12 +72,10 @@ struct CollapseArgs {
     double* __restrict__ new_q;
     unsigned* __restrict__ work;
     int32_t* __restrict__ tri_cand;
-    unsigned* counter;     // [0] the ring pass's queue, [kExactCount] exact-list length
+    unsigned* counter;     // exact-list length
     int32_t* exact_list;   // candidates the ring pass left to the exact pass
-    unsigned chunk;        // candidates per queue pop
+    unsigned chunk;        // consecutive candidates per tile
 };
-
-constexpr int kExactCount = 16;  // counter slot (64 bytes after the queue)
 
 __device__ __forceinline__ V3<double> vtx(const CollapseArgs& A, int id)
 {
@@ -202,7 +200,7 @@ __device__ void ring_candidate_fused(const CollapseArgs& A, int64_t c, int tl, i
         A.status[c] = st;
         A.work[c] = work;
         if (!EXACT && (work & kNeedExact)) {
-            const unsigned k = atomicAdd(A.counter + kExactCount, 1u);
+            const unsigned k = atomicAdd(A.counter, 1u);
             A.exact_list[k] = (int32_t)c;
         }
     }
@@ -313,29 +311,26 @@ __device__ void ring_candidate(const CollapseArgs& A, int64_t c, int tl, int wba
         A.status[c] = st;
         A.work[c] = work;
         if (!EXACT && (work & kNeedExact)) {
-            const unsigned k = atomicAdd(A.counter + kExactCount, 1u);
+            const unsigned k = atomicAdd(A.counter, 1u);
             A.exact_list[k] = (int32_t)c;
         }
     }
 }
 
-// Persistent: tiles pop chunks of candidates from an atomic queue, so rings
-// of 4..200 tets balance across the machine (the queue start is uniform
-// across a tile).
+// A tile per `chunk` consecutive candidates, as many tiles as that takes: the
+// hardware's block scheduler balances the uneven rings.  Bound by the latency
+// of its gathers (candidate -> ring ids -> vertices), so the more waves wait
+// the better.  (Persistent tiles popping candidates from one atomic counter
+// ran at the counter's rate, ~6 ns per pop: 200k candidates of 24-tet rings,
+// chunk 1: 1446 us for the whole batch, 360 us this way.)
 template <int TILE>
 __global__ __launch_bounds__(kBlock) void collapse_ring_kernel(CollapseArgs A)
 {
     const int tl = threadIdx.x % TILE;
     const int wbase = (threadIdx.x % 64) - tl;
-    for (;;) {
-        unsigned start = 0;
-        if (tl == 0) start = atomicAdd(A.counter, A.chunk);
-        start = __shfl(start, 0, TILE);
-        if ((int64_t)start >= A.n) break;
-        int64_t end = (int64_t)start + A.chunk;
-        if (end > A.n) end = A.n;
-        for (int64_t c = start; c < end; ++c) ring_candidate<TILE, false>(A, c, tl, wbase);
-    }
+    const int64_t c0 = (xcd_block() * (int64_t)(kBlock / TILE) + threadIdx.x / TILE) * A.chunk;
+    const int64_t c1 = c0 + A.chunk < A.n ? c0 + A.chunk : A.n;
+    for (int64_t c = c0; c < c1; ++c) ring_candidate<TILE, false>(A, c, tl, wbase);
 }
 
 // the candidates the filter pass listed, with the exact predicate; a tile per
@@ -346,16 +341,12 @@ __global__ __launch_bounds__(kBlock) void collapse_ring_exact_kernel(CollapseArg
     const int tl = threadIdx.x % TILE;
     const int wbase = (threadIdx.x % 64) - tl;
     const int64_t stride = (int64_t)gridDim.x * (kBlock / TILE);
-    const int64_t listed = A.counter[kExactCount];
+    const int64_t listed = *A.counter;
     for (int64_t k = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / TILE; k < listed; k += stride)
         ring_candidate<TILE, true>(A, A.exact_list[k], tl, wbase);
 }
 
-__global__ void reset_queue(unsigned* c)
-{
-    c[0] = 0u;
-    c[kExactCount] = 0u;
-}
+__global__ void reset_list(unsigned* c) { *c = 0u; }
 
 template <bool F32>
 __global__ __launch_bounds__(kBlock) void collapse_point_kernel(CollapseArgs A)
@@ -571,18 +562,15 @@ RingFn ring_fn(int tile, bool exact)
 }
 
 // every launch of one batch, in order, on stream s (graph-capturable: the
-// queue counter is cleared by a kernel)
+// list's length is cleared by a kernel)
 int enqueue(twg_ctx* ctx, const CollapseArgs& A, int tile, bool f32, hipStream_t s)
 {
     RingFn ring = ring_fn(tile, false);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(ring),
-                                                     kBlock, 0) != hipSuccess || per_cu < 1)
-        per_cu = 1;
-    int64_t need = (A.n * tile + kBlock - 1) / kBlock;
-    const unsigned gring = (unsigned)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)ctx->num_cus * per_cu));
+    const int64_t per = (int64_t)(kBlock / tile) * A.chunk;  // candidates per block
+    const unsigned gring = (unsigned)((A.n + per - 1) / per);
+    const int64_t need = (A.n * tile + kBlock - 1) / kBlock;
     const unsigned gexact = (unsigned)std::min<int64_t>(std::max<int64_t>(need, 1), 2048);
-    hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, s, A.counter);
+    hipLaunchKernelGGL(reset_list, dim3(1), dim3(1), 0, s, A.counter);
     TWG_LAUNCHED();
     hipLaunchKernelGGL(ring, dim3(gring), dim3(kBlock), 0, s, A);
     TWG_LAUNCHED();
