@@ -376,7 +376,7 @@ __global__ __launch_bounds__(kBlock) void collapse_point_kernel(CollapseArgs A)
 constexpr int kFaceGroup = 64;
 // facets listed per wave in the face pass (a triangle's neighbourhood)
 constexpr int kFaceListCap = 64;
-constexpr int kFaceListBytes = kFaceListCap * (32 + 8 + 72);
+constexpr int kFaceListBytes = kFaceListCap * kCertEntryBytes;
 
 template <bool F32>
 __global__ __launch_bounds__(kBlock) void collapse_face_kernel(CollapseArgs A)
@@ -410,8 +410,8 @@ __global__ __launch_bounds__(kBlock) void collapse_face_kernel(CollapseArgs A)
     const BvhWalk W = walk(A.sf);
     unsigned char* mine = face_lists + (threadIdx.x / 64) * kFaceListBytes;
     LdsNode32W* lst = (LdsNode32W*)mine;
-    LdsU32* fr = (LdsU32*)(mine + kFaceListCap * 32);
-    LdsF64* tri = (LdsF64*)(mine + kFaceListCap * 40);
+    LdsU32* fr = (LdsU32*)(mine + kFaceListCap * 32);  // the work lists, then the certificates
+    LdsF32* cert = (LdsF32*)(mine + kFaceListCap * 32);
     double lo[3], hi[3], amax = 0.0;
     bool fin = true;
 #pragma unroll
@@ -428,14 +428,10 @@ __global__ __launch_bounds__(kBlock) void collapse_face_kernel(CollapseArgs A)
         hi[j] += pad;
     }
     const int nl = fin ? collect_facets<64>(W, lo, hi, lst, fr, kFaceListCap, r, 0) : -1;
-    for (int e = r; e < nl; e += 64) {
-        const double* f = W.tri + 9 * (int64_t)lst[e].leaf;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) tri[9 * e + q] = f[q];
-    }
-    wave_sync();
+    const CertFrame F = cert_frame(lo, hi, amax, A.eps2, A.d);
+    cert_list<64>(W, lst, cert, nl, F, A.eps2, r);
     if (face_out_group<F32, kFaceGroup, false>(W, ld3(t9), ld3(t9 + 3), ld3(t9 + 6), A.eps2, A.d,
-                                               A.T_sf, A.sqrtT_sf, r, gbase, lst, tri, nl) &&
+                                               A.T_sf, A.sqrtT_sf, r, gbase, lst, cert, F, nl) &&
         r == 0)
         atomicOr(A.work + c, kFaceOut);
 }

@@ -150,45 +150,80 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     if (STATS) flush_stats(st, stats);
 }
 
-// face_out_listed for the wave's 64 triangles at once (a list of nl <= 128
-// facets, nl >= 0; act: the lane has a triangle, t9 its corners).  Every lane
-// tests its triangle's first sample; most triangles outside the envelope stop
-// there.  The other samples of the triangles still open are then spread over
-// the wave: the concatenation of their sequences (the first samples left
-// out) is cut into 64 consecutive blocks of K = ceil(total / 64) and lane r
-// walks block r, moving to the next open triangle when one ends.  A lane
-// takes the triangle it moves to -- its corners' address, list mask and the
-// facet that held its first sample -- from the triangle's own lane (shuffles,
-// every lane active; the corners are read again from memory, which keeps 18
-// registers free through the walk: 898 -> 946 M checks/s on 20 M queries),
-// and a sample found outside is passed to that lane by ballot.  The
-// decision -- some sample has no facet within eps -- does not depend on which
-// lane tests which sample, so it is face_out_listed's.  Returns the lane's
-// own triangle's decision.
-__device__ bool faces_wave_listed(bool act, const double* t9, double eps2, double d, double sqrtT,
-                                  LdsNode32W* lst, LdsF64c* tri, int nl, int lane)
+// What a lane keeps of its triangle while the wave's list is made: its corners
+// in the list's frame, the one SampleGen::init rotates to the front first, and
+// the box face_list_mask compares the list with.  (The corners themselves,
+// 18 registers, are read again by the few lanes that need them.)
+struct WaveFace {
+    bool act;
+    int first;
+    const double* t9;
+    V3<float> q[3];
+    float mlo[3], mhi[3];
+};
+
+// face_out_sampled for the wave's 64 triangles at once (a list of nl <= 128
+// facets, nl >= 0, with its certificates).  Every lane scans the facets near its triangle
+// for one that holds its first corner: none, and the triangle is out; one
+// that certifies all three corners, and it is in.  The samples of the
+// triangles still open -- they straddle facets, or reach the limit -- are
+// then spread over the wave: the concatenation of their sequences (the first
+// samples left out) is cut into 64 consecutive blocks of K = ceil(total / 64)
+// and lane r walks block r, moving to the next open triangle when one ends
+// and passing over the samples between two certified by one facet on one
+// row.  A lane takes the triangle it moves to -- its corners' address, list
+// mask and the facet that held its first sample -- from the triangle's own
+// lane (shuffles, every lane active; the corners are read again from memory,
+// which keeps 18 registers free through the walk), and a sample found outside
+// is passed to that lane by ballot.  The decision -- some sample has no facet
+// within eps -- does not depend on which lane tests which sample, so it is
+// face_out_sampled's.  Returns the lane's own triangle's decision.
+__device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double eps2, double d,
+                                  LdsNode32W* lst, LdsF32* cert, int nl, const CertFrame& F, int lane)
 {
-    bool out = false;
+    bool out = T.act, open_lane = false;
     int64_t rem = 0;  // samples after the first, while the triangle is open
     uint64_t mk[2] = {0ull, 0ull};
     int hl = -1;
-    if (act) {
-        const V3<double> a = ld3(t9), b = ld3(t9 + 3), c = ld3(t9 + 6);
-        const double l = fmax(len2(a - b), fmax(len2(b - c), len2(c - a)));
-        if (!(__builtin_sqrt(l) / d <= kMaxEdgeSamples)) {
-            out = true;
-        } else {
-            face_list_mask(lst, nl, a, b, c, sqrtT, mk);
-            SampleGen g;
-            g.init(a, b, c, d);
-            V3<double> s;
-            g.next(s);  // every sequence has a first sample
-            if (!in_envelope_masked<true>(lst, tri, nl, mk, s, eps2, sqrtT, hl)) out = true;
-            else rem = g.skip(INT64_MAX);
+    const double* t9 = T.t9;
+    if (T.act) {
+        face_list_mask(lst, nl, T.mlo, T.mhi, mk);
+        uint64_t unsure[2] = {0ull, 0ull};
+        bool all = false;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            uint64_t mm = 64 * w < nl ? mk[w] : 0ull;
+            while (mm && !all) {
+                const int i = 64 * w + __builtin_ctzll(mm);
+                LdsF32* ci = cert + kCertFloats * i;
+                const int r = cert_class(ci, T.q[0], F);
+                if (r == 0) unsure[w] |= mm & (0ull - mm);
+                mm &= mm - 1;
+                if (r > 0) {
+                    hl = i;
+                    all = F.runs && cert_class(ci, T.q[1], F) > 0 && cert_class(ci, T.q[2], F) > 0;
+                }
+            }
         }
+        if (hl < 0 && (unsure[0] | unsure[1])) {
+            const V3<double> p0 = ld3(t9 + 3 * T.first);
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+                for (uint64_t mm = unsure[w]; mm && hl < 0; mm &= mm - 1) {
+                    const int i = 64 * w + __builtin_ctzll(mm);
+                    if (facet_d2(W, lst[i].leaf, p0) <= eps2) hl = i;
+                }
+        }
+        out = hl < 0;
+        open_lane = hl >= 0 && !all;
+    }
+    if (__ballot(open_lane) == 0ull) return out;
+    if (open_lane) {
+        SampleGen g;
+        g.init(ld3(t9), ld3(t9 + 3), ld3(t9 + 6), d);
+        rem = g.skip(INT64_MAX) - 1;
     }
     const unsigned long long open = __ballot(rem > 0);
-    if (open == 0ull) return out;
     int64_t incl = rem;
     for (int off = 1; off < 64; off <<= 1) {
         const int64_t o = __shfl_up(incl, off, 64);
@@ -197,6 +232,7 @@ __device__ bool faces_wave_listed(bool act, const double* t9, double eps2, doubl
     const int64_t total = __shfl(incl, 63, 64);
     const int64_t K = (total + 63) / 64;
     const int64_t first = (int64_t)lane * K;
+    const int64_t mine = total - first < K ? total - first : K;
     // the triangle holding remaining sample `first`: the first lane f with
     // incl[f] > first (a binary search, each lane its own)
     int f = 0;
@@ -222,8 +258,8 @@ __device__ bool faces_wave_listed(bool act, const double* t9, double eps2, doubl
             g2.skip(1 + ofs);
         }
     }
-    for (int64_t j = 0; j < K; ++j) {
-        const bool have = f < 64 && first + j < total;
+    for (int64_t j = 0; __ballot(j < mine);) {
+        const bool have = j < mine;
         V3<double> s;
         bool got = have && g2.next(s);
         const bool need = have && !got;
@@ -244,7 +280,16 @@ __device__ bool faces_wave_listed(bool act, const double* t9, double eps2, doubl
                 got = g2.next(s);
             }
         }
-        const bool o2 = got && !in_envelope_masked<true>(lst, tri, nl, m2, s, eps2, sqrtT, h2);
+        bool sure = false;
+        const bool o2 = got && !in_envelope_cert<false>(W, lst, cert, nl, m2, s, F, eps2, h2, sure);
+        ++j;
+        if (got && sure && F.runs && j < mine) {
+            const int64_t left = g2.run_left(mine - j);
+            if (left > 0 && cert_class(cert + kCertFloats * h2, cert_local(F, g2.run_at(left)), F) > 0) {
+                g2.k += (int)left;
+                j += left;
+            }
+        }
         // the triangles found outside, to their lanes
         unsigned long long ob = __ballot(o2);
         while (ob) {
@@ -259,87 +304,146 @@ __device__ bool faces_wave_listed(bool act, const double* t9, double eps2, doubl
 // One triangle per lane, as faces_kernel, for batches walked in Morton
 // order: the wave's 64 consecutive triangles lie close together, so the wave
 // lists once (collect_facets, LDS) the facets whose boxes meet the box of its
-// triangles padded by more than sqrt(T), with their triangles, and tests its
-// samples against the list (in_envelope_list) instead of walking the tree
-// per sample.  A wave whose list exceeds CAP entries walks the tree (from
-// global memory: the LDS holds the lists).
+// triangles padded by more than sqrt(T), with their certificates, and tests
+// its triangles against the list (faces_wave_listed) instead of walking the
+// tree per sample.  Blocks of one wave: a block's LDS is free for the next one
+// as soon as its wave ends.  3 M triangles on 246 k facets: 2.73 -> 1.37 ms
+// for the kernel, with the certificates, the wider tree rounds of
+// collect_facets, the rows through LDS, the split waves and the short blocks;
+// half of what is left waits for memory, the VALU is busy for a third of it.
+// xcd_block for work that is uneven along the items (sorted queries): each XCD
+// takes runs of 64 consecutive blocks in turn instead of a contiguous eighth,
+// so no XCD is left with a long eighth (3 M triangles 2187 -> 1812 us with the
+// one-wave blocks of faces_list_kernel: 31 % of the CU time had been idle).
+__device__ __forceinline__ int64_t xcd_run_block()
+{
+    const unsigned g = gridDim.x, b = blockIdx.x;
+    const unsigned whole = g / 512 * 512;
+    if (b >= whole) return b;
+    const unsigned k = b / 8;
+    return (int64_t)(k / 64) * 512 + (b % 8) * 64 + k % 64;
+}
+
+constexpr int kFaceSplit = 8;
 template <bool F32, int CAP>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void faces_list_kernel(
-    BvhView B, const double* __restrict__ tri9, int64_t n, double eps2, double d, double T,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void faces_list_kernel(
+    BvhView B, const double* __restrict__ tri9, int64_t n, double eps2, double d, double T_,
     double sqrtT, uint8_t* __restrict__ out, unsigned* n_pending, int64_t* pending,
     const int32_t* __restrict__ order, unsigned long long* lstat)
 {
-    constexpr int kWaveBytes = CAP * (32 + 8 + 72);
-        __shared__ __align__(16) unsigned char lists[(kBlock / 64) * kWaveBytes];
+    constexpr int kWaveBytes = CAP * kCertEntryBytes;
+    static_assert(CAP <= 128, "two list-mask words");
+    __shared__ __align__(16) unsigned char mine[kWaveBytes];
     const BvhWalk W = walk(B);
-    const int lane = threadIdx.x % 64;
-    unsigned char* mine = lists + (threadIdx.x / 64) * kWaveBytes;
+    const int lane = threadIdx.x;
     LdsNode32W* lst = (LdsNode32W*)mine;
-    LdsU32* fr = (LdsU32*)(mine + CAP * 32);
-    LdsF64* tri = (LdsF64*)(mine + CAP * 40);
-    int64_t i = xcd_block() * kBlock + threadIdx.x;
-    bool act = false;
-    const double* t = tri9;
-    if (i < n) {
-        if (order) i = order[i];
-        t = tri9 + 9 * i;
-        if (certainly_not_collinear(t, t + 3, t + 6)) {
-            act = true;
-        } else {
+    LdsU32* fr = (LdsU32*)(mine + CAP * 32);  // the work lists, then the certificates
+    LdsF32* cert = (LdsF32*)(mine + CAP * 32);
+    int64_t i = xcd_run_block() * 64 + threadIdx.x;
+    const int row = i < n ? (order ? order[i] : (int)i) : -1;
+    if (i < n) i = row;
+    // the wave's 64 triangles through LDS, nine lanes to a row: each line of a
+    // row comes in once (nine 8-byte loads per lane, a row apart from lane to
+    // lane, took 60 k of the wave's 300 k cycles)
+    LdsF64* rows = (LdsF64*)mine;
+    static_assert(64 * 9 * 8 <= kWaveBytes, "room for the wave's triangles");
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        const int e = 64 * k + lane, src = __shfl(row, e / 9, 64);
+        rows[e] = src >= 0 ? tri9[9 * (int64_t)src + e % 9] : 0.0;
+    }
+    wave_sync();
+    double t[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) t[k] = rows[9 * lane + k];
+    wave_sync();  // read before the list takes its place
+    WaveFace T;
+    T.act = false;
+    T.first = 0;
+    T.t9 = tri9 + 9 * (int64_t)(row >= 0 ? row : 0);
+    if (row >= 0) {
+        const V3<double> a = ld3(t), b = ld3(t + 3), c = ld3(t + 6);
+        if (!certainly_not_collinear(t, t + 3, t + 6)) {
             unsigned k = atomicAdd(n_pending, 1u);
             pending[k] = i;
+        } else {
+            const double l0 = len2(a - b), l1 = len2(b - c), l2 = len2(c - a);
+            const double N = __builtin_sqrt(fmax(l0, fmax(l1, l2))) / d;
+            T.act = N <= kMaxEdgeSamples;
+            if (!T.act) out[i] = 1;
+            else if (N > 1) T.first = !(l2 < l0) && !(l2 < l1) ? 2 : (!(l1 < l0) ? 1 : 0);
         }
     }
-    // the box of the wave's triangles, padded
-    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    if (act)
+    // The lanes [s, s + w) at a time: all 64, unless their facets do not fit the
+    // list -- the Morton order jumps inside the wave, say -- then its halves, down
+    // to kFaceSplit lanes, which walk the tree.  (Whole waves walking it, 5.8 %
+    // of them, ran on alone for half of the kernel's time.)
+    bool walked = false;
+    for (int s = 0, w = 64; s < 64;) {
+        WaveFace U = T;
+        U.act = T.act && lane >= s && lane < s + w;
+        if (__ballot(U.act)) {
+            V3<double> a = mk3<double>(INFINITY, INFINITY, INFINITY), b = a, c = a;
+            if (U.act) {
+                a = ld3(T.t9);
+                b = ld3(T.t9 + 3);
+                c = ld3(T.t9 + 6);
+            }
+            const bool fin = !U.act || (is_finite(a.x) && is_finite(a.y) && is_finite(a.z) && is_finite(b.x) &&
+                                        is_finite(b.y) && is_finite(b.z) && is_finite(c.x) && is_finite(c.y) &&
+                                        is_finite(c.z));
+            // the box of the lanes' triangles, padded
+            const V3<double> l3 = mk3(fmin(a.x, fmin(b.x, c.x)), fmin(a.y, fmin(b.y, c.y)), fmin(a.z, fmin(b.z, c.z)));
+            const V3<double> h3 = mk3(fmax(a.x, fmax(b.x, c.x)), fmax(a.y, fmax(b.y, c.y)), fmax(a.z, fmax(b.z, c.z)));
+            double lo[3] = {l3.x, l3.y, l3.z};
+            double hi[3] = {U.act ? h3.x : -INFINITY, U.act ? h3.y : -INFINITY, U.act ? h3.z : -INFINITY};
+            double amax = 0.0;
 #pragma unroll
-        for (int k = 0; k < 9; ++k) {
-            lo[k % 3] = t[k] < lo[k % 3] ? t[k] : lo[k % 3];
-            hi[k % 3] = t[k] > hi[k % 3] ? t[k] : hi[k % 3];
+            for (int k = 0; k < 3; ++k) {
+                for (int off = 32; off > 0; off >>= 1) {
+                    const double ol = __shfl_xor(lo[k], off, 64), oh = __shfl_xor(hi[k], off, 64);
+                    lo[k] = ol < lo[k] ? ol : lo[k];
+                    hi[k] = oh > hi[k] ? oh : hi[k];
+                }
+                amax = fmax(amax, fmax(fabs(lo[k]), fabs(hi[k])));
+            }
+            const double pad = 1.0001 * sqrtT + 1e-9 * amax;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                lo[k] -= pad;
+                hi[k] += pad;
+            }
+            // a coordinate that is not finite can leave the lanes with different
+            // boxes (min / max ignore NaN): no list for them
+            const int nl = __ballot(!fin) ? -1 : collect_facets<64>(W, lo, hi, lst, fr, CAP, lane, 0);
+            if (nl >= 0) {
+                const CertFrame F = cert_frame(lo, hi, amax, eps2, d);
+                face_mask_box(a, b, c, sqrtT, U.mlo, U.mhi);
+                U.q[0] = cert_local(F, sel3(U.first, a, b, c));
+                U.q[1] = cert_local(F, sel3(U.first, b, c, a));
+                U.q[2] = cert_local(F, sel3(U.first, c, a, b));
+                cert_list<64>(W, lst, cert, nl, F, eps2, lane);
+                const bool o = faces_wave_listed(W, U, eps2, d, lst, cert, nl, F, lane);
+                if (U.act) out[i] = o ? 1 : 0;
+                wave_sync();  // the list's last reads
+            } else if (w > kFaceSplit) {
+                w /= 2;
+                continue;
+            } else {
+                walked = true;
+                Stats st;
+                if (U.act) out[i] = face_out_sampled<F32, false>(W, T.t9, eps2, d, T_, sqrtT, st) ? 1 : 0;
+            }
         }
-    double amax = 0.0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        for (int off = 32; off > 0; off >>= 1) {
-            const double ol = __shfl_xor(lo[k], off, 64), oh = __shfl_xor(hi[k], off, 64);
-            lo[k] = ol < lo[k] ? ol : lo[k];
-            hi[k] = oh > hi[k] ? oh : hi[k];
-        }
-        amax = fmax(amax, fmax(fabs(lo[k]), fabs(hi[k])));
+        s += w;
+        w = s & -s;
     }
-    const double pad = 1.0001 * sqrtT + 1e-9 * amax;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        lo[k] -= pad;
-        hi[k] += pad;
-    }
-    // a coordinate that is not finite can leave the lanes with different
-    // boxes (min / max ignore NaN): then the whole wave walks the tree
-    bool fin = true;
-    if (act)
-#pragma unroll
-        for (int k = 0; k < 9; ++k) fin = fin && is_finite(t[k]);
-    const int nl = __ballot(!fin) ? -1 : collect_facets<64>(W, lo, hi, lst, fr, CAP, lane, 0);
-    if (lstat && lane == 0) atomicAdd(lstat + (nl >= 0 ? 0 : 1), 1ull);
-    for (int e = lane; e < nl; e += 64) {
-        const double* f = B.tri + 9 * (int64_t)lst[e].leaf;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) tri[9 * e + k] = f[k];
-    }
-    list_neighbours<64>(W, lst, nl, lane);
-    static_assert(CAP <= 128, "two list-mask words");
-    if (nl < 0) {
-        if (act) out[i] = face_out_listed<F32>(W, t, eps2, d, T, sqrtT, lst, tri, nl) ? 1 : 0;
-        return;
-    }
-    const bool o = faces_wave_listed(act, t, eps2, d, sqrtT, lst, tri, nl, lane);
-    if (act) out[i] = o ? 1 : 0;
+    if (lstat && lane == 0) atomicAdd(lstat + (walked ? 1 : 0), 1ull);
 }
 
 // facets listed per wave in faces_group_kernel<F32, 64>
 constexpr int kGroupListCap = 64;
-constexpr int kGroupListBytes = kGroupListCap * (32 + 8 + 72);
+constexpr int kGroupListBytes = kGroupListCap * kCertEntryBytes;
 
 // A group of G lanes per triangle, its samples spread over the lanes
 // (face_out_group).  Small batches run G = 64 (a wave per triangle), so that
@@ -371,14 +475,15 @@ __global__ __launch_bounds__(kBlock) void faces_group_kernel(BvhView B, const do
     }
     int nl = -1;
     LdsNode32W* lst = nullptr;
-    LdsF64* tri = nullptr;
+    LdsF32* cert = nullptr;
+    CertFrame F = {};
     if (G == 64) {
         // the facets near the triangle, listed in the wave's LDS (the tree
         // walk when they do not fit or a coordinate is not finite)
         unsigned char* mine = face_lists + (threadIdx.x / 64) * kGroupListBytes;
         lst = (LdsNode32W*)mine;
-        LdsU32* fr = (LdsU32*)(mine + kGroupListCap * 32);
-        tri = (LdsF64*)(mine + kGroupListCap * 40);
+        LdsU32* fr = (LdsU32*)(mine + kGroupListCap * 32);  // the work lists, then the certificates
+        cert = (LdsF32*)(mine + kGroupListCap * 32);
         double lo[3], hi[3], amax = 0.0;
         bool fin = true;
 #pragma unroll
@@ -397,15 +502,12 @@ __global__ __launch_bounds__(kBlock) void faces_group_kernel(BvhView B, const do
         // (listed from the global tree: measured ~5 % faster than through the
         // LDS copy of its top here)
         nl = fin ? collect_facets<64>(walk(B), lo, hi, lst, fr, kGroupListCap, r, 0) : -1;
-        for (int e = r; e < nl; e += 64) {
-            const double* f = B.tri + 9 * (int64_t)lst[e].leaf;
-#pragma unroll
-            for (int q = 0; q < 9; ++q) tri[9 * e + q] = f[q];
-        }
+        F = cert_frame(lo, hi, amax, eps2, d);
+        cert_list<64>(W, lst, cert, nl, F, eps2, r);
         list_neighbours<64>(walk(B), lst, nl, r);
     }
     const bool o = face_out_group<F32, G, true, true>(W, ld3(t), ld3(t + 3), ld3(t + 6), eps2, d, T, sqrtT, r,
-                                          gbase, lst, tri, nl);
+                                                      gbase, lst, cert, F, nl);
     if (r == 0) out[i] = o ? 1 : 0;
 }
 
@@ -836,9 +938,9 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
             hipLaunchKernelGGL((faces_group_kernel<true, 64>), gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order);
     } else if (order && !stats && n >= kFaceListDensity * B->nf) {
         if (precision == TWG_FP64)
-            hipLaunchKernelGGL((faces_list_kernel<false, kFaceListCap>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
+            hipLaunchKernelGGL((faces_list_kernel<false, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
         else
-            hipLaunchKernelGGL((faces_list_kernel<true, kFaceListCap>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
+            hipLaunchKernelGGL((faces_list_kernel<true, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
     } else if (precision == TWG_FP64) {
         if (stats) hipLaunchKernelGGL((faces_kernel<false, true>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, stats, n_pending, pending, order);
         else hipLaunchKernelGGL((faces_kernel<false, false>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, stats, n_pending, pending, order);

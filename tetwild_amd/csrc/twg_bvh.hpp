@@ -381,11 +381,10 @@ __device__ __forceinline__ float f32_down(double x)
 }
 __device__ __forceinline__ float f32_up(double x) { return -f32_down(-x); }
 
-template <typename R, typename S>
-__device__ __forceinline__ bool boxes_meet(const R* alo, const R* ahi, const S* blo, const S* bhi)
+__device__ __forceinline__ bool box_meets(const BvhNode32& r, const float lof[3], const float hif[3])
 {
-    return alo[0] <= bhi[0] && alo[1] <= bhi[1] && alo[2] <= bhi[2] && ahi[0] >= blo[0] &&
-           ahi[1] >= blo[1] && ahi[2] >= blo[2];
+    return r.lo[0] <= hif[0] && r.hi[0] >= lof[0] && r.lo[1] <= hif[1] && r.hi[1] >= lof[1] &&
+           r.lo[2] <= hif[2] && r.hi[2] >= lof[2];
 }
 
 __device__ __forceinline__ void put_lds(LdsNode32W* d, const BvhNode32& s)
@@ -401,17 +400,23 @@ __device__ __forceinline__ void put_lds(LdsNode32W* d, const BvhNode32& s)
 
 // The facets whose boxes meet the box [lo, hi], found by the G lanes of a
 // group (G a power of two up to 64, lane gl, the group's first lane gbase in
-// the wave) expanding a work list of internal nodes that meet the box (fr:
-// two buffers of cap entries).  A lane expands one node: its children from
-// the walker's FP64 LDS copy when they are there, else its children and
-// grandchildren from the FP32 records in global memory, read together (one
-// memory latency for two levels; a grandchild's box lies inside its
-// parent's, and FP32 boxes are rounded outward, so no facet is lost).
-// Ballots place what meets the box -- leaves into lst as FP32 records,
-// internal nodes into the next work list.  Returns the number of facets in
-// lst, or -1 (nothing usable in lst) when more than cap facets, or more than
-// cap nodes in one work list, meet the box, when the box is not finite, or
-// for a one-facet tree.  Every lane of the group calls it.
+// the wave) from a work list of nodes that meet the box (fr: two buffers of
+// cap entries), level by level.  Each round reads, for n listed nodes, their
+// descendants lv levels down, as many levels as fill the group (64 nodes for
+// a list of one) and two at least, one node per lane from the FP32 records in global memory: a
+// node's box lies inside its ancestors', so the levels between need no test,
+// and FP32 boxes are rounded outward, so no facet is lost.  The rounds are a
+// chain of dependent reads, five for 250 k facets (two levels a round, children
+// and grandchildren of a node read by one lane, took nine rounds of twelve
+// loads each: 84 k of a wave's cycles against 61 k; 60 k smoothing problems
+// 1753 -> 1662 us).  Leaves lie on the last two levels (the median
+// splits of the build), and rounds end on the last level at the latest, where
+// a lane whose slot is empty looks at its parent.  Ballots place what meets the
+// box -- leaves into lst as FP32 records, internal nodes into the next work
+// list.  Returns the number of facets in lst, or -1 (nothing usable in lst)
+// when more than cap facets, or more than cap nodes in one work list, meet the
+// box, when the box is not finite, or for a one-facet tree.  Every lane of the
+// group calls it.
 template <int G>
 __device__ int collect_facets(const BvhWalk& W, const double lo[3], const double hi[3],
                               LdsNode32W* lst, LdsU32* fr, int cap, int gl, int gbase)
@@ -432,75 +437,36 @@ __device__ int collect_facets(const BvhWalk& W, const double lo[3], const double
     LdsU32* nxt = fr + cap;
     if (gl == 0) cur[0] = 1u;
     wave_sync();
+    int below_root = 64 - __builtin_clzll((unsigned long long)(W.nf - 1));  // levels below the listed nodes
     int ncur = 1, nl = 0;
     while (ncur > 0) {
+        int lv = below_root < 2 ? below_root : 2;
+        while (lv < below_root && (ncur << (lv + 1)) <= G) ++lv;
+        below_root -= lv;
+        const int total = ncur << lv;
         int nn = 0;
-        for (int i0 = 0; i0 < ncur; i0 += G) {
-            const int i = i0 + gl;
-            // up to four candidates: slot k holds node id[k] (0: none)
-            BvhNode32 cand[4];
-            int64_t id[4] = {0, 0, 0, 0};
-            bool ok[4] = {false, false, false, false};
-            if (i < ncur) {
-                const int64_t ch = 2 * (int64_t)cur[i];
-                if (ch < W.ncache && W.top64) {
-                    const BvhNode64 L64 = from_lds(W.c64 + ch), R64 = from_lds(W.c64 + ch + 1);
-                    ok[0] = boxes_meet(L64.lo, L64.hi, lo, hi);
-                    ok[1] = boxes_meet(R64.lo, R64.hi, lo, hi);
-                    id[0] = ch;
-                    id[1] = ch + 1;
-                    cand[0].leaf = L64.leaf;
-                    cand[1].leaf = R64.leaf;
-                    if (ok[0] && L64.leaf >= 0) cand[0] = W.n32[ch];
-                    if (ok[1] && R64.leaf >= 0) cand[1] = W.n32[ch + 1];
-                } else {
-                    BvhNode32 C[2], GC[4];
-                    if (ch < W.ncache) {
-                        C[0] = from_lds(W.c32 + ch);
-                        C[1] = from_lds(W.c32 + ch + 1);
-                    } else {
-                        C[0] = W.n32[ch];
-                        C[1] = W.n32[ch + 1];
-                    }
-                    // grandchildren slots exist for an internal child (read
-                    // before the child is known to be internal; used only then)
-                    const int64_t g0 = 2 * ch;
-                    if (g0 + 1 < W.nnode) {
-                        GC[0] = W.n32[g0];
-                        GC[1] = W.n32[g0 + 1];
-                    }
-                    if (g0 + 3 < W.nnode) {
-                        GC[2] = W.n32[g0 + 2];
-                        GC[3] = W.n32[g0 + 3];
-                    }
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        if (!boxes_meet(C[h].lo, C[h].hi, lof, hif)) continue;
-                        if (C[h].leaf >= 0) {
-                            cand[2 * h] = C[h];
-                            id[2 * h] = ch + h;
-                            ok[2 * h] = true;
-                        } else {
-#pragma unroll
-                            for (int e = 0; e < 2; ++e) {
-                                cand[2 * h + e] = GC[2 * h + e];
-                                id[2 * h + e] = 2 * (ch + h) + e;
-                                ok[2 * h + e] = boxes_meet(GC[2 * h + e].lo, GC[2 * h + e].hi, lof, hif);
-                            }
-                        }
-                    }
+        for (int t0 = 0; t0 < total; t0 += G) {
+            const int t = t0 + gl;
+            bool ok = false;
+            BvhNode32 N;
+            N.leaf = -2;
+            int64_t id = 0;
+            if (t < total) {
+                id = ((int64_t)cur[t >> lv] << lv) + (t & ((1 << lv) - 1));
+                if (id < W.nnode) N = W.n32[id];
+                if (below_root == 0 && N.leaf == -2 && (id & 1) == 0) {
+                    N = W.n32[id >> 1];
+                    if (N.leaf < 0) N.leaf = -2;  // (a listed node's descendant: never so)
                 }
+                ok = N.leaf != -2 && box_meets(N, lof, hif);
             }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const bool leaf = ok[k] && cand[k].leaf >= 0, inner = ok[k] && cand[k].leaf < 0;
-                const unsigned long long ml = __ballot(leaf) & gm, mi = __ballot(inner) & gm;
-                const int pl = nl + __popcll(ml & below), qi = nn + __popcll(mi & below);
-                if (leaf && pl < cap) put_lds(lst + pl, cand[k]);
-                if (inner && qi < cap) nxt[qi] = (uint32_t)id[k];
-                nl += __popcll(ml);
-                nn += __popcll(mi);
-            }
+            const bool leaf = ok && N.leaf >= 0, inner = ok && N.leaf < 0;
+            const unsigned long long ml = __ballot(leaf) & gm, mi = __ballot(inner) & gm;
+            const int pl = nl + __popcll(ml & below), qi = nn + __popcll(mi & below);
+            if (leaf && pl < cap) put_lds(lst + pl, N);
+            if (inner && qi < cap) nxt[qi] = (uint32_t)id;
+            nl += __popcll(ml);
+            nn += __popcll(mi);
         }
         if (nl > cap || nn > cap) return -1;
         wave_sync();
@@ -638,18 +604,10 @@ __device__ __forceinline__ void face_mask_box(V3<double> a, V3<double> b, V3<dou
     }
 }
 
-__device__ __forceinline__ bool box_meets(const BvhNode32& r, const float lof[3], const float hif[3])
-{
-    return r.lo[0] <= hif[0] && r.hi[0] >= lof[0] && r.lo[1] <= hif[1] && r.hi[1] >= lof[1] &&
-           r.lo[2] <= hif[2] && r.hi[2] >= lof[2];
-}
-
 template <class L>
-__device__ __forceinline__ void face_list_mask(L lst, int nl, V3<double> a, V3<double> b,
-                                               V3<double> c, double sqrtT, uint64_t mk[2])
+__device__ __forceinline__ void face_list_mask(L lst, int nl, const float lof[3], const float hif[3],
+                                               uint64_t mk[2])
 {
-    float lof[3], hif[3];
-    face_mask_box(a, b, c, sqrtT, lof, hif);
     // the two words in registers (an array indexed at run time would go to
     // scratch memory), eight records read before their tests
     const int n = nl < 128 ? nl : 128;
@@ -673,6 +631,14 @@ __device__ __forceinline__ void face_list_mask(L lst, int nl, V3<double> a, V3<d
     }
     mk[0] = w[0];
     mk[1] = w[1];
+}
+template <class L>
+__device__ __forceinline__ void face_list_mask(L lst, int nl, V3<double> a, V3<double> b,
+                                               V3<double> c, double sqrtT, uint64_t mk[2])
+{
+    float lof[3], hif[3];
+    face_mask_box(a, b, c, sqrtT, lof, hif);
+    face_list_mask(lst, nl, lof, hif, mk);
 }
 
 // in_envelope_list over the list positions set in mask (two 64-bit words;
@@ -748,6 +714,232 @@ __device__ __forceinline__ bool in_envelope_masked(LdsNode32W* lst, LdsF64c* tri
             const int i = 64 * w + __builtin_ctzll(m);
             m &= m - 1;
             if (tri_d2(tri + 9 * i, p) <= eps2) {
+                hl = i;
+                return true;
+            }
+        }
+    }
+    return false;
+}
+
+// ---- certified FP32 decisions for the listed facets ------------------------
+// A sample's exact test against a facet (point_tri_d2, FP64) is some 240
+// instructions once the lanes of a wave diverge over its seven regions, and a
+// sample away from the limit does not need it.  Per listed facet the group
+// keeps (LDS, kCertFloats floats) its unit normal and the outward unit
+// normals of its edges in its plane, each with its offset from an origin o in
+// the middle of the list's box.  In that frame, with q = p - o in FP32, h the
+// distance from the plane and e_i the distances past the edges:
+//   h^2 + max(e_i, 0)^2 is at most the squared distance (the projection lies
+//   past edge i's line), so above (eps + mu)^2 the facet does not hold p;
+//   it is the squared distance when the projection is inside (all e_i <= 0) or
+//   its foot on the line of the edge it is furthest past lies on the edge, so
+//   below (eps - mu)^2 the facet holds p.
+// Everything else (the eps band, the corner regions, a facet without a frame)
+// is left to FP64.  mu covers every rounding: with R the distance from o to
+// the list box's corners every |q|, |offset| <= 4 R, so h and e_i are within
+// 2^-20 R (twelve products and sums of 2^-24 relative error); mu = 2^-17 R +
+// 2^-46 max|coordinate| is the margin on distances, eta = mu / 2 on the signs
+// of the e_i.  A facet gets a frame only when the rounding of its own
+// point_tri_d2 (2^-46 (edge + R)^2 over the squared sine of its angle at
+// vertex 0) stays below mu eps / 4 and its determinant is above the 1e-30
+// where point_tri_d2 leaves the interior out; others hold NaN, which fails
+// every comparison.  The FP64 test's outcome is the certified one in every
+// certified case, so decisions are unchanged.
+//   Measured: 3 M triangles of 6-11 samples on 246 k facets 3.19 -> 2.57 ms, 200 k
+// collapse candidates 360 -> 317 us, 12 triangles of ~800 samples 199 -> 159 us.
+constexpr int kCertFloats = 20;  // 80 bytes: 16-byte reads, 16 bank phases
+constexpr int kCertEntryBytes = 32 + 4 * kCertFloats;  // a list entry and its certificate
+typedef __attribute__((address_space(3))) float LdsF32;
+
+struct CertFrame {
+    double o[3];
+    double mu;  // the margin on distances (above eps / 4: no certificates)
+    float in2, out2, eta;
+    bool runs;  // samples between two certified ones on a line are certified
+};
+
+// The frame for a list made for the box [lo, hi] (padded, so it holds every
+// point tested); amax: the box's largest coordinate magnitude before padding,
+// d: the sampling distance.  runs: a facet's distance is convex, so it holds
+// what lies between points that it holds, up to how far the samples are from
+// their lines and triangles -- at most 16 ulp of edge^2 / d + max|coordinate|
+// (the rows' starts carry the rounding of the triangle's angles) with edges of
+// at most 2 R, which has to stay below mu / 4.
+__device__ __forceinline__ CertFrame cert_frame(const double lo[3], const double hi[3], double amax,
+                                                double eps2, double d)
+{
+    CertFrame F;
+    double r2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        F.o[k] = 0.5 * (lo[k] + hi[k]);
+        const double h = 0.5 * (hi[k] - lo[k]);
+        r2 += h * h;
+    }
+    const double R = __builtin_sqrt(r2), eps = __builtin_sqrt(eps2);
+    F.mu = 0x1p-17 * R + 0x1p-46 * amax;
+    F.eta = (float)(0.5 * F.mu);
+    F.runs = 4.0 * r2 + amax * d <= F.mu * d * 0x1p44;
+    F.in2 = -1.0f;
+    F.out2 = __builtin_inff();
+    // (squares in FP32 need room on both sides; NaN fails)
+    if (F.mu <= 0.25 * eps && eps2 > 1e-24 && r2 < 1e24) {
+        F.in2 = (float)((eps - F.mu) * (eps - F.mu) * (1.0 - 0x1p-20));
+        F.out2 = (float)((eps + F.mu) * (eps + F.mu) * (1.0 + 0x1p-20));
+    }
+    return F;
+}
+
+// writes facet t's entry (9 doubles) into c
+template <class P>
+__device__ __forceinline__ void cert_write(P c, const double* t, const CertFrame& F, double eps2)
+{
+    const V3<double> o = mk3(F.o[0], F.o[1], F.o[2]);
+    const V3<double> a = ld3(t) - o, b = ld3(t + 3) - o, d = ld3(t + 6) - o;
+    const V3<double> e0 = b - a, e1 = d - a, e2 = d - b;
+    const V3<double> n = cross(e0, e1);
+    const double a00 = len2(e0), a11 = len2(e1), a01 = dot(e0, e1), nn = len2(n);
+    const double det = a00 * a11 - a01 * a01;
+    const double r = 0x1p17 * F.mu;  // >= R
+    const double big = (a00 > a11 ? a00 : a11) + r * r;
+    const bool ok = det > 1e-29 && nn > 1e-29 && F.in2 > 0.0f &&
+                    big * a00 * a11 <= F.mu * __builtin_sqrt(eps2) * 0x1p44 * nn;
+    const double lim = 4.0 * r;  // an offset beyond it keeps its sign and stays out of reach
+    const V3<double> un = mulv(n, 1.0 / __builtin_sqrt(nn));
+    V3<double> m[3] = {cross(e0, un), cross(e2, un), cross(un, e1)};
+    const V3<double> at[3] = {a, b, a};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) m[k] = mulv(m[k], 1.0 / len(m[k]));
+    double off[4] = {dot(un, a), dot(m[0], at[0]), dot(m[1], at[1]), dot(m[2], at[2])};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) off[k] = off[k] > lim ? lim : (off[k] < -lim ? -lim : off[k]);
+    const float bad = __builtin_nanf("");
+    c[0] = ok ? (float)un.x : bad;
+    c[1] = ok ? (float)un.y : bad;
+    c[2] = ok ? (float)un.z : bad;
+    c[3] = ok ? (float)off[0] : bad;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        c[4 + 4 * k] = (float)m[k].x;
+        c[5 + 4 * k] = (float)m[k].y;
+        c[6 + 4 * k] = (float)m[k].z;
+        c[7 + 4 * k] = (float)off[k + 1];
+    }
+    c[16] = (float)dot(m[0], m[1]);
+    c[17] = (float)dot(m[1], m[2]);
+    c[18] = (float)dot(m[2], m[0]);
+    c[19] = 0.0f;
+}
+
+// the entries of a whole collect_facets list (lanes gl, gl + G, ...); ends
+// with the group's writes visible
+template <int G>
+__device__ __forceinline__ void cert_list(const BvhWalk& W, LdsNode32W* lst, LdsF32* cert, int nl,
+                                          const CertFrame& F, double eps2, int gl)
+{
+    for (int e = gl; e < nl; e += G)
+        cert_write(cert + kCertFloats * e, W.tri + 9 * (int64_t)lst[e].leaf, F, eps2);
+    wave_sync();
+}
+
+__device__ __forceinline__ V3<float> cert_local(const CertFrame& F, V3<double> p)
+{
+    return mk3((float)(p.x - F.o[0]), (float)(p.y - F.o[1]), (float)(p.z - F.o[2]));
+}
+
+// 1: the facet holds the point, -1: it does not, 0: FP64 decides
+template <class P>
+__device__ __forceinline__ int cert_class(P c, V3<float> q, const CertFrame& F)
+{
+    float v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = c[k];
+    float s[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        s[k] = __builtin_fmaf(v[4 * k], q.x, __builtin_fmaf(v[4 * k + 1], q.y,
+                              __builtin_fmaf(v[4 * k + 2], q.z, -v[4 * k + 3])));
+    const float me = s[1] > s[2] ? (s[1] > s[3] ? s[1] : s[3]) : (s[2] > s[3] ? s[2] : s[3]);
+    const float mp = me > 0.0f ? me : 0.0f;
+    const float lb2 = __builtin_fmaf(mp, mp, s[0] * s[0]);
+    int r = lb2 > F.out2 ? -1 : 0;
+    if (lb2 < F.in2) {
+        if (me < -F.eta) {
+            r = 1;
+        } else {
+            // past (or at) one edge: the foot on its line, against the others
+            const float g01 = c[16], g12 = c[17], g20 = c[18];
+            const bool i0 = me == s[1], i1 = !i0 && me == s[2];
+            const float fa = i0 ? s[2] - me * g01 : (i1 ? s[1] - me * g01 : s[1] - me * g20);
+            const float fb = i0 ? s[3] - me * g20 : (i1 ? s[3] - me * g12 : s[2] - me * g12);
+            if (fa < -F.eta && fb < -F.eta) r = 1;
+        }
+    }
+    return r;
+}
+
+// in_envelope_list / in_envelope_masked with the certificates: the facet at
+// hl first (NB: then its neighbours), then the positions set in mask, in
+// ascending order; positions no certificate decides go to FP64 at the end.
+// The decision is in_envelope_masked's; hl may become another facet that
+// holds p.  sure: set when the facet left in hl is certified.
+template <bool NB, class L, class P, class M>
+__device__ __forceinline__ bool in_envelope_cert(const BvhWalk& W, L lst, P cert, int nl, M mask,
+                                                 V3<double> p, const CertFrame& F, double eps2,
+                                                 int& hl, bool& sure)
+{
+    const V3<float> q = cert_local(F, p);
+    uint64_t open[2] = {0ull, 0ull}, done[2] = {0ull, 0ull};
+    auto mark = [](uint64_t (&w)[2], int i) {
+        const uint64_t b = 1ull << (i & 63);
+        w[0] |= i < 64 ? b : 0ull;
+        w[1] |= i < 64 ? 0ull : b;
+    };
+    sure = true;
+    if (hl >= 0) {
+        const int r = cert_class(cert + kCertFloats * hl, q, F);
+        if (r > 0) return true;
+        mark(done, hl);
+        if (r == 0) mark(open, hl);
+        const uint32_t pk = NB ? (uint32_t)lst[hl].pad : 0xffffffffu;
+        if (NB)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const uint32_t u = (pk >> (8 * k)) & 0xffu;
+                if (u != 0xffu) {
+                    const int ru = cert_class(cert + kCertFloats * u, q, F);
+                    if (ru > 0) {
+                        hl = (int)u;
+                        return true;
+                    }
+                    mark(done, (int)u);
+                    if (ru == 0) mark(open, (int)u);
+                }
+            }
+    }
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        uint64_t mm = 64 * w < nl ? mask[w] & ~done[w] : 0ull;
+        while (mm) {
+            const int i = 64 * w + __builtin_ctzll(mm);
+            mm &= mm - 1;
+            const int r = cert_class(cert + kCertFloats * i, q, F);
+            if (r > 0) {
+                hl = i;
+                return true;
+            }
+            if (r == 0) open[w] |= 1ull << (i & 63);
+        }
+    }
+    sure = false;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        uint64_t mm = open[w];
+        while (mm) {
+            const int i = 64 * w + __builtin_ctzll(mm);
+            mm &= mm - 1;
+            if (facet_d2(W, lst[i].leaf, p) <= eps2) {
                 hl = i;
                 return true;
             }
@@ -1005,25 +1197,39 @@ __device__ bool face_out_listed(const BvhWalk& B, const double* t9, double eps2,
 
 // face_out_sampled's decision computed by a group of G lanes (G a power of
 // two up to 64, groups aligned in the wave; every lane of a group passes the
-// same triangle), against a collect_facets list (lst, tri, nl >= 0; its box
-// holding the triangle padded by more than sqrt(T)) or the tree (nl < 0).  The sampler's sequence of `total` samples is cut into G
+// same triangle), against a collect_facets list with its certificates (lst,
+// cert, F, nl >= 0; its box holding the triangle padded by more than sqrt(T))
+// or the tree (nl < 0).  A facet that certifies the three corners settles the
+// triangle.  Otherwise the sampler's sequence of `total` samples is cut into G
 // consecutive blocks of K = ceil(total / G); lane r moves to sample r K
 // (SampleGen::skip passes whole rows by their headers) and tests its block
-// in order, one sample per step, and after each step a ballot over the group
-// stops it at the first sample found outside.  The decision -- some sample
-// has no facet within eps -- does not depend on which lane tests which
-// sample, so it equals face_out_sampled's.  For batches of few triangles
-// with many samples each, where one lane per triangle leaves most of the
-// machine idle.
+// in order -- when a facet certifies a sample and the last one of the lane's
+// run along the same row, the ones between are passed over -- and after each
+// step a ballot over the group stops it at the first sample found outside.
+// The decision -- some sample has no facet within eps -- does not depend on
+// which lane tests which sample, so it equals face_out_sampled's.  For batches
+// of few triangles with many samples each, where one lane per triangle leaves
+// most of the machine idle.
 template <bool F32, int G, bool SUBTREE = true, bool NB = false>
 __device__ bool face_out_group(const BvhWalk& B, V3<double> a, V3<double> b, V3<double> c,
                                double eps2, double d, double T, double sqrtT, int r, int gbase,
-                               LdsNode32W* lst = nullptr, LdsF64c* tri = nullptr, int nl = -1)
+                               LdsNode32W* lst, LdsF32* cert, const CertFrame& F, int nl)
 {
     static_assert(G >= 2 && G <= 64 && (G & (G - 1)) == 0, "group size");
     {
         double l = fmax(len2(a - b), fmax(len2(b - c), len2(c - a)));
         if (!(__builtin_sqrt(l) / d <= kMaxEdgeSamples)) return true;
+    }
+    const unsigned long long gmask = G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull;
+    if (nl > 0 && F.runs) {
+        const V3<float> qa = cert_local(F, a), qb = cert_local(F, b), qc = cert_local(F, c);
+        bool all = false;
+        for (int e = r; e < nl; e += G) {
+            LdsF32* ce = cert + kCertFloats * e;
+            all = all || (cert_class(ce, qa, F) > 0 && cert_class(ce, qb, F) > 0 &&
+                          cert_class(ce, qc, F) > 0);
+        }
+        if ((__ballot(all) >> gbase) & gmask) return false;
     }
     int64_t total;
     {
@@ -1033,17 +1239,30 @@ __device__ bool face_out_group(const BvhWalk& B, V3<double> a, V3<double> b, V3<
     }
     const int64_t K = (total + G - 1) / G;
     const int64_t first = (int64_t)r * K;
+    const int64_t mine = total - first < K ? total - first : K;
     SampleGen g;
     g.init(a, b, c, d);
     g.skip(first);
     int hint = -1, hl = -1;
     Stats st;
-    const unsigned long long gmask = G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull;
-    for (int64_t j = 0; j < K; ++j) {
+    const uint64_t mask[2] = {~0ull >> (nl < 64 && nl > 0 ? 64 - nl : 0),
+                              nl > 64 ? ~0ull >> (128 - nl) : 0ull};
+    for (int64_t j = 0; (__ballot(j < mine) >> gbase) & gmask;) {
         V3<double> q = a;
-        const bool have = first + j < total && g.next(q);
-        const bool out = have && !(nl >= 0 ? in_envelope_list<NB>(lst, tri, nl, q, eps2, sqrtT, hl)
-                                           : in_envelope<F32, false, SUBTREE>(B, q, eps2, T, sqrtT, hint, st));
+        const bool have = j < mine && g.next(q);
+        bool out = false, sure = false;
+        if (have) {
+            if (nl >= 0) out = !in_envelope_cert<NB>(B, lst, cert, nl, mask, q, F, eps2, hl, sure);
+            else out = !in_envelope<F32, false, SUBTREE>(B, q, eps2, T, sqrtT, hint, st);
+        }
+        ++j;
+        if (sure && !out && F.runs && j < mine) {
+            const int64_t left = g.run_left(mine - j);
+            if (left > 0 && cert_class(cert + kCertFloats * hl, cert_local(F, g.run_at(left)), F) > 0) {
+                g.k += (int)left;
+                j += left;
+            }
+        }
         if ((__ballot(out) >> gbase) & gmask) return true;
     }
     return false;

@@ -407,6 +407,25 @@ struct SampleGen {
         }
     }
 
+    // the samples still to come of the run (edge or row) that the last sample
+    // lies on, at most `most`, and the left-th of them (the expressions of next())
+    __device__ __forceinline__ int64_t run_left(int64_t most) const
+    {
+        int64_t n = 0;
+        // (phase 5 with k = 1: the sample before was v2, not on the edge's run)
+        if (phase == 0 || phase == 7 || (phase == 5 && k > 1)) n = (int64_t)N - k + 1;
+        else if (phase == 3) n = (int64_t)N1 - k + 1;
+        return n < most ? n : most;
+    }
+    __device__ __forceinline__ V3<double> run_at(int64_t left) const
+    {
+        const double kk = (double)(k + left - 1);
+        if (phase == 3) return rowv + mulv(mulv(normalize(v1 - v0), kk), d);
+        const V3<double> s = phase == 0 ? v0 : (phase == 5 ? v1 : v2);
+        const V3<double> e = phase == 0 ? v1 : (phase == 5 ? v2 : v0);
+        return s + mulv(mulv(normalize(e - s), d), kk);
+    }
+
     // Writes what SampleGenC needs after init(): the (rotated) triangle, the
     // edge directions, the rows' angles and the edge counts, each computed
     // with the expression next() and skip() use.
@@ -695,6 +714,25 @@ struct SampleGenC {
                 return done;
             }
         }
+    }
+
+    // the samples still to come of the run (edge or row) that the last sample
+    // lies on, at most `most`, and the left-th of them (SampleGen's)
+    __device__ __forceinline__ int64_t run_left(int64_t most) const
+    {
+        int64_t n = 0;
+        // (phase 5 with k = 1: the sample before was v2, not on the edge's run)
+        if (phase == 0 || phase == 7 || (phase == 5 && k > 1)) n = (int64_t)N - k + 1;
+        else if (phase == 3) n = (int64_t)N1 - k + 1;
+        return n < most ? n : most;
+    }
+    __device__ __forceinline__ V3<double> run_at(int64_t left) const
+    {
+        const double kk = (double)(k + left - 1);
+        if (phase == 3) return rowv + mulv(mulv(at(kFrN01), kk), d);
+        const int so = phase == 0 ? kFrV0 : (phase == 5 ? kFrV1 : kFrV2);
+        const int eo = phase == 0 ? kFrN01 : (phase == 5 ? kFrN12 : kFrN20);
+        return at(so) + mulv(mulv(at(eo), d), kk);
     }
 
     // SampleGen::next
