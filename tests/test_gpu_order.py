@@ -1,0 +1,69 @@
+"""The query order and the list kernels' edges: batches around a sort tile, the
+two- and three-pass sorts, clustered and degenerate boxes, and waves whose
+facets overflow their list, each against the per-query tree walk (the
+statistics path, whose decisions the other tests pin to the oracle)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [65536, 65537, 4096 * 17 - 1, (1 << 18) - 1, 1 << 18, 300001])
+@pytest.mark.parametrize("where", ["spread", "cluster", "one_place"])
+def test_sorted_batches(n, where):
+    import torch
+
+    from tetwild_amd import workloads as W
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    V, F = W.bumpy_sphere(freq=24, seed=2)
+    surf = ctx.surface(V, F)
+    eps = 2e-3
+    Q = W.query_triangles(V, F, n, eps=eps, edge=0.004, seed=n % 7)
+    if where != "spread":  # about one facet, the last items far away and not finite
+        c = V[F[5]].mean(0)
+        Q = c + (Q.reshape(n, 3, 3) * (0.02 if where == "cluster" else 0.0)).reshape(n, 3, 3)
+        if where == "one_place":
+            Q = Q + np.array([[0, 0, 0], [0.004, 0, 0], [0, 0.004, 0.001]])
+        Q[-3:-1] += 1e6
+        Q = np.ascontiguousarray(Q.reshape(n, 9))
+        Q[-1, 4] = np.inf
+    tq = torch.from_numpy(Q).to("cuda:0")
+    for prec in (0, 1):
+        out = ctx.envelope_faces(surf, tq, eps * eps, eps, precision=prec)
+        walk, _ = ctx.envelope_faces(surf, tq, eps * eps, eps, precision=prec, stats=True)
+        assert torch.equal(out, walk), (prec, int((out != walk).sum()))
+        p3 = tq[:, :3].contiguous()
+        pout = ctx.envelope_points(surf, p3, eps * eps, precision=prec)
+        pwalk, _ = ctx.envelope_points(surf, p3, eps * eps, precision=prec, stats=True)
+        assert torch.equal(pout, pwalk), prec
+    ctx.close()
+
+
+@pytest.mark.parametrize("eps,edge", [(1e-3, 0.03), (0.05, 0.02), (1e-9, 1e-7), (0.0, 0.004)])
+def test_lists_overflow_and_limits(eps, edge):
+    """Dense facets under wide queries (every list overflows), an envelope wider
+    than the facets, one far below the coordinates' rounding, and eps = 0"""
+    import torch
+
+    from tetwild_amd import workloads as W
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    V, F = W.bumpy_sphere(freq=40, seed=3)
+    surf = ctx.surface(V, F)
+    d = max(eps, 1e-9) if edge < 1e-3 else max(eps, 2e-3)
+    Q = W.query_triangles(V, F, 70000, eps=eps, edge=edge, seed=5)
+    for nf in (len(F), 700):  # 2.2 and 100 queries a facet
+        s = surf if nf == len(F) else ctx.surface(V, F[:nf])
+        tq = torch.from_numpy(Q).to("cuda:0")
+        for prec in (0, 1):
+            out = ctx.envelope_faces(s, tq, eps * eps, d, precision=prec)
+            walk, _ = ctx.envelope_faces(s, tq, eps * eps, d, precision=prec, stats=True)
+            assert torch.equal(out, walk), (nf, prec, int((out != walk).sum()))
+            p3 = tq[:, :3].contiguous()
+            assert torch.equal(ctx.envelope_points(s, p3, eps * eps, precision=prec),
+                               ctx.envelope_points(s, p3, eps * eps, precision=prec, stats=True)[0])
+        small = tq[:200].contiguous()  # a wave per triangle
+        o = ctx.envelope_faces(s, small, eps * eps, d)
+        assert torch.equal(o, ctx.envelope_faces(s, small, eps * eps, d, stats=True)[0])
+    ctx.close()

@@ -50,76 +50,103 @@ __global__ __launch_bounds__(kBlock) void points_kernel(BvhView B, const double*
     if (STATS) flush_stats(st, stats);
 }
 
+// xcd_block for work that is uneven along the items (sorted queries): each XCD
+// takes runs of 64 consecutive blocks in turn instead of a contiguous eighth,
+// so no XCD is left with a long eighth (3 M triangles 2187 -> 1812 us with the
+// one-wave blocks of faces_list_kernel: 31 % of the CU time had been idle).
+__device__ __forceinline__ int64_t xcd_run_block()
+{
+    const unsigned g = gridDim.x, b = blockIdx.x;
+    const unsigned whole = g / 512 * 512;
+    if (b >= whole) return b;
+    const unsigned k = b / 8;
+    return (int64_t)(k / 64) * 512 + (b % 8) * 64 + k % 64;
+}
+
+// Waves whose facets do not fit their list take their items in halves, down to
+// this many lanes.
+constexpr int kListSplit = 8;
+
 // points_kernel for batches walked in Morton order with many points per
 // facet: the wave's 64 consecutive points lie close together, so the wave
 // lists once (collect_facets, LDS) the facets whose boxes meet the box of its
-// points padded by more than sqrt(T), with their triangles, and each lane
-// tests its point against the list (in_envelope_list).  A wave whose list
-// exceeds CAP entries, or that holds a coordinate that is not finite, walks
-// the tree (from global memory: the LDS holds the lists).
+// points padded by more than sqrt(T), with their certificates, and each lane
+// tests its point against the list (in_envelope_cert).  Blocks of one wave and
+// split waves as faces_list_kernel; lanes that no list serves, or that hold a
+// coordinate that is not finite, walk the tree.
 template <bool F32, int CAP>
-__global__ __launch_bounds__(kBlock) void points_list_kernel(BvhView B, const double* __restrict__ p3,
-                                                             int64_t n, double eps2, double T,
-                                                             double sqrtT, uint8_t* __restrict__ out,
-                                                             const int32_t* __restrict__ order,
-                                                             unsigned long long* lstat)
+__global__ __launch_bounds__(64) void points_list_kernel(BvhView B, const double* __restrict__ p3,
+                                                         int64_t n, double eps2, double T,
+                                                         double sqrtT, uint8_t* __restrict__ out,
+                                                         const int32_t* __restrict__ order,
+                                                         unsigned long long* lstat)
 {
-    constexpr int kWaveBytes = CAP * (32 + 8 + 72);
-    __shared__ __align__(16) unsigned char lists[(kBlock / 64) * kWaveBytes];
+    __shared__ __align__(16) unsigned char mine[CAP * kCertEntryBytes];
     const BvhWalk W = walk(B);
-    const int lane = threadIdx.x % 64;
-    unsigned char* mine = lists + (threadIdx.x / 64) * kWaveBytes;
+    const int lane = threadIdx.x;
     LdsNode32W* lst = (LdsNode32W*)mine;
-    LdsU32* fr = (LdsU32*)(mine + CAP * 32);
-    LdsF64* tri = (LdsF64*)(mine + CAP * 40);
-    int64_t i = xcd_block() * kBlock + threadIdx.x;
-    const bool act = i < n;
+    LdsU32* fr = (LdsU32*)(mine + CAP * 32);  // the work lists, then the certificates
+    LdsF32* cert = (LdsF32*)(mine + CAP * 32);
+    int64_t i = xcd_run_block() * 64 + lane;
+    const bool have = i < n;
     V3<double> p = mk3(0.0, 0.0, 0.0);
-    if (act) {
+    if (have) {
         if (order) i = order[i];
         p = ld3(p3 + 3 * i);
     }
-    double lo[3] = {act ? p.x : INFINITY, act ? p.y : INFINITY, act ? p.z : INFINITY};
-    double hi[3] = {act ? p.x : -INFINITY, act ? p.y : -INFINITY, act ? p.z : -INFINITY};
-    double amax = 0.0;
+    const bool fin = is_finite(p.x) && is_finite(p.y) && is_finite(p.z);
+    bool walked = false;
+    for (int s = 0, w = 64; s < 64;) {
+        const bool act = have && lane >= s && lane < s + w;
+        if (__ballot(act)) {
+            double lo[3] = {act ? p.x : INFINITY, act ? p.y : INFINITY, act ? p.z : INFINITY};
+            double hi[3] = {act ? p.x : -INFINITY, act ? p.y : -INFINITY, act ? p.z : -INFINITY};
+            double amax = 0.0;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        for (int off = 32; off > 0; off >>= 1) {
-            const double ol = __shfl_xor(lo[k], off, 64), oh = __shfl_xor(hi[k], off, 64);
-            lo[k] = ol < lo[k] ? ol : lo[k];
-            hi[k] = oh > hi[k] ? oh : hi[k];
+            for (int k = 0; k < 3; ++k) {
+                for (int off = 32; off > 0; off >>= 1) {
+                    const double ol = __shfl_xor(lo[k], off, 64), oh = __shfl_xor(hi[k], off, 64);
+                    lo[k] = ol < lo[k] ? ol : lo[k];
+                    hi[k] = oh > hi[k] ? oh : hi[k];
+                }
+                amax = fmax(amax, fmax(fabs(lo[k]), fabs(hi[k])));
+            }
+            const double pad = 1.0001 * sqrtT + 1e-9 * amax;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                lo[k] -= pad;
+                hi[k] += pad;
+            }
+            // a coordinate that is not finite can leave the lanes with different
+            // boxes (min / max ignore NaN): no list for them
+            const int nl = __ballot(act && !fin) ? -1 : collect_facets<64>(W, lo, hi, lst, fr, CAP, lane, 0);
+            if (nl >= 0) {
+                const CertFrame F = cert_frame(lo, hi, amax, eps2, 1.0);
+                cert_list<64>(W, lst, cert, nl, F, eps2, lane);
+                if (act) {
+                    uint64_t mk[2];
+                    int hl = -1;
+                    bool sure;
+                    point_list_mask(lst, nl, p, sqrtT, mk);
+                    out[i] = in_envelope_cert<false>(W, lst, cert, nl, mk, p, F, eps2, hl, sure) ? 0 : 1;
+                }
+                wave_sync();  // the list's last reads
+            } else if (w > kListSplit) {
+                w /= 2;
+                continue;
+            } else {
+                walked = true;
+                if (act) {
+                    int hint = -1;
+                    Stats st;
+                    out[i] = in_envelope<F32, false>(W, p, eps2, T, sqrtT, hint, st) ? 0 : 1;
+                }
+            }
         }
-        amax = fmax(amax, fmax(fabs(lo[k]), fabs(hi[k])));
+        s += w;
+        w = s & -s;
     }
-    const double pad = 1.0001 * sqrtT + 1e-9 * amax;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        lo[k] -= pad;
-        hi[k] += pad;
-    }
-    // a coordinate that is not finite can leave the lanes with different
-    // boxes (min / max ignore NaN): then the whole wave walks the tree
-    const bool fin = !act || (is_finite(p.x) && is_finite(p.y) && is_finite(p.z));
-    const int nl = __ballot(!fin) ? -1 : collect_facets<64>(W, lo, hi, lst, fr, CAP, lane, 0);
-    if (lstat && lane == 0) atomicAdd(lstat + (nl >= 0 ? 0 : 1), 1ull);
-    for (int e = lane; e < nl; e += 64) {
-        const double* f = B.tri + 9 * (int64_t)lst[e].leaf;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) tri[9 * e + k] = f[k];
-    }
-    wave_sync();
-    if (act) {
-        bool in;
-        if (nl >= 0) {
-            int hl = -1;
-            in = in_envelope_list(lst, tri, nl, p, eps2, sqrtT, hl);
-        } else {
-            int hint = -1;
-            Stats st;
-            in = in_envelope<F32, false>(W, p, eps2, T, sqrtT, hint, st);
-        }
-        out[i] = in ? 0 : 1;
-    }
+    if (lstat && lane == 0) atomicAdd(lstat + (walked ? 1 : 0), 1ull);
 }
 
 // Triangles the degeneracy filter cannot settle are queued (pending[],
@@ -162,27 +189,20 @@ struct WaveFace {
     float mlo[3], mhi[3];
 };
 
-// face_out_sampled for the wave's 64 triangles at once (a list of nl <= 128
-// facets, nl >= 0, with its certificates).  Every lane scans the facets near its triangle
-// for one that holds its first corner: none, and the triangle is out; one
-// that certifies all three corners, and it is in.  The samples of the
-// triangles still open -- they straddle facets, or reach the limit -- are
-// then spread over the wave: the concatenation of their sequences (the first
-// samples left out) is cut into 64 consecutive blocks of K = ceil(total / 64)
-// and lane r walks block r, moving to the next open triangle when one ends
-// and passing over the samples between two certified by one facet on one
-// row.  A lane takes the triangle it moves to -- its corners' address, list
-// mask and the facet that held its first sample -- from the triangle's own
-// lane (shuffles, every lane active; the corners are read again from memory,
-// which keeps 18 registers free through the walk), and a sample found outside
-// is passed to that lane by ballot.  The decision -- some sample has no facet
-// within eps -- does not depend on which lane tests which sample, so it is
-// face_out_sampled's.  Returns the lane's own triangle's decision.
+// face_out_sampled for the wave's triangles at once (a list of nl <= 128
+// facets, nl >= 0, with its certificates).  Every lane scans the facets near
+// its triangle for one that holds its first corner: none, and the triangle is
+// out; one that certifies all three corners, and it is in.  The few triangles
+// still open -- they straddle facets, or reach the limit -- are sampled by
+// their lanes, which pass over the samples between two that one facet
+// certifies on a row.  (Spreading the open triangles' samples over the wave
+// takes two more samplers per lane and their registers: 3 M triangles of 6-11
+// samples 1568 us against 1551, of ~20 samples 3205 against 3028.)  Returns the
+// lane's decision.
 __device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double eps2, double d,
-                                  LdsNode32W* lst, LdsF32* cert, int nl, const CertFrame& F, int lane)
+                                  LdsNode32W* lst, LdsF32* cert, int nl, const CertFrame& F)
 {
     bool out = T.act, open_lane = false;
-    int64_t rem = 0;  // samples after the first, while the triangle is open
     uint64_t mk[2] = {0ull, 0ull};
     int hl = -1;
     const double* t9 = T.t9;
@@ -217,85 +237,22 @@ __device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double ep
         out = hl < 0;
         open_lane = hl >= 0 && !all;
     }
-    if (__ballot(open_lane) == 0ull) return out;
     if (open_lane) {
         SampleGen g;
         g.init(ld3(t9), ld3(t9 + 3), ld3(t9 + 6), d);
-        rem = g.skip(INT64_MAX) - 1;
-    }
-    const unsigned long long open = __ballot(rem > 0);
-    int64_t incl = rem;
-    for (int off = 1; off < 64; off <<= 1) {
-        const int64_t o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-    }
-    const int64_t total = __shfl(incl, 63, 64);
-    const int64_t K = (total + 63) / 64;
-    const int64_t first = (int64_t)lane * K;
-    const int64_t mine = total - first < K ? total - first : K;
-    // the triangle holding remaining sample `first`: the first lane f with
-    // incl[f] > first (a binary search, each lane its own)
-    int f = 0;
-    for (int step = 32; step > 0; step >>= 1) {
-        const int probe = f + step - 1;
-        const int64_t v = __shfl(incl, probe < 63 ? probe : 63, 64);
-        if (probe < 63 && v <= first) f = probe + 1;
-    }
-    if (first >= total) f = 64;  // no samples for this lane
-    const int fs = f < 64 ? f : lane;
-    const int64_t ofs = first - (__shfl(incl, fs, 64) - __shfl(rem, fs, 64));
-    // the lane's triangle: corners, mask and hint from its owner
-    SampleGen g2;
-    uint64_t m2[2];
-    int h2;
-    {
-        const double* ct = (const double*)__shfl((long long)(uintptr_t)t9, fs, 64);
-        m2[0] = __shfl(mk[0], fs, 64);
-        m2[1] = __shfl(mk[1], fs, 64);
-        h2 = __shfl(hl, fs, 64);
-        if (f < 64) {
-            g2.init(ld3(ct), ld3(ct + 3), ld3(ct + 6), d);
-            g2.skip(1 + ofs);
-        }
-    }
-    for (int64_t j = 0; __ballot(j < mine);) {
-        const bool have = j < mine;
         V3<double> s;
-        bool got = have && g2.next(s);
-        const bool need = have && !got;
-        if (__ballot(need)) {
-            // the next open triangle after f (one exists: first + j < total)
-            const unsigned long long later = f >= 63 ? 0ull : open & ~((2ull << f) - 1ull);
-            const int nf = need && later ? __ffsll((long long)later) - 1 : lane;
-            const double* ct = (const double*)__shfl((long long)(uintptr_t)t9, nf, 64);
-            const uint64_t n0 = __shfl(mk[0], nf, 64), n1 = __shfl(mk[1], nf, 64);
-            const int nh = __shfl(hl, nf, 64);
-            if (need && later) {
-                f = nf;
-                m2[0] = n0;
-                m2[1] = n1;
-                h2 = nh;
-                g2.init(ld3(ct), ld3(ct + 3), ld3(ct + 6), d);
-                g2.skip(1);
-                got = g2.next(s);
+        g.next(s);  // the first corner
+        while (g.next(s)) {
+            bool sure;
+            if (!in_envelope_cert<false>(W, lst, cert, nl, mk, s, F, eps2, hl, sure)) {
+                out = true;
+                break;
             }
-        }
-        bool sure = false;
-        const bool o2 = got && !in_envelope_cert<false>(W, lst, cert, nl, m2, s, F, eps2, h2, sure);
-        ++j;
-        if (got && sure && F.runs && j < mine) {
-            const int64_t left = g2.run_left(mine - j);
-            if (left > 0 && cert_class(cert + kCertFloats * h2, cert_local(F, g2.run_at(left)), F) > 0) {
-                g2.k += (int)left;
-                j += left;
+            if (sure && F.runs) {
+                const int64_t left = g.run_left(INT64_MAX);
+                if (left > 0 && cert_class(cert + kCertFloats * hl, cert_local(F, g.run_at(left)), F) > 0)
+                    g.k += (int)left;
             }
-        }
-        // the triangles found outside, to their lanes
-        unsigned long long ob = __ballot(o2);
-        while (ob) {
-            const int l = __ffsll((long long)ob) - 1;
-            ob &= ob - 1;
-            if (__shfl(f, l, 64) == lane) out = true;
         }
     }
     return out;
@@ -307,28 +264,15 @@ __device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double ep
 // triangles padded by more than sqrt(T), with their certificates, and tests
 // its triangles against the list (faces_wave_listed) instead of walking the
 // tree per sample.  Blocks of one wave: a block's LDS is free for the next one
-// as soon as its wave ends.  3 M triangles on 246 k facets: 2.73 -> 1.37 ms
-// for the kernel, with the certificates, the wider tree rounds of
-// collect_facets, the rows through LDS, the split waves and the short blocks;
-// half of what is left waits for memory, the VALU is busy for a third of it.
-// xcd_block for work that is uneven along the items (sorted queries): each XCD
-// takes runs of 64 consecutive blocks in turn instead of a contiguous eighth,
-// so no XCD is left with a long eighth (3 M triangles 2187 -> 1812 us with the
-// one-wave blocks of faces_list_kernel: 31 % of the CU time had been idle).
-__device__ __forceinline__ int64_t xcd_run_block()
-{
-    const unsigned g = gridDim.x, b = blockIdx.x;
-    const unsigned whole = g / 512 * 512;
-    if (b >= whole) return b;
-    const unsigned k = b / 8;
-    return (int64_t)(k / 64) * 512 + (b % 8) * 64 + k % 64;
-}
-
-constexpr int kFaceSplit = 8;
-template <bool F32, int CAP>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void faces_list_kernel(
-    BvhView B, const double* __restrict__ tri9, int64_t n, double eps2, double d, double T_,
-    double sqrtT, uint8_t* __restrict__ out, unsigned* n_pending, int64_t* pending,
+// as soon as its wave ends.  Three waves a SIMD hold its 168 registers (four
+// spill 70 of them: 1574 us a call against 1423).  3 M triangles on 246 k
+// facets: 2.73 -> 1.22 ms for the kernel, with the certificates, the wider tree
+// rounds of collect_facets, the rows through LDS, the split waves, the short
+// blocks and the open triangles on their own lanes; the VALU is busy for some
+// 40 % of it, the rest waits for the list's chain of reads.
+template <int CAP>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void faces_list_kernel(
+    BvhView B, const double* __restrict__ tri9, int64_t n, double eps2, double d, double T_, double sqrtT, uint8_t* __restrict__ out, unsigned* n_pending, int64_t* pending,
     const int32_t* __restrict__ order, unsigned long long* lstat)
 {
     constexpr int kWaveBytes = CAP * kCertEntryBytes;
@@ -376,7 +320,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     }
     // The lanes [s, s + w) at a time: all 64, unless their facets do not fit the
     // list -- the Morton order jumps inside the wave, say -- then its halves, down
-    // to kFaceSplit lanes, which walk the tree.  (Whole waves walking it, 5.8 %
+    // to kListSplit lanes, which walk the tree.  (Whole waves walking it, 5.8 %
     // of them, ran on alone for half of the kernel's time.)
     bool walked = false;
     for (int s = 0, w = 64; s < 64;) {
@@ -423,16 +367,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
                 U.q[1] = cert_local(F, sel3(U.first, b, c, a));
                 U.q[2] = cert_local(F, sel3(U.first, c, a, b));
                 cert_list<64>(W, lst, cert, nl, F, eps2, lane);
-                const bool o = faces_wave_listed(W, U, eps2, d, lst, cert, nl, F, lane);
+                const bool o = faces_wave_listed(W, U, eps2, d, lst, cert, nl, F);
                 if (U.act) out[i] = o ? 1 : 0;
                 wave_sync();  // the list's last reads
-            } else if (w > kFaceSplit) {
+            } else if (w > kListSplit) {
                 w /= 2;
                 continue;
             } else {
+                // (left to the exact pass: 1551 -> 1685 us)
                 walked = true;
                 Stats st;
-                if (U.act) out[i] = face_out_sampled<F32, false>(W, T.t9, eps2, d, T_, sqrtT, st) ? 1 : 0;
+                if (U.act) out[i] = face_out_sampled<true, false>(W, T.t9, eps2, d, T_, sqrtT, st) ? 1 : 0;
             }
         }
         s += w;
@@ -538,18 +483,17 @@ __global__ void zero_u64x2(unsigned long long* p)
 constexpr int64_t kSortMin = 1 << 16;
 // face batches below this size run a wave per triangle (faces_group_kernel)
 constexpr int64_t kWaveMax = 1 << 16;
-// facets per wave list in faces_list_kernel (80: four blocks per CU; the
-// kernel keeps no LDS copy of the tree top -- 48 entries with a 16 KB copy
-// ran 8 % slower), and the queries per facet from which a wave's 64
-// triangles (about 64 / density facets apart) usually fit it: measured on
-// 1 M facets, 20 M queries ran 540 -> 720 M checks/s with the lists, 2 M
-// queries 422 -> 395 (overflowing lists), so sparser batches keep faces_kernel
+// Facets per wave list in faces_list_kernel, and the queries per facet from
+// which a wave's 64 triangles (about 64 / density facets apart) fit it whole or
+// in halves.  Measured against faces_kernel: 800 k triangles on 246 k facets
+// (3.2 a facet) 1629 -> 1027 us with the lists, 200 k on 512 k (0.4) 1082 ->
+// 2153, so sparser batches keep faces_kernel.
 constexpr int kFaceListCap = 80;
-constexpr int64_t kFaceListDensity = 8;
-// the same for points_list_kernel (64 entries, no LDS copy of the tree top:
-// 32 entries with a 16 KB copy ran 2.00 G checks/s on 20 M points, this 2.92 G)
+constexpr int64_t kFaceListDensity = 2;
+// the same for points_list_kernel: 1 M points on 246 k facets (4 a facet) 593
+// -> 576 us, 4 M on 72 k (56) 980 -> 829, but 300 k on 512 k (0.6) 418 -> 822
 constexpr int kPointListCap = 64;
-constexpr int64_t kPointListDensity = 8;
+constexpr int64_t kPointListDensity = 2;
 
 __global__ __launch_bounds__(kBlock) void nearest_kernel(BvhView B, const double* __restrict__ p3,
                                                          int64_t n, double* __restrict__ cp3,
@@ -896,9 +840,9 @@ int twg_envelope_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_
         if (int r = morton_order(ctx, p3, n, 3, B->lo, B->hi, &order)) return r;
     if (order && !stats && n >= kPointListDensity * B->nf) {
         if (precision == TWG_FP64)
-            hipLaunchKernelGGL((points_list_kernel<false, kPointListCap>), g, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
+            hipLaunchKernelGGL((points_list_kernel<false, kPointListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, p3, n, eps2, T, sT, out, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
         else
-            hipLaunchKernelGGL((points_list_kernel<true, kPointListCap>), g, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
+            hipLaunchKernelGGL((points_list_kernel<true, kPointListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, p3, n, eps2, T, sT, out, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
     } else if (precision == TWG_FP64) {
         if (stats) hipLaunchKernelGGL((points_kernel<false, true>), g, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out, stats, order);
         else hipLaunchKernelGGL((points_kernel<false, false>), g, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out, stats, order);
@@ -937,10 +881,8 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
         else
             hipLaunchKernelGGL((faces_group_kernel<true, 64>), gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order);
     } else if (order && !stats && n >= kFaceListDensity * B->nf) {
-        if (precision == TWG_FP64)
-            hipLaunchKernelGGL((faces_list_kernel<false, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
-        else
-            hipLaunchKernelGGL((faces_list_kernel<true, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
+        // (the list's boxes, and the few tree walks', are the FP32 ones in either precision)
+        hipLaunchKernelGGL(faces_list_kernel<kFaceListCap>, dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
     } else if (precision == TWG_FP64) {
         if (stats) hipLaunchKernelGGL((faces_kernel<false, true>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, stats, n_pending, pending, order);
         else hipLaunchKernelGGL((faces_kernel<false, false>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, stats, n_pending, pending, order);

@@ -722,6 +722,33 @@ __device__ __forceinline__ bool in_envelope_masked(LdsNode32W* lst, LdsF64c* tri
     return false;
 }
 
+// The positions of a collect_facets list (nl <= 128 entries) whose FP32 boxes
+// can hold a facet within sqrt(T) of p (the tree walk's box test)
+template <class L>
+__device__ __forceinline__ void point_list_mask(L lst, int nl, V3<double> p, double sqrtT, uint64_t mk[2])
+{
+    const V3<float> pf = mk3((float)p.x, (float)p.y, (float)p.z);
+    const float Tf = f32_threshold(p, sqrtT);
+    uint64_t w[2] = {0ull, 0ull};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int e1 = nl - 64 * h < 64 ? nl - 64 * h : 64;
+        uint64_t m = 0ull;
+        for (int e0 = 0; e0 < e1; e0 += 8) {  // eight records read before their tests
+            BvhNode32 r[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (e0 + u < e1) r[u] = from_lds(lst + 64 * h + e0 + u);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (e0 + u < e1) m |= (uint64_t)(box_d2(pf, r[u].lo, r[u].hi) <= Tf) << (e0 + u);
+        }
+        w[h] = m;
+    }
+    mk[0] = w[0];
+    mk[1] = w[1];
+}
+
 // ---- certified FP32 decisions for the listed facets ------------------------
 // A sample's exact test against a facet (point_tri_d2, FP64) is some 240
 // instructions once the lanes of a wave diverge over its seven regions, and a
