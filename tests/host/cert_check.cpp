@@ -155,7 +155,7 @@ int main()
             int hl = -1;
             if (mask[0] && rng() % 2) hl = __builtin_ctzll(mask[0]);
             bool sure = false;
-            const bool got = in_envelope_cert<false>(W, L.data(), C.data(), nl, mask, p, S.F, S.eps2, hl, sure);
+            const bool got = in_envelope_cert(W, L.data(), C.data(), nl, mask, p, S.F, S.eps2, hl, sure);
             CHECK(got == ref, "set %d: list decision %d, FP64 %d\n", s, got, ref);
             CHECK(!got || (hl >= 0 && d2(&T[9 * hl], p) <= S.eps2), "set %d: the facet left does not hold p\n", s);
             ++lists;

@@ -6,8 +6,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <vector>
 
+#include "build.hpp"
 #include "twg_bvh.hpp"
 #include "twg_internal.hpp"
 
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(64) void points_list_kernel(BvhView B, const double
                     int hl = -1;
                     bool sure;
                     point_list_mask(lst, nl, p, sqrtT, mk);
-                    out[i] = in_envelope_cert<false>(W, lst, cert, nl, mk, p, F, eps2, hl, sure) ? 0 : 1;
+                    out[i] = in_envelope_cert(W, lst, cert, nl, mk, p, F, eps2, hl, sure) ? 0 : 1;
                 }
                 wave_sync();  // the list's last reads
             } else if (w > kListSplit) {
@@ -244,7 +246,7 @@ __device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double ep
         g.next(s);  // the first corner
         while (g.next(s)) {
             bool sure;
-            if (!in_envelope_cert<false>(W, lst, cert, nl, mk, s, F, eps2, hl, sure)) {
+            if (!in_envelope_cert(W, lst, cert, nl, mk, s, F, eps2, hl, sure)) {
                 out = true;
                 break;
             }
@@ -449,9 +451,8 @@ __global__ __launch_bounds__(kBlock) void faces_group_kernel(BvhView B, const do
         nl = fin ? collect_facets<64>(walk(B), lo, hi, lst, fr, kGroupListCap, r, 0) : -1;
         F = cert_frame(lo, hi, amax, eps2, d);
         cert_list<64>(W, lst, cert, nl, F, eps2, r);
-        list_neighbours<64>(walk(B), lst, nl, r);
     }
-    const bool o = face_out_group<F32, G, true, true>(W, ld3(t), ld3(t + 3), ld3(t + 6), eps2, d, T, sqrtT, r,
+    const bool o = face_out_group<F32, G>(W, ld3(t), ld3(t + 3), ld3(t + 6), eps2, d, T, sqrtT, r,
                                                       gbase, lst, cert, F, nl);
     if (r == 0) out[i] = o ? 1 : 0;
 }
@@ -616,6 +617,11 @@ float round_up(double v)
 
 using namespace twg;
 
+// Surfaces from this size on are built on the device (build.hip), smaller ones
+// on the host: 64 facets take 59 us on the host and 169 on the device, 512 take
+// 187 and 180, 5,120 take 2.0 ms and 0.32, 246,420 take 121 ms and 0.96.
+constexpr int64_t kDeviceBuildMin = 512;
+
 extern "C" {
 
 int twg_bvh_build(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F, int64_t nf,
@@ -624,6 +630,18 @@ int twg_bvh_build(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F, i
     TWG_REQUIRE(ctx && out, "twg_bvh_build: NULL argument");
     TWG_REQUIRE(nf >= 1 && nv >= 1 && V && F, "twg_bvh_build: empty surface");
     TWG_REQUIRE(nf < (int64_t(1) << 30), "twg_bvh_build: too many facets (%lld)", (long long)nf);
+    if (nf >= kDeviceBuildMin && nv < (int64_t(1) << 31)) {
+        if (int r = bind(ctx)) return r;
+        std::unique_ptr<twg_bvh, int (*)(twg_bvh*)> B(new twg_bvh(), twg_bvh_destroy);
+        B->device = ctx->device;
+        B->nf = nf;
+        int64_t bad = -1;
+        if (int r = bvh_build_device(ctx, V, nv, F, nf, B.get(), &bad)) return r;
+        TWG_REQUIRE(bad < 0, "twg_bvh_build: facet %lld has vertex id %d outside [0, %lld)",
+                    (long long)(bad / 3), F[bad], (long long)nv);
+        *out = B.release();
+        return TWG_OK;
+    }
     for (int64_t f = 0; f < 3 * nf; ++f)
         TWG_REQUIRE(F[f] >= 0 && F[f] < nv, "twg_bvh_build: facet %lld has vertex id %d outside [0, %lld)",
                     (long long)(f / 3), F[f], (long long)nv);
@@ -672,59 +690,6 @@ int twg_bvh_build(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F, i
         }
     }
     B->rmax = rmax;
-    // edge adjacency in tree order: corners identified by their coordinates'
-    // bits (facets of a triangle soup share edges too); edges of one vertex
-    // twice are skipped; an edge of more than two facets links them in a cycle
-    std::vector<int32_t> adj(3 * nf, -1);
-    {
-        const int64_t nc = 3 * nf;
-        auto bits = [&](int64_t c, int k) {
-            uint64_t u;
-            std::memcpy(&u, &tri[3 * c + k], 8);
-            return u;
-        };
-        std::vector<int64_t> corner(nc);
-        for (int64_t c = 0; c < nc; ++c) corner[c] = c;
-        std::sort(corner.begin(), corner.end(), [&](int64_t a, int64_t b) {
-            for (int k = 0; k < 3; ++k)
-                if (bits(a, k) != bits(b, k)) return bits(a, k) < bits(b, k);
-            return a < b;
-        });
-        std::vector<int64_t> vid(nc);
-        int64_t id = -1;
-        for (int64_t i = 0; i < nc; ++i) {
-            const int64_t c = corner[i];
-            if (i == 0 || bits(c, 0) != bits(corner[i - 1], 0) || bits(c, 1) != bits(corner[i - 1], 1) ||
-                bits(c, 2) != bits(corner[i - 1], 2))
-                ++id;
-            vid[c] = id;
-        }
-        struct Edge {
-            int64_t a, b;
-            int64_t slot;  // 3 facet + k
-        };
-        std::vector<Edge> es;
-        es.reserve(nc);
-        for (int64_t f = 0; f < nf; ++f)
-            for (int k = 0; k < 3; ++k) {
-                const int64_t u = vid[3 * f + k], w = vid[3 * f + (k + 1) % 3];
-                if (u != w) es.push_back({std::min(u, w), std::max(u, w), 3 * f + k});
-            }
-        std::sort(es.begin(), es.end(), [](const Edge& x, const Edge& y) {
-            return x.a != y.a ? x.a < y.a : (x.b != y.b ? x.b < y.b : x.slot < y.slot);
-        });
-        for (size_t i = 0; i < es.size();) {
-            size_t j = i;
-            while (j < es.size() && es[j].a == es[i].a && es[j].b == es[i].b) ++j;
-            if (j - i >= 2)
-                for (size_t r = i; r < j; ++r) {
-                    const size_t o = r + 1 < j ? r + 1 : i;
-                    adj[es[r].slot] = (int32_t)(es[o].slot / 3);
-                    if (j - i == 2) adj[es[o].slot] = (int32_t)(es[r].slot / 3);
-                }
-            i = j;
-        }
-    }
     B->nnode = max_node(1, 0, nf) + 1;
     std::vector<BvhNode64> nodes(B->nnode);
     for (auto& N : nodes) {
@@ -758,23 +723,23 @@ int twg_bvh_build(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F, i
     }
     int r = bind(ctx);
     hipError_t e = hipSuccess;
-    if (!r) e = hipMalloc(&B->node64, sizeof(BvhNode64) * B->nnode);
-    if (!r && e == hipSuccess) e = hipMalloc(&B->node32, sizeof(BvhNode32) * B->nnode);
-    if (!r && e == hipSuccess) e = hipMalloc(&B->tri, sizeof(double) * 9 * nf);
-    if (!r && e == hipSuccess) e = hipMalloc(&B->adj, sizeof(int32_t) * 3 * nf);
-    if (!r && e == hipSuccess)
+    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const size_t b64 = up(sizeof(BvhNode64) * B->nnode), b32 = up(sizeof(BvhNode32) * B->nnode),
+                 btri = up(sizeof(double) * 9 * nf);
+    if (!r) e = hipMalloc(&B->mem, b64 + b32 + btri);
+    if (!r && e == hipSuccess) {
+        char* m = static_cast<char*>(B->mem);
+        B->node64 = reinterpret_cast<BvhNode64*>(m);
+        B->node32 = reinterpret_cast<BvhNode32*>(m + b64);
+        B->tri = reinterpret_cast<double*>(m + b64 + b32);
         e = hipMemcpy(B->node64, nodes.data(), sizeof(BvhNode64) * B->nnode, hipMemcpyHostToDevice);
+    }
     if (!r && e == hipSuccess)
         e = hipMemcpy(B->node32, n32.data(), sizeof(BvhNode32) * B->nnode, hipMemcpyHostToDevice);
     if (!r && e == hipSuccess)
         e = hipMemcpy(B->tri, tri.data(), sizeof(double) * 9 * nf, hipMemcpyHostToDevice);
-    if (!r && e == hipSuccess)
-        e = hipMemcpy(B->adj, adj.data(), sizeof(int32_t) * 3 * nf, hipMemcpyHostToDevice);
     if (r || e != hipSuccess) {
-        if (B->node64) (void)hipFree(B->node64);
-        if (B->node32) (void)hipFree(B->node32);
-        if (B->tri) (void)hipFree(B->tri);
-        if (B->adj) (void)hipFree(B->adj);
+        if (B->mem) (void)hipFree(B->mem);
         delete B;
         return r ? r : hip_fail(e, "twg_bvh_build upload", __FILE__, __LINE__);
     }
@@ -787,10 +752,7 @@ int twg_bvh_destroy(twg_bvh* B)
     if (!B) return TWG_OK;
     (void)hipSetDevice(B->device);
     (void)hipDeviceSynchronize();
-    if (B->node64) (void)hipFree(B->node64);
-    if (B->node32) (void)hipFree(B->node32);
-    if (B->adj) (void)hipFree(B->adj);
-    if (B->tri) (void)hipFree(B->tri);
+    if (B->mem) (void)hipFree(B->mem);
     delete B;
     return TWG_OK;
 }

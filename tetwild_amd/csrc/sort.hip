@@ -3,23 +3,13 @@
 // neighbouring threads (and, through the XCD-aware block order, each XCD's
 // L2) visit the same tree paths.  Results never depend on the order.
 #include <cmath>
+#include <utility>
 
 #include "twg_internal.hpp"
 #include "twg_math.hpp"
 
 namespace twg {
 namespace {
-
-__device__ __forceinline__ uint64_t spread3d(uint64_t v)
-{
-    v &= 0x1FFFFF;
-    v = (v | v << 32) & 0x1F00000000FFFFull;
-    v = (v | v << 16) & 0x1F0000FF0000FFull;
-    v = (v | v << 8) & 0x100F00F00F00F00Full;
-    v = (v | v << 4) & 0x10C30C30C30C30C3ull;
-    v = (v | v << 2) & 0x1249249249249249ull;
-    return v;
-}
 
 // the item's place: a point, or a triangle's centroid
 __device__ __forceinline__ void item_place(const double* __restrict__ p, int stride, double c[3])
@@ -108,11 +98,11 @@ __device__ __forceinline__ uint32_t morton_key(const double* __restrict__ p, int
     return (uint32_t)(key >> (63 - bits));
 }
 
-// keys (first pass) and the block's digit counts
-template <bool FIRST>
+// keys (first pass) and the block's digit counts; KV: a (key, item) pair
+template <class KV, bool FIRST>
 __global__ __launch_bounds__(kBlock) void digit_count(const double* __restrict__ items, int64_t n,
                                                       int stride, const double* __restrict__ box,
-                                                      int bits, int shift, uint2* __restrict__ kv,
+                                                      int bits, int shift, KV* __restrict__ kv,
                                                       unsigned* __restrict__ count)
 {
     __shared__ unsigned h[kDigits];
@@ -123,14 +113,15 @@ __global__ __launch_bounds__(kBlock) void digit_count(const double* __restrict__
     for (int r = 0; r < kSortItems; ++r) {
         const int64_t i = base + r * kBlock + threadIdx.x;
         if (i >= n) break;
-        uint32_t key;
+        KV v;
         if (FIRST) {
-            key = morton_key(items + (int64_t)stride * i, stride, box, bits);
-            kv[i] = make_uint2(key, (uint32_t)i);
+            v.x = morton_key(items + (int64_t)stride * i, stride, box, bits);
+            v.y = (uint32_t)i;
+            kv[i] = v;
         } else {
-            key = kv[i].x;
+            v.x = kv[i].x;
         }
-        atomicAdd(&h[(key >> shift) & (kDigits - 1)], 1u);
+        atomicAdd(&h[(unsigned)(v.x >> shift) & (kDigits - 1)], 1u);
     }
     __syncthreads();
     for (int d = threadIdx.x; d < kDigits; d += kBlock) count[(int64_t)d * gridDim.x + blockIdx.x] = h[d];
@@ -190,11 +181,11 @@ __global__ __launch_bounds__(kBlock) void digit_scan(unsigned* __restrict__ coun
 // round; the lanes of a round that share a digit find each other by ballots
 // over its bits, and the wave's LDS counters carry the rounds.  LAST: only the
 // item ids are written.
-template <bool LAST>
-__global__ __launch_bounds__(kBlock) void digit_place(const uint2* __restrict__ in, int64_t n, int shift,
+template <class KV, bool LAST>
+__global__ __launch_bounds__(kBlock) void digit_place(const KV* __restrict__ in, int64_t n, int shift,
                                                       const unsigned* __restrict__ count,
                                                       const unsigned* __restrict__ total,
-                                                      uint2* __restrict__ out, int32_t* __restrict__ order)
+                                                      KV* __restrict__ out, int32_t* __restrict__ order)
 {
     constexpr int W = kBlock / 64;
     __shared__ unsigned at[W][kDigits];
@@ -204,17 +195,18 @@ __global__ __launch_bounds__(kBlock) void digit_place(const uint2* __restrict__ 
     __syncthreads();
     const int64_t base = (int64_t)blockIdx.x * kSortTile + w * (64 * kSortItems);
     const unsigned long long below = (1ull << lane) - 1ull;
-    uint2 kv[kSortItems];
+    KV kv[kSortItems];
     unsigned rank[kSortItems];
 #pragma unroll
     for (int r = 0; r < kSortItems; ++r) {
         const int64_t i = base + r * 64 + lane;
-        kv[r] = i < n ? in[i] : make_uint2(0u, 0u);
+        kv[r].x = kv[r].y = 0;
+        if (i < n) kv[r] = in[i];
     }
 #pragma unroll
     for (int r = 0; r < kSortItems; ++r) {
         const bool ok = base + r * 64 + lane < n;
-        const unsigned d = (kv[r].x >> shift) & (kDigits - 1);
+        const unsigned d = (unsigned)(kv[r].x >> shift) & (kDigits - 1);
         unsigned long long same = __ballot(ok);
 #pragma unroll
         for (int b = 0; b < kDigitBits; ++b) {
@@ -247,13 +239,37 @@ __global__ __launch_bounds__(kBlock) void digit_place(const uint2* __restrict__ 
 #pragma unroll
     for (int r = 0; r < kSortItems; ++r) {
         if (base + r * 64 + lane >= n) continue;
-        const unsigned p = at[w][(kv[r].x >> shift) & (kDigits - 1)] + rank[r];
+        const unsigned p = at[w][(unsigned)(kv[r].x >> shift) & (kDigits - 1)] + rank[r];
         if (LAST) order[p] = (int32_t)kv[r].y;
         else out[p] = kv[r];
     }
 }
 
 }  // namespace
+
+size_t sort_pairs_bytes(int64_t n)
+{
+    return (size_t)((n + kSortTile - 1) / kSortTile) * kDigits * 4 + kDigits * 4;
+}
+
+int sort_pairs(ulonglong2* kv[2], int64_t n, int bits, void* work, hipStream_t s)
+{
+    unsigned* total = static_cast<unsigned*>(work);
+    unsigned* count = total + kDigits;
+    const unsigned nb = (unsigned)((n + kSortTile - 1) / kSortTile);
+    for (int shift = 0; shift < bits; shift += kDigitBits) {
+        hipLaunchKernelGGL((digit_count<ulonglong2, false>), dim3(nb), dim3(kBlock), 0, s, nullptr, n, 0, nullptr,
+                           0, shift, kv[0], count);
+        TWG_LAUNCHED();
+        hipLaunchKernelGGL(digit_scan, dim3(kDigits), dim3(kBlock), 0, s, count, (int)nb, total);
+        TWG_LAUNCHED();
+        hipLaunchKernelGGL((digit_place<ulonglong2, false>), dim3(nb), dim3(kBlock), 0, s, kv[0], n, shift, count,
+                           total, kv[1], nullptr);
+        TWG_LAUNCHED();
+        std::swap(kv[0], kv[1]);
+    }
+    return TWG_OK;
+}
 
 int morton_order(twg_ctx* ctx, const double* items, int64_t n, int stride, const double* lo,
                  const double* hi, const int32_t** order)
@@ -283,13 +299,13 @@ int morton_order(twg_ctx* ctx, const double* items, int64_t n, int stride, const
     for (int p = 0; p < passes; ++p) {
         uint2 *from = kv[p % 2], *to = kv[1 - p % 2];
         const int shift = p * kDigitBits;
-        if (p == 0) hipLaunchKernelGGL(digit_count<true>, g, b, 0, s, items, n, stride, box, bits, shift, from, count);
-        else hipLaunchKernelGGL(digit_count<false>, g, b, 0, s, items, n, stride, box, bits, shift, from, count);
+        if (p == 0) hipLaunchKernelGGL((digit_count<uint2, true>), g, b, 0, s, items, n, stride, box, bits, shift, from, count);
+        else hipLaunchKernelGGL((digit_count<uint2, false>), g, b, 0, s, items, n, stride, box, bits, shift, from, count);
         TWG_LAUNCHED();
         hipLaunchKernelGGL(digit_scan, dim3(kDigits), b, 0, s, count, (int)nb, total);
         TWG_LAUNCHED();
-        if (p + 1 < passes) hipLaunchKernelGGL(digit_place<false>, g, b, 0, s, from, n, shift, count, total, to, out);
-        else hipLaunchKernelGGL(digit_place<true>, g, b, 0, s, from, n, shift, count, total, to, out);
+        if (p + 1 < passes) hipLaunchKernelGGL((digit_place<uint2, false>), g, b, 0, s, from, n, shift, count, total, to, out);
+        else hipLaunchKernelGGL((digit_place<uint2, true>), g, b, 0, s, from, n, shift, count, total, to, out);
         TWG_LAUNCHED();
     }
     *order = out;

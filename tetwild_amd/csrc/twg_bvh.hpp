@@ -46,9 +46,8 @@ struct twg_bvh {
     BvhNode64* node64 = nullptr;
     BvhNode32* node32 = nullptr;
     double* tri = nullptr;  // nf x 9, tree order
-    // nf x 3, tree order: the facet across edge k (vertices k, k+1), -1 none
-    int32_t* adj = nullptr;
     std::vector<int32_t> order;  // tree position -> caller's facet id
+    void* mem = nullptr;         // the one allocation behind the three arrays
 };
 
 namespace twg {
@@ -91,9 +90,8 @@ struct BvhView {
     const double* __restrict__ tri;
     int64_t nf;
     int64_t nnode;  // node slots (array length)
-    const int32_t* __restrict__ adj;  // nf x 3 edge neighbours (tree positions)
 };
-static_assert(sizeof(BvhView) == 48, "BvhView: kernel-argument layout");
+static_assert(sizeof(BvhView) == 40, "BvhView: kernel-argument layout");
 
 // What the traversals read: the view plus an optional copy of the top of the
 // tree in LDS (node slots [0, ncache), the levels every traversal walks
@@ -106,7 +104,6 @@ struct BvhWalk {
     const double* __restrict__ tri;
     int64_t nf;
     int64_t nnode;
-    const int32_t* __restrict__ adj;
     LdsNode64* c64;
     LdsNode32* c32;
     int64_t ncache;
@@ -124,7 +121,6 @@ __device__ __forceinline__ BvhWalk walk(const BvhView& B)
     w.tri = B.tri;
     w.nf = B.nf;
     w.nnode = B.nnode;
-    w.adj = B.adj;
     w.c64 = nullptr;
     w.c32 = nullptr;
     w.ncache = 0;
@@ -395,7 +391,7 @@ __device__ __forceinline__ void put_lds(LdsNode32W* d, const BvhNode32& s)
         d->hi[k] = s.hi[k];
     }
     d->leaf = s.leaf;
-    d->pad = -1;  // no neighbours recorded (list_neighbours fills them)
+    d->pad = -1;  // no neighbours recorded
 }
 
 // The facets whose boxes meet the box [lo, hi], found by the G lanes of a
@@ -480,31 +476,6 @@ __device__ int collect_facets(const BvhWalk& W, const double lo[3], const double
 
 typedef __attribute__((address_space(3))) double LdsF64;
 typedef __attribute__((address_space(3))) const double LdsF64c;
-
-// For each entry of a collect_facets list (lanes gl, gl + G, ...), the list
-// positions of its facet's three edge neighbours (the tree's adjacency),
-// packed 8 bits each into the entry's pad field; 0xff where the neighbour is
-// not in the list or the tree has no adjacency.  Lists of up to 255 entries.
-// Every lane of the group calls it; it ends with the group's writes visible.
-template <int G>
-__device__ void list_neighbours(const BvhWalk& W, LdsNode32W* lst, int nl, int gl)
-{
-    if (W.adj && nl > 0 && nl < 256) {
-        for (int e = gl; e < nl; e += G) {
-            const int64_t f = lst[e].leaf;
-            const int a0 = W.adj[3 * f], a1 = W.adj[3 * f + 1], a2 = W.adj[3 * f + 2];
-            uint32_t q0 = 0xffu, q1 = 0xffu, q2 = 0xffu;
-            for (int i = 0; i < nl; ++i) {
-                const int li = lst[i].leaf;
-                q0 = li == a0 ? (uint32_t)i : q0;
-                q1 = li == a1 ? (uint32_t)i : q1;
-                q2 = li == a2 ? (uint32_t)i : q2;
-            }
-            lst[e].pad = (int32_t)(q0 | (q1 << 8) | (q2 << 16) | 0xff000000u);
-        }
-    }
-    wave_sync();
-}
 
 // facet_d2 of a triangle held in LDS (9 doubles): the same computation on
 // the same values
@@ -907,11 +878,11 @@ __device__ __forceinline__ int cert_class(P c, V3<float> q, const CertFrame& F)
 }
 
 // in_envelope_list / in_envelope_masked with the certificates: the facet at
-// hl first (NB: then its neighbours), then the positions set in mask, in
+// hl first, then the positions set in mask, in
 // ascending order; positions no certificate decides go to FP64 at the end.
 // The decision is in_envelope_masked's; hl may become another facet that
 // holds p.  sure: set when the facet left in hl is certified.
-template <bool NB, class L, class P, class M>
+template <class L, class P, class M>
 __device__ __forceinline__ bool in_envelope_cert(const BvhWalk& W, L lst, P cert, int nl, M mask,
                                                  V3<double> p, const CertFrame& F, double eps2,
                                                  int& hl, bool& sure)
@@ -929,21 +900,6 @@ __device__ __forceinline__ bool in_envelope_cert(const BvhWalk& W, L lst, P cert
         if (r > 0) return true;
         mark(done, hl);
         if (r == 0) mark(open, hl);
-        const uint32_t pk = NB ? (uint32_t)lst[hl].pad : 0xffffffffu;
-        if (NB)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const uint32_t u = (pk >> (8 * k)) & 0xffu;
-                if (u != 0xffu) {
-                    const int ru = cert_class(cert + kCertFloats * u, q, F);
-                    if (ru > 0) {
-                        hl = (int)u;
-                        return true;
-                    }
-                    mark(done, (int)u);
-                    if (ru == 0) mark(open, (int)u);
-                }
-            }
     }
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
@@ -1237,7 +1193,7 @@ __device__ bool face_out_listed(const BvhWalk& B, const double* t9, double eps2,
 // which lane tests which sample, so it equals face_out_sampled's.  For batches
 // of few triangles with many samples each, where one lane per triangle leaves
 // most of the machine idle.
-template <bool F32, int G, bool SUBTREE = true, bool NB = false>
+template <bool F32, int G, bool SUBTREE = true>
 __device__ bool face_out_group(const BvhWalk& B, V3<double> a, V3<double> b, V3<double> c,
                                double eps2, double d, double T, double sqrtT, int r, int gbase,
                                LdsNode32W* lst, LdsF32* cert, const CertFrame& F, int nl)
@@ -1279,7 +1235,7 @@ __device__ bool face_out_group(const BvhWalk& B, V3<double> a, V3<double> b, V3<
         const bool have = j < mine && g.next(q);
         bool out = false, sure = false;
         if (have) {
-            if (nl >= 0) out = !in_envelope_cert<NB>(B, lst, cert, nl, mask, q, F, eps2, hl, sure);
+            if (nl >= 0) out = !in_envelope_cert(B, lst, cert, nl, mask, q, F, eps2, hl, sure);
             else out = !in_envelope<F32, false, SUBTREE>(B, q, eps2, T, sqrtT, hint, st);
         }
         ++j;
@@ -1312,13 +1268,12 @@ inline BvhView bvh_view(const twg_bvh* b)
     v.tri = b->tri;
     v.nf = b->nf;
     v.nnode = b->nnode;
-    v.adj = b->adj;
     return v;
 }
 
 inline BvhView no_bvh()
 {
-    BvhView v = {nullptr, nullptr, nullptr, 0, 0, nullptr};
+    BvhView v = {nullptr, nullptr, nullptr, 0, 0};
     return v;
 }
 

@@ -25,7 +25,7 @@ struct twg_ctx {
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
     // further growable slots: 0 the queue of tets the orientation filter left
-    // undecided, 1 query ordering keys and values, 2 sort temporary storage
+    // undecided, 1 query ordering keys and values, 2 its digit counts
     void* slot[4] = {nullptr, nullptr, nullptr, nullptr};
     size_t slot_bytes[4] = {0, 0, 0, 0};
     // device address of smooth.hip's file-scope scratch array on this
@@ -53,6 +53,11 @@ int ensure_slot(twg_ctx* ctx, int i, size_t bytes);
 // order only affects speed: every query's result is independent of it.
 int morton_order(twg_ctx* ctx, const double* items, int64_t n, int stride, const double* lo,
                  const double* hi, const int32_t** order);
+
+// Stable sort of n (key, value) pairs by the low `bits` bits of their keys:
+// kv[0] in and, after the call, out; kv[1] as large; work: sort_pairs_bytes(n).
+size_t sort_pairs_bytes(int64_t n);
+int sort_pairs(ulonglong2* kv[2], int64_t n, int bits, void* work, hipStream_t s);
 
 // Activates ctx->device for the calling thread.
 int bind(twg_ctx* ctx);

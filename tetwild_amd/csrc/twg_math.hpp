@@ -430,6 +430,18 @@ TWG_HD bool certainly_not_collinear(const double* p, const double* q, const doub
     return false;
 }
 
+// the low 21 bits of v, three apart (a coordinate's share of a Morton code)
+__device__ __forceinline__ uint64_t spread3d(uint64_t v)
+{
+    v &= 0x1FFFFF;
+    v = (v | v << 32) & 0x1F00000000FFFFull;
+    v = (v | v << 16) & 0x1F0000FF0000FFull;
+    v = (v | v << 8) & 0x100F00F00F00F00Full;
+    v = (v | v << 4) & 0x10C30C30C30C30C3ull;
+    v = (v | v << 2) & 0x1249249249249249ull;
+    return v;
+}
+
 // XCD-aware block order: blocks are dispatched round-robin over the 8 XCDs of
 // an MI355X, so block b runs on XCD b % 8.  Remapping b -> (b % 8) * (G / 8) +
 // b / 8 gives every XCD a contiguous range of the work, so neighbouring items
