@@ -67,3 +67,47 @@ def test_lists_overflow_and_limits(eps, edge):
         o = ctx.envelope_faces(s, small, eps * eps, d)
         assert torch.equal(o, ctx.envelope_faces(s, small, eps * eps, d, stats=True)[0])
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 32767, 32768, 65535])
+@pytest.mark.parametrize("reach", ["near", "far", "wide"])
+def test_small_points_and_nearest(n, reach):
+    """Lanes-per-point kernels: the decision and the nearest facet of every
+    point, where groups decide, where their lists overflow (an envelope wider
+    than the list holds) and where they cannot be sure (far points, ties on a
+    flat grid), NaN and infinite points among them, against the oracle"""
+    import torch
+
+    from oracle import oracle as O
+    from tetwild_amd import workloads as W
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    V, F = W.bumpy_sphere(freq=12, seed=3)
+    if reach == "far":  # a flat grid: ties above its edges and corners
+        g = np.arange(20.0)
+        V = np.stack(np.meshgrid(g, g, [0.0], indexing="ij"), -1).reshape(-1, 3)
+        q = (np.arange(19)[:, None] * 20 + np.arange(19)).reshape(-1)
+        F = np.concatenate([np.stack([q, q + 20, q + 1], 1), np.stack([q + 1, q + 20, q + 21], 1)]).astype(np.int32)
+    r = np.random.default_rng(n)
+    k = min(n, 3000)  # distinct points, repeated over the batch
+    P = V[r.integers(0, len(V), k)] + r.normal(size=(k, 3)) * (0.02 if reach != "far" else 0.0)
+    if reach == "far":
+        P[:, 2] += r.uniform(0, 5, k) * (np.arange(k) % 3)
+    eps = 0.4 if reach == "wide" else 0.02
+    surf = ctx.surface(V, F)
+    S = O.Surface(V, F[surf.order()])
+    cp, d2, fid = S.nearest(P)
+    at = np.arange(n) % k
+    Q = np.ascontiguousarray(P[at])
+    tq = torch.from_numpy(Q).to("cuda:0")
+    for prec in (0, 1):
+        out = ctx.envelope_points(surf, tq, eps * eps, precision=prec).cpu().numpy()
+        assert np.array_equal(out, S.point_out(P, eps * eps)[at]), prec
+    gcp, gd2, gf = (t.cpu().numpy() for t in ctx.nearest(surf, tq))
+    assert np.array_equal(gcp, cp[at]) and np.array_equal(gd2, d2[at]) and np.array_equal(gf, fid[at])
+    if n > 16:
+        Q[3], Q[7, 1] = np.nan, np.inf
+        tq = torch.from_numpy(Q).to("cuda:0")
+        out = ctx.envelope_points(surf, tq, eps * eps)
+        assert torch.equal(out, ctx.envelope_points(surf, tq, eps * eps, stats=True)[0])
+    ctx.close()

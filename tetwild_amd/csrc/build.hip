@@ -72,7 +72,21 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long v)
     return v;
 }
 
-// the centroids' box, and the first id out of range
+// the block's largest v (every thread calls it), in thread 0
+__device__ __forceinline__ unsigned long long block_max(unsigned long long v)
+{
+    __shared__ unsigned long long w[kBlock / 64];
+    v = wave_max(v);
+    if (threadIdx.x % 64 == 0) w[threadIdx.x / 64] = v;
+    __syncthreads();
+    for (int k = 1; k < kBlock / 64; ++k) v = threadIdx.x == 0 && w[k] > v ? w[k] : v;
+    __syncthreads();
+    return v;
+}
+
+// the centroids' box, and the first id out of range: few blocks, an atomic of
+// each on the scalars (an atomic per wave of a full grid took 260 us)
+constexpr unsigned kCheckBlocks = 256;
 __global__ __launch_bounds__(kBlock) void build_check(BuildArgs A)
 {
     unsigned long long lo[3], hi[3], bad = ~0ull;
@@ -92,12 +106,12 @@ __global__ __launch_bounds__(kBlock) void build_check(BuildArgs A)
             hi[c] = o > hi[c] ? o : hi[c];
         }
     }
-    bad = ~wave_max(~bad);
+    bad = ~block_max(~bad);
     for (int c = 0; c < 3; ++c) {
-        lo[c] = wave_max(lo[c]);
-        hi[c] = wave_max(hi[c]);
+        lo[c] = block_max(lo[c]);
+        hi[c] = block_max(hi[c]);
     }
-    if (threadIdx.x % 64) return;
+    if (threadIdx.x) return;
     if (bad != ~0ull) atomicMin(&A.sc->bad, bad);
     for (int c = 0; c < 3; ++c) {
         atomicMin(&A.sc->lo[c], ~lo[c]);
@@ -145,8 +159,8 @@ __global__ __launch_bounds__(kBlock) void build_facets(BuildArgs A, const ulongl
             r = r < l ? l : r;
         }
     }
-    const unsigned long long m = wave_max(f2u(r));  // not negative: its bits order it
-    if (threadIdx.x % 64 == 0 && m) atomicMax(&A.sc->rmax, m);
+    const unsigned long long m = block_max(f2u(r));  // not negative: its bits order it
+    if (threadIdx.x == 0 && m) atomicMax(&A.sc->rmax, m);
 }
 
 // Node n at depth d of the tree over nf facets: from its children, its facet
@@ -287,7 +301,7 @@ int bvh_build_device(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F
     const dim3 b(kBlock), gf(grid_for(nf));
     hipLaunchKernelGGL(build_init, dim3(1), dim3(1), 0, s, A);
     TWG_LAUNCHED();
-    hipLaunchKernelGGL(build_check, dim3(std::min<unsigned>(grid_for(nf), 1024u)), b, 0, s, A);
+    hipLaunchKernelGGL(build_check, dim3(std::min<unsigned>(grid_for(nf), kCheckBlocks)), b, 0, s, A);
     TWG_LAUNCHED();
     hipLaunchKernelGGL(build_keys, gf, b, 0, s, A, kv[0]);
     TWG_LAUNCHED();

@@ -69,6 +69,48 @@ __device__ __forceinline__ int64_t xcd_run_block()
 // this many lanes.
 constexpr int kListSplit = 8;
 
+// points_kernel for small batches: sixteen lanes per point, which list the
+// facets within reach (collect_facets) and test one each -- a chain of a few
+// reads instead of a walk's, with lanes to spare, in the caller's order.  On
+// 246 k facets 4,096 points 143 -> 17 us, 65 k 169 -> 53, 400 k 282 -> 240, but
+// 1 M 451 -> 563 (there the sort pays, and from two points a facet on the wave
+// lists).  Dense batches of 65 k points and more keep the wave lists too.
+// (Eight and thirty-two lanes: 58 and 61 us for 65 k.)
+constexpr int kPointGroup = 16;
+constexpr int kPointGroupCap = 32;
+constexpr int64_t kPointGroupMax = 1 << 19;
+constexpr int64_t kPointGroupDensity = 8;
+template <bool F32>
+__global__ __launch_bounds__(kBlock) void points_group_kernel(BvhView B, const double* __restrict__ p3,
+                                                              int64_t n, double eps2, double T,
+                                                              double sqrtT, uint8_t* __restrict__ out)
+{
+    constexpr int G = kPointGroup;
+    __shared__ __align__(16) unsigned char lists[(kBlock / G) * kPointGroupCap * 40];
+    const BvhWalk W = walk(B);
+    const int gl = threadIdx.x % G, gbase = (threadIdx.x % 64) - gl;
+    const int64_t i = (int64_t)blockIdx.x * (kBlock / G) + threadIdx.x / G;
+    if (i >= n) return;
+    unsigned char* mine = lists + (threadIdx.x / G) * (kPointGroupCap * 40);
+    LdsNode32W* lst = (LdsNode32W*)mine;
+    const V3<double> p = ld3(p3 + 3 * i);
+    const double pad = 1.0001 * sqrtT + 1e-9 * fmax(fabs(p.x), fmax(fabs(p.y), fabs(p.z)));
+    const double lo[3] = {p.x - pad, p.y - pad, p.z - pad}, hi[3] = {p.x + pad, p.y + pad, p.z + pad};
+    const int nl = collect_facets<G>(W, lo, hi, lst, (LdsU32*)(mine + kPointGroupCap * 32), kPointGroupCap,
+                                     gl, gbase);
+    bool in = false;
+    if (nl >= 0) {
+        for (int e = gl; e < nl && !in; e += G) in = facet_d2(W, lst[e].leaf, p) <= eps2;
+        const unsigned long long gm = (G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull) << gbase;
+        in = (__ballot(in) & gm) != 0ull;
+    } else {
+        int hint = -1;
+        Stats st;
+        in = in_envelope<F32, false>(W, p, eps2, T, sqrtT, hint, st);
+    }
+    if (gl == 0) out[i] = in ? 0 : 1;
+}
+
 // points_kernel for batches walked in Morton order with many points per
 // facet: the wave's 64 consecutive points lie close together, so the wave
 // lists once (collect_facets, LDS) the facets whose boxes meet the box of its
@@ -496,23 +538,69 @@ constexpr int64_t kFaceListDensity = 2;
 constexpr int kPointListCap = 64;
 constexpr int64_t kPointListDensity = 2;
 
+// Nearest facets.  nearest_facet's walk is a chain of some 500 dependent
+// reads (2.9 ms for any batch up to 65 k points near 246 k facets, 11 ms a
+// third of a radius away from them), so kNearestGroup lanes take a point
+// (nearest_facet_try: lists of the facets around it).  Where they cannot be
+// sure of the walk's result -- far queries, ties -- the walk runs: in the group
+// itself for small batches, which have the lanes (4,096 far points 11 -> 2.2
+// ms, 65 k 10.5 -> 14.7), else by nearest_rest_kernel, a point per lane.
+// 4,096 points 2951 -> 37 us, 1 M 10.5 -> 3.7 ms.  (8, 16 and 64 lanes a
+// point: 65, 45 and 35 us for 4,096, 6.6, 4.7 and 5.7 ms for 1 M.)
+constexpr int kNearestGroup = 32;
+constexpr int kNearestCap = 64;  // facets listed per group
+constexpr int64_t kNearestWalkMax = 1 << 15;
+template <bool WALK>
 __global__ __launch_bounds__(kBlock) void nearest_kernel(BvhView B, const double* __restrict__ p3,
                                                          int64_t n, double* __restrict__ cp3,
                                                          double* __restrict__ d2out,
-                                                         int32_t* __restrict__ fout)
+                                                         int32_t* __restrict__ fout,
+                                                         const int32_t* __restrict__ order, int64_t base)
 {
+    constexpr int G = kNearestGroup;
     __shared__ __align__(16) unsigned char cache[kPointCacheBytes];
+    __shared__ __align__(16) unsigned char lists[(kBlock / G) * kNearestCap * 40];
     const BvhWalk W = cache_tree_top<false, kPointCacheBytes>(B, cache);
-    const int64_t i = xcd_block() * kBlock + threadIdx.x;
+    const int gl = threadIdx.x % G, gbase = (threadIdx.x % 64) - gl;
+    int64_t i = base + xcd_block() * (int64_t)(kBlock / G) + threadIdx.x / G;
     if (i >= n) return;
+    if (order) i = order[i];
+    unsigned char* mine = lists + (threadIdx.x / G) * (kNearestCap * 40);
+    LdsNode32W* lst = (LdsNode32W*)mine;
+    LdsU32* fr = (LdsU32*)(mine + kNearestCap * 32);
     V3<double> np;
     double sq;
-    int best = nearest_facet(W, ld3(p3 + 3 * i), np, sq);
+    const int f = WALK ? nearest_facet_group<G>(W, ld3(p3 + 3 * i), np, sq, lst, fr, kNearestCap, gl, gbase)
+                       : nearest_facet_try<G>(W, ld3(p3 + 3 * i), np, sq, lst, fr, kNearestCap, gl, gbase);
+    if (gl != 0) return;
+    fout[i] = f;
+    if (!WALK && f < 0) return;
     cp3[3 * i + 0] = np.x;
     cp3[3 * i + 1] = np.y;
     cp3[3 * i + 2] = np.z;
     d2out[i] = sq;
-    fout[i] = best;
+}
+
+// the points nearest_kernel<false> left (facet -1), one per lane
+__global__ __launch_bounds__(kBlock) void nearest_rest_kernel(BvhView B, const double* __restrict__ p3,
+                                                              int64_t n, double* __restrict__ cp3,
+                                                              double* __restrict__ d2out,
+                                                              int32_t* __restrict__ fout,
+                                                              const int32_t* __restrict__ order)
+{
+    int64_t i = xcd_block() * kBlock + threadIdx.x;
+    if (i < n && order) i = order[i];
+    __shared__ __align__(16) unsigned char cache[kPointCacheBytes];
+    if (!__syncthreads_or(i < n && fout[i] < 0)) return;
+    const BvhWalk W = cache_tree_top<false, kPointCacheBytes>(B, cache);
+    if (i >= n || fout[i] >= 0) return;
+    V3<double> np;
+    double sq;
+    fout[i] = nearest_facet(W, ld3(p3 + 3 * i), np, sq);
+    cp3[3 * i + 0] = np.x;
+    cp3[3 * i + 1] = np.y;
+    cp3[3 * i + 2] = np.z;
+    d2out[i] = sq;
 }
 
 __global__ __launch_bounds__(kBlock) void sample_count_kernel(const double* __restrict__ tri9,
@@ -797,10 +885,15 @@ int twg_envelope_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_
     double T = bvh_prune_threshold(B, eps2), sT = std::sqrt(T);
     dim3 g(grid_for(n)), b(kBlock);
     BvhView v = bvh_view(B);
+    const bool group = !stats && (n < kSortMin || (n < kPointGroupMax && n < kPointGroupDensity * B->nf));
     const int32_t* order = nullptr;
-    if (n >= kSortMin)
+    if (n >= kSortMin && !group)
         if (int r = morton_order(ctx, p3, n, 3, B->lo, B->hi, &order)) return r;
-    if (order && !stats && n >= kPointListDensity * B->nf) {
+    if (group) {
+        const dim3 gg(grid_for(n * kPointGroup));
+        if (precision == TWG_FP64) hipLaunchKernelGGL(points_group_kernel<false>, gg, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out);
+        else hipLaunchKernelGGL(points_group_kernel<true>, gg, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out);
+    } else if (order && !stats && n >= kPointListDensity * B->nf) {
         if (precision == TWG_FP64)
             hipLaunchKernelGGL((points_list_kernel<false, kPointListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, p3, n, eps2, T, sT, out, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
         else
@@ -893,8 +986,25 @@ int twg_nearest_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_t
     TWG_REQUIRE(n == 0 || (d2 && facet), "twg_nearest_points: NULL output");
     if (n == 0) return TWG_OK;
     if (int r = bind(ctx)) return r;
-    hipLaunchKernelGGL(nearest_kernel, dim3(grid_for(n)), dim3(kBlock), 0, ctx->cur, bvh_view(B), p3,
-                       n, cp3, d2, facet);
+    const dim3 b(kBlock);
+    BvhView v = bvh_view(B);
+    const int32_t* order = nullptr;
+    if (n >= kSortMin && n < (int64_t(1) << 31))
+        if (int r = morton_order(ctx, p3, n, 3, B->lo, B->hi, &order)) return r;
+    constexpr int64_t kPart = 1 << 26;  // a launch holds fewer than 2^32 threads
+    for (int64_t at = 0; at < n; at += kPart) {
+        const dim3 g(grid_for(std::min(n - at, kPart) * kNearestGroup));
+        if (n < kNearestWalkMax)
+            hipLaunchKernelGGL(nearest_kernel<true>, g, b, 0, ctx->cur, v, p3, n, cp3, d2, facet, order, at);
+        else
+            hipLaunchKernelGGL(nearest_kernel<false>, g, b, 0, ctx->cur, v, p3, n, cp3, d2, facet, order, at);
+        TWG_LAUNCHED();
+    }
+    if (n < kNearestWalkMax) return TWG_OK;
+    // (walks far from the surface gain nothing from the order below some 250 k
+    // points: 65 k 10.5 ms without and 12.1 with it, 1 M 41 and 30)
+    hipLaunchKernelGGL(nearest_rest_kernel, dim3(grid_for(n)), b, 0, ctx->cur, v, p3, n, cp3, d2, facet,
+                       n < (1 << 18) ? nullptr : order);
     TWG_LAUNCHED();
     return TWG_OK;
 }

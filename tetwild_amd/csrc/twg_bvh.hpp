@@ -1019,7 +1019,7 @@ __device__ __forceinline__ int nearest_facet(const BvhWalk& B, V3<double> p, V3<
 
 // nearest_facet's result (facet, np, sq -- bit for bit) computed by the G
 // lanes of a group (lane gl, first lane gbase in the wave; G a power of two up
-// to 64), or by nearest_facet itself where the group cannot be sure to agree.
+// to 64), or -1 where the group cannot be sure to agree.
 // The walk starts from the hint facet h with sq = s0 = |v0(h) - p|^2 and
 // takes a facet only when its distance is strictly below the best so far.
 // The group lists the facets whose boxes meet a cube around p (collect_facets)
@@ -1033,13 +1033,12 @@ __device__ __forceinline__ int nearest_facet(const BvhWalk& B, V3<double> p, V3<
 // walk cannot prune that path (it prunes a box only at or above the best so
 // far, never below D) and nothing it visits later replaces f, so it returns
 // f -- taken here.  Otherwise (ties, a box at or above D, a list too long for
-// cap, a query that is not finite, three cubes without a facet) nearest_facet
-// walks.  Every lane of the group calls it with the same p.
+// cap, a query that is not finite, three cubes without a facet): -1.  Every lane of the group calls it with the same p.
 template <int G>
-__device__ int nearest_facet_group(const BvhWalk& B, V3<double> p, V3<double>& np, double& sq,
+__device__ int nearest_facet_try(const BvhWalk& B, V3<double> p, V3<double>& np, double& sq,
                                    LdsNode32W* lst, LdsU32* fr, int cap, int gl, int gbase)
 {
-    if (B.nf < 2) return nearest_facet(B, p, np, sq);
+    if (B.nf < 2) return -1;
     int64_t na = 1;
     while (node64(B, na).leaf < 0) {
         const BvhNode64 L = node64(B, 2 * na), R = node64(B, 2 * na + 1);
@@ -1049,7 +1048,7 @@ __device__ int nearest_facet_group(const BvhWalk& B, V3<double> p, V3<double>& n
     const int h = HL.leaf;
     const V3<double> v0 = ld3(B.tri + 9 * (int64_t)h);
     const double s0 = len2(v0 - p), sr0 = __builtin_sqrt(s0);
-    if (!(s0 <= 1.0e300)) return nearest_facet(B, p, np, sq);
+    if (!(s0 <= 1.0e300)) return -1;
     // more than the rounding of a facet distance: ~1e-7 (|p| + d + 2 edge) in
     // distance units (the root box's diagonal bounds every edge)
     const BvhNode64 root = node64(B, 1);
@@ -1121,7 +1120,16 @@ __device__ int nearest_facet_group(const BvhWalk& B, V3<double> p, V3<double>& n
         sq = m;
         return wf;
     }
-    return nearest_facet(B, p, np, sq);
+    return -1;
+}
+
+// nearest_facet by the group's lanes, walking itself where they are not sure
+template <int G>
+__device__ int nearest_facet_group(const BvhWalk& B, V3<double> p, V3<double>& np, double& sq,
+                                   LdsNode32W* lst, LdsU32* fr, int cap, int gl, int gbase)
+{
+    const int f = nearest_facet_try<G>(B, p, np, sq, lst, fr, cap, gl, gbase);
+    return f >= 0 ? f : nearest_facet(B, p, np, sq);
 }
 
 // Triangles whose longest edge exceeds kMaxEdgeSamples sampling distances are
