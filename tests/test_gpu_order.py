@@ -111,3 +111,38 @@ def test_small_points_and_nearest(n, reach):
         out = ctx.envelope_points(surf, tq, eps * eps)
         assert torch.equal(out, ctx.envelope_points(surf, tq, eps * eps, stats=True)[0])
     ctx.close()
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 95, 96, 97, 140])
+def test_rows_per_wave(rows):
+    """Triangles of about `rows` sample rows, a wave each: the row table's one
+    and two rounds, its last rows and the sampler beyond it; needles and short
+    triangles among them, against the oracle"""
+    import torch
+
+    from oracle import oracle as O
+    from tetwild_amd import workloads as W
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    V, F = W.bumpy_sphere(freq=6, seed=3)
+    V = V * 4.0
+    d, eps = 0.01, 0.012
+    surf = ctx.surface(V, F)
+    S = O.Surface(V, F[surf.order()])
+    Q = W.query_triangles(V, F, 40, eps=eps, edge=(rows + 0.5) * d * 0.75 ** 0.5 / 0.75, seed=rows)
+    Q = Q.reshape(-1, 3, 3)
+    # in the plane of a facet, within the envelope: every sample is tested
+    T = V[F[:10]]
+    c = T.mean(1, keepdims=True)
+    size = np.linalg.norm(T - c, axis=2).min(1)
+    flat = c + (T - c) * (rows * d / (1.5 * size))[:, None, None]
+    needle = flat.copy()
+    needle[:, 2] = needle[:, 0] + 0.5 * (needle[:, 1] - needle[:, 0]) + 0.01 * (needle[:, 2] - needle[:, 0])
+    short = c + (T - c) * (0.4 * d / size)[:, None, None]
+    Q = np.ascontiguousarray(np.concatenate([Q, flat, needle, short]).reshape(-1, 9))
+    ref, _ = S.face_out(Q, eps * eps, d)
+    assert 0 < ref.sum() < len(ref)
+    for prec in (0, 1):
+        out = ctx.envelope_faces(surf, torch.from_numpy(Q).to("cuda:0"), eps * eps, d, precision=prec)
+        assert np.array_equal(out.cpu().numpy(), ref), prec
+    ctx.close()

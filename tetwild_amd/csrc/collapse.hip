@@ -382,8 +382,8 @@ template <bool F32>
 __global__ __launch_bounds__(kBlock) void collapse_face_kernel(CollapseArgs A)
 {
     __shared__ __align__(16) unsigned char face_lists[(kBlock / 64) * kFaceListBytes];
+    __shared__ double seg[(kBlock / 64) * kWaveSegBytes / 8];
     const int r = threadIdx.x % kFaceGroup;
-    const int gbase = (threadIdx.x % 64) - r;
     const int64_t k = (xcd_block() * (int64_t)kBlock + threadIdx.x) / kFaceGroup;
     if (k >= A.n_tri) return;
     const int64_t c = A.tri_cand[k];
@@ -430,8 +430,8 @@ __global__ __launch_bounds__(kBlock) void collapse_face_kernel(CollapseArgs A)
     const int nl = fin ? collect_facets<64>(W, lo, hi, lst, fr, kFaceListCap, r, 0) : -1;
     const CertFrame F = cert_frame(lo, hi, amax, A.eps2, A.d);
     cert_list<64>(W, lst, cert, nl, F, A.eps2, r);
-    if (face_out_group<F32, kFaceGroup, false>(W, ld3(t9), ld3(t9 + 3), ld3(t9 + 6), A.eps2, A.d,
-                                               A.T_sf, A.sqrtT_sf, r, gbase, lst, cert, F, nl) &&
+    if (face_out_wave<F32, false>(W, ld3(t9), ld3(t9 + 3), ld3(t9 + 6), A.eps2, A.d, A.T_sf, A.sqrtT_sf, r,
+                                  lst, cert, F, nl, (LdsF64*)seg + (threadIdx.x / 64) * (kWaveSegBytes / 8)) &&
         r == 0)
         atomicOr(A.work + c, kFaceOut);
 }

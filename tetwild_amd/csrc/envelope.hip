@@ -430,30 +430,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
     if (lstat && lane == 0) atomicAdd(lstat + (walked ? 1 : 0), 1ull);
 }
 
-// facets listed per wave in faces_group_kernel<F32, 64>
-constexpr int kGroupListCap = 64;
-constexpr int kGroupListBytes = kGroupListCap * kCertEntryBytes;
-
-// A group of G lanes per triangle, its samples spread over the lanes
-// (face_out_group).  Small batches run G = 64 (a wave per triangle), so that
-// few triangles with many samples each still fill the machine.  Same outputs
-// and pending queue as faces_kernel.
-template <bool F32, int G>
-__global__ __launch_bounds__(kBlock) void faces_group_kernel(BvhView B, const double* __restrict__ tri9,
-                                                             int64_t n, double eps2, double d,
-                                                             double T, double sqrtT,
-                                                             uint8_t* __restrict__ out,
-                                                             unsigned* n_pending, int64_t* pending,
-                                                             const int32_t* __restrict__ order)
+// A wave per triangle, its samples spread over the lanes (face_out_wave): for
+// small batches, so that few triangles with many samples each still fill the
+// machine.  Same outputs and pending queue as faces_kernel.  The tree is read
+// from global memory throughout (listing through an LDS copy of its top ran
+// ~5 % slower here, and only lists that do not fit walk it).
+constexpr int kWaveListCap = 64;
+constexpr int kWaveListBytes = kWaveListCap * kCertEntryBytes;
+template <bool F32>
+__global__ __launch_bounds__(kBlock) void faces_wave_kernel(BvhView B, const double* __restrict__ tri9,
+                                                            int64_t n, double eps2, double d,
+                                                            double T, double sqrtT,
+                                                            uint8_t* __restrict__ out,
+                                                            unsigned* n_pending, int64_t* pending)
 {
-    __shared__ __align__(16) unsigned char cache[kTreeCacheBytes];
-    __shared__ __align__(16) unsigned char face_lists[G == 64 ? (kBlock / 64) * kGroupListBytes : 16];
-    const BvhWalk W = cache_tree_top<F32>(B, cache);
-    const int r = threadIdx.x % G;
-    const int gbase = (threadIdx.x % 64) - r;
-    int64_t i = (xcd_block() * (int64_t)kBlock + threadIdx.x) / G;
+    __shared__ __align__(16) unsigned char face_lists[(kBlock / 64) * kWaveListBytes];
+    __shared__ double seg[(kBlock / 64) * kWaveSegBytes / 8];
+    const BvhWalk W = walk(B);
+    const int r = threadIdx.x % 64;
+    const int64_t i = (xcd_block() * (int64_t)kBlock + threadIdx.x) / 64;
     if (i >= n) return;
-    if (order) i = order[i];
     const double* t = tri9 + 9 * i;
     if (!certainly_not_collinear(t, t + 3, t + 6)) {
         if (r == 0) {
@@ -462,40 +458,35 @@ __global__ __launch_bounds__(kBlock) void faces_group_kernel(BvhView B, const do
         }
         return;
     }
-    int nl = -1;
-    LdsNode32W* lst = nullptr;
-    LdsF32* cert = nullptr;
+    // the facets near the triangle, listed in the wave's LDS (the tree walk
+    // when they do not fit or a coordinate is not finite)
+    unsigned char* mine = face_lists + (threadIdx.x / 64) * kWaveListBytes;
+    LdsNode32W* lst = (LdsNode32W*)mine;
+    LdsU32* fr = (LdsU32*)(mine + kWaveListCap * 32);  // the work lists, then the certificates
+    LdsF32* cert = (LdsF32*)(mine + kWaveListCap * 32);
+    double lo[3], hi[3], amax = 0.0;
+    bool fin = true;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        lo[j] = fmin(t[j], fmin(t[3 + j], t[6 + j]));
+        hi[j] = fmax(t[j], fmax(t[3 + j], t[6 + j]));
+        fin = fin && is_finite(t[j]) && is_finite(t[3 + j]) && is_finite(t[6 + j]);
+        amax = fmax(amax, fmax(fabs(lo[j]), fabs(hi[j])));
+    }
+    const double pad = 1.0001 * sqrtT + 1e-9 * amax;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        lo[j] -= pad;
+        hi[j] += pad;
+    }
+    const int nl = fin ? collect_facets<64>(W, lo, hi, lst, fr, kWaveListCap, r, 0) : -1;
     CertFrame F = {};
-    if (G == 64) {
-        // the facets near the triangle, listed in the wave's LDS (the tree
-        // walk when they do not fit or a coordinate is not finite)
-        unsigned char* mine = face_lists + (threadIdx.x / 64) * kGroupListBytes;
-        lst = (LdsNode32W*)mine;
-        LdsU32* fr = (LdsU32*)(mine + kGroupListCap * 32);  // the work lists, then the certificates
-        cert = (LdsF32*)(mine + kGroupListCap * 32);
-        double lo[3], hi[3], amax = 0.0;
-        bool fin = true;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            lo[j] = fmin(t[j], fmin(t[3 + j], t[6 + j]));
-            hi[j] = fmax(t[j], fmax(t[3 + j], t[6 + j]));
-            fin = fin && is_finite(t[j]) && is_finite(t[3 + j]) && is_finite(t[6 + j]);
-            amax = fmax(amax, fmax(fabs(lo[j]), fabs(hi[j])));
-        }
-        const double pad = 1.0001 * sqrtT + 1e-9 * amax;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            lo[j] -= pad;
-            hi[j] += pad;
-        }
-        // (listed from the global tree: measured ~5 % faster than through the
-        // LDS copy of its top here)
-        nl = fin ? collect_facets<64>(walk(B), lo, hi, lst, fr, kGroupListCap, r, 0) : -1;
+    if (nl >= 0) {
         F = cert_frame(lo, hi, amax, eps2, d);
         cert_list<64>(W, lst, cert, nl, F, eps2, r);
     }
-    const bool o = face_out_group<F32, G>(W, ld3(t), ld3(t + 3), ld3(t + 6), eps2, d, T, sqrtT, r,
-                                                      gbase, lst, cert, F, nl);
+    const bool o = face_out_wave<F32>(W, ld3(t), ld3(t + 3), ld3(t + 6), eps2, d, T, sqrtT, r, lst, cert, F, nl,
+                                      (LdsF64*)seg + (threadIdx.x / 64) * (kWaveSegBytes / 8));
     if (r == 0) out[i] = o ? 1 : 0;
 }
 
@@ -524,7 +515,7 @@ __global__ void zero_u64x2(unsigned long long* p)
 
 // batches at least this large are walked in Morton order of their queries
 constexpr int64_t kSortMin = 1 << 16;
-// face batches below this size run a wave per triangle (faces_group_kernel)
+// face batches below this size run a wave per triangle (faces_wave_kernel)
 constexpr int64_t kWaveMax = 1 << 16;
 // Facets per wave list in faces_list_kernel, and the queries per facet from
 // which a wave's 64 triangles (about 64 / density facets apart) fit it whole or
@@ -932,9 +923,9 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
     if (n < kWaveMax && !stats) {
         dim3 gw(grid_for(n * 64));
         if (precision == TWG_FP64)
-            hipLaunchKernelGGL((faces_group_kernel<false, 64>), gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order);
+            hipLaunchKernelGGL(faces_wave_kernel<false>, gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending);
         else
-            hipLaunchKernelGGL((faces_group_kernel<true, 64>), gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order);
+            hipLaunchKernelGGL(faces_wave_kernel<true>, gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending);
     } else if (order && !stats && n >= kFaceListDensity * B->nf) {
         // (the list's boxes, and the few tree walks', are the FP32 ones in either precision)
         hipLaunchKernelGGL(faces_list_kernel<kFaceListCap>, dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);

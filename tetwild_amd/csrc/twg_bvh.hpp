@@ -1186,75 +1186,135 @@ __device__ bool face_out_listed(const BvhWalk& B, const double* t9, double eps2,
     });
 }
 
-// face_out_sampled's decision computed by a group of G lanes (G a power of
-// two up to 64, groups aligned in the wave; every lane of a group passes the
-// same triangle), against a collect_facets list with its certificates (lst,
-// cert, F, nl >= 0; its box holding the triangle padded by more than sqrt(T))
-// or the tree (nl < 0).  A facet that certifies the three corners settles the
-// triangle.  Otherwise the sampler's sequence of `total` samples is cut into G
-// consecutive blocks of K = ceil(total / G); lane r moves to sample r K
-// (SampleGen::skip passes whole rows by their headers) and tests its block
-// in order -- when a facet certifies a sample and the last one of the lane's
-// run along the same row, the ones between are passed over -- and after each
-// step a ballot over the group stops it at the first sample found outside.
-// The decision -- some sample has no facet within eps -- does not depend on
-// which lane tests which sample, so it equals face_out_sampled's.  For batches
-// of few triangles with many samples each, where one lane per triangle leaves
-// most of the machine idle.
-template <bool F32, int G, bool SUBTREE = true>
-__device__ bool face_out_group(const BvhWalk& B, V3<double> a, V3<double> b, V3<double> c,
-                               double eps2, double d, double T, double sqrtT, int r, int gbase,
-                               LdsNode32W* lst, LdsF32* cert, const CertFrame& F, int nl)
+// LDS of face_out_wave per wave: a triangle's segment record and header
+// (SampleGen::store_seg) and its row table
+constexpr int kWaveRows = 96;
+constexpr int kWaveSegBytes = kSegRec * 8 + kSegHdr * 4 + kWaveRows * kSegRow * 8;
+typedef __attribute__((address_space(3))) int LdsI32;
+
+// face_out_sampled's decision computed by a wave (every lane passes the same
+// triangle, r its lane), against a collect_facets list with its certificates
+// (lst, cert, F, nl >= 0; its box holding the triangle padded by more than
+// sqrt(T)) or the tree (nl < 0).  A facet that certifies the three corners
+// settles the triangle.  Otherwise the sampler's sequence of `total` samples is
+// cut into 64 consecutive blocks of K = ceil(total / 64); lane r finds sample
+// r K and tests its block in order -- when a facet certifies a sample and the
+// last one of the lane's run along the same row, the ones between are passed
+// over -- and after each step a ballot stops the wave at the first sample
+// found outside.  A triangle of up to kWaveRows rows has them made a row per
+// lane in LDS (seg, kWaveSegBytes; seg_row: a row needs nothing from the ones
+// before it); the lanes of a taller one pass whole rows by their headers
+// (SampleGen::skip), one after another.  12 triangles of ~800 samples: 159 ->
+// 66 us, 30 k of ~90 797 -> 343.  The decision -- some sample has no facet within eps -- does
+// not depend on which lane tests which sample, so it equals
+// face_out_sampled's.  For batches of few triangles with many samples each,
+// where one lane per triangle leaves most of the machine idle.
+template <bool F32, bool SUBTREE = true>
+__device__ bool face_out_wave(const BvhWalk& B, V3<double> a, V3<double> b, V3<double> c, double eps2,
+                              double d, double T, double sqrtT, int r, LdsNode32W* lst, LdsF32* cert,
+                              const CertFrame& F, int nl, LdsF64* seg)
 {
-    static_assert(G >= 2 && G <= 64 && (G & (G - 1)) == 0, "group size");
     {
         double l = fmax(len2(a - b), fmax(len2(b - c), len2(c - a)));
         if (!(__builtin_sqrt(l) / d <= kMaxEdgeSamples)) return true;
     }
-    const unsigned long long gmask = G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull;
     if (nl > 0 && F.runs) {
         const V3<float> qa = cert_local(F, a), qb = cert_local(F, b), qc = cert_local(F, c);
         bool all = false;
-        for (int e = r; e < nl; e += G) {
+        for (int e = r; e < nl; e += 64) {
             LdsF32* ce = cert + kCertFloats * e;
             all = all || (cert_class(ce, qa, F) > 0 && cert_class(ce, qb, F) > 0 &&
                           cert_class(ce, qc, F) > 0);
         }
-        if ((__ballot(all) >> gbase) & gmask) return false;
+        if (__ballot(all)) return false;
     }
-    int64_t total;
-    {
-        SampleGen cnt;
-        cnt.init(a, b, c, d);
-        total = cnt.skip(INT64_MAX);
-    }
-    const int64_t K = (total + G - 1) / G;
-    const int64_t first = (int64_t)r * K;
-    const int64_t mine = total - first < K ? total - first : K;
     SampleGen g;
     g.init(a, b, c, d);
-    g.skip(first);
+    const int rows = g.phase != 9 && g.M >= 1 ? g.M : 0;
+    const bool table = rows <= kWaveRows;
+    LdsF64* row = seg + kSegRec;
+    LdsI32* hdr = (LdsI32*)(row + kWaveRows * kSegRow);
+    SegFace S;
+    int64_t total;
+    if (table) {
+        if (r == 0) g.store_seg(seg, hdr, 0);
+        wave_sync();
+        int made = rows, sum = 0;  // the rows before the first that ends, their samples
+        for (int m0 = 0; m0 < rows; m0 += 64) {
+            const int m = m0 + r;
+            int rc = 0;
+            if (m < rows) {
+                V3<double> st = mk3(0.0, 0.0, 0.0);
+                rc = seg_row(seg, d, m + 1, st);
+                row[kSegRow * m] = st.x;
+                row[kSegRow * m + 1] = st.y;
+                row[kSegRow * m + 2] = st.z;
+                row[kSegRow * m + 3] = (double)rc;
+            }
+            const unsigned long long end = __ballot(m < rows && rc == 0);
+            if (end && made > m0 + __builtin_ctzll(end)) made = m0 + __builtin_ctzll(end);
+            sum += m < made ? rc : 0;
+        }
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        if (r == 0) hdr[kShRows] = made;
+        wave_sync();
+        S.load(hdr);
+        total = S.total(sum);
+    } else {
+        total = g.skip(INT64_MAX);
+        g.init(a, b, c, d);
+    }
+    const int64_t K = (total + 63) / 64;
+    const int64_t first = (int64_t)r * K;
+    const int64_t mine = total - first < K ? total - first : K;
+    int ss = 0, sk = 0, sc = 0;
+    if (mine > 0) {
+        if (table) {
+            S.seek(row, first, ss, sk);
+            sc = S.count(row, ss);
+        } else {
+            g.skip(first);
+        }
+    }
     int hint = -1, hl = -1;
     Stats st;
     const uint64_t mask[2] = {~0ull >> (nl < 64 && nl > 0 ? 64 - nl : 0),
                               nl > 64 ? ~0ull >> (128 - nl) : 0ull};
-    for (int64_t j = 0; (__ballot(j < mine) >> gbase) & gmask;) {
+    for (int64_t j = 0; __ballot(j < mine);) {
         V3<double> q = a;
-        const bool have = j < mine && g.next(q);
-        bool out = false, sure = false;
+        bool have = j < mine, out = false, sure = false;
+        if (have && table) {
+            while (sk >= sc) {  // past the segments with no samples left
+                sk = 0;
+                if (++ss >= S.nseg()) {
+                    have = false;
+                    break;
+                }
+                sc = S.count(row, ss);
+            }
+            if (have) q = S.sample(seg, row, ss, sk++, d);
+        } else if (have) {
+            have = g.next(q);
+        }
         if (have) {
             if (nl >= 0) out = !in_envelope_cert(B, lst, cert, nl, mask, q, F, eps2, hl, sure);
             else out = !in_envelope<F32, false, SUBTREE>(B, q, eps2, T, sqrtT, hint, st);
         }
         ++j;
         if (sure && !out && F.runs && j < mine) {
-            const int64_t left = g.run_left(mine - j);
-            if (left > 0 && cert_class(cert + kCertFloats * hl, cert_local(F, g.run_at(left)), F) > 0) {
-                g.k += (int)left;
-                j += left;
+            int64_t left = mine - j;
+            if (table) left = sc - sk < left ? sc - sk : left;
+            else left = g.run_left(left);
+            if (left > 0) {
+                const V3<double> e = table ? S.sample(seg, row, ss, sk + (int)left - 1, d) : g.run_at(left);
+                if (cert_class(cert + kCertFloats * hl, cert_local(F, e), F) > 0) {
+                    j += left;
+                    if (table) sk += (int)left;
+                    else g.k += (int)left;
+                }
             }
         }
-        if ((__ballot(out) >> gbase) & gmask) return true;
+        if (__ballot(out)) return true;
     }
     return false;
 }
