@@ -104,6 +104,7 @@ int twg_ctx_destroy(twg_ctx* ctx)
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     for (int i = 0; i < 4; ++i)
         if (ctx->slot[i]) (void)hipFree(ctx->slot[i]);
+    if (ctx->host_out) (void)hipHostFree(ctx->host_out);
     if (ctx->list_stats) (void)hipFree(ctx->list_stats);
     if (ctx->order) (void)hipEventDestroy(ctx->order);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);

@@ -4,13 +4,19 @@
 // getFilterEnergy (src/tetwild/LocalOperations.cpp:605-693), in one pass over
 // the per-tet slim energies resident in HBM.
 //
-// Each block walks a contiguous range of the tets; blocks reduce through LDS
-// in a fixed tree and write partials; one block reduces the partials in the same fixed
-// order.  The result is deterministic for a given device (the grid depends
+// Each block walks a contiguous range of the tets; waves reduce by shuffles in
+// a fixed tree, a block's four waves in order, and one block reduces the blocks'
+// partials the same way.  Bound by the latency of the locked flags' gathers
+// (ids, then four bytes each), so all flags of a thread's four tets are read
+// before any is used (four blocks a CU; two and eight 60 and 70 us against 57).
+// 3.1 M tets with locks 75 -> 57 us a call, 24 tets 43 -> 30: the flags tested
+// one after another, an LDS tree over 128-byte records and a copy of the
+// result after the kernels took the difference.  The result is deterministic for a given device (the grid depends
 // only on the CU count).  Max, second max, counts and the histogram are exact;
 // the sum differs from the reference's sequential loop by rounding only.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "twg_internal.hpp"
 #include "twg_math.hpp"
@@ -48,26 +54,35 @@ __device__ __forceinline__ void combine(Partial& a, const Partial& b)
     for (int k = 0; k < 11; ++k) a.buckets[k] += b.buckets[k];
 }
 
-// fixed-shape tree over the block: thread t combines t + s for s = 128 .. 1
+// the wave's partials into every lane (a fixed tree: lanes 32 apart first)
+__device__ __forceinline__ void wave_combine(Partial& p)
+{
+    for (int off = 32; off > 0; off >>= 1) {
+        Partial q;
+        q.sum = __shfl_xor(p.sum, off, 64);
+        q.max = __shfl_xor(p.max, off, 64);
+        q.second = __shfl_xor(p.second, off, 64);
+        q.count = __shfl_xor(p.count, off, 64);
+        q.bad = __shfl_xor(p.bad, off, 64);
+#pragma unroll
+        for (int k = 0; k < 11; ++k) q.buckets[k] = __shfl_xor(p.buckets[k], off, 64);
+        combine(p, q);
+    }
+}
+
+// the block's partials, its waves' in order, in thread 0
 __device__ void block_reduce(Partial& p, Partial* lds)
 {
-    const int t = threadIdx.x;
-    lds[t] = p;
+    wave_combine(p);
+    if (threadIdx.x % 64 == 0) lds[threadIdx.x / 64] = p;
     __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (t < s) {
-            Partial q = lds[t];
-            combine(q, lds[t + s]);
-            lds[t] = q;
-        }
-        __syncthreads();
-    }
-    p = lds[0];
+    if (threadIdx.x == 0)
+        for (int w = 1; w < kBlock / 64; ++w) combine(p, lds[w]);
 }
 
 __global__ __launch_bounds__(kBlock) void energy_partial_kernel(ReduceArgs A)
 {
-    __shared__ Partial lds[kBlock];
+    __shared__ Partial lds[kBlock / 64];
     Partial p;
     p.sum = 0.0;
     p.max = 0.0;
@@ -76,6 +91,8 @@ __global__ __launch_bounds__(kBlock) void energy_partial_kernel(ReduceArgs A)
     p.bad = 0;
 #pragma unroll
     for (int k = 0; k < 11; ++k) p.buckets[k] = 0;
+    // counts of one thread: far below 2^32
+    unsigned count = 0, bad = 0, bucket[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     // Each block walks its own contiguous range (blocks in XCD order, so the
     // vertex flags its tets read stay in one L2), kUnroll coalesced elements
     // per thread per step with their loads issued before any is used.
@@ -96,6 +113,23 @@ __global__ __launch_bounds__(kBlock) void energy_partial_kernel(ReduceArgs A)
             ev[u] = in ? A.e[i] : 0.0;
             tv[u] = in && use_locks ? A.tets[i] : make_int4(0, 0, 0, 0);
         }
+        // isTetLocked_ui (:1377-1384): bit 0 locked, bit 1 an id out of range
+        unsigned lk[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            lk[u] = 0u;
+            if (!use_locks) continue;
+            const int4 t = tv[u];
+            const int id[4] = {t.x, t.y, t.z, t.w};
+            unsigned out = 0u, any = 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool in = id[j] >= 0 && id[j] < A.nv;
+                out |= in ? 0u : 2u;
+                any |= A.nv > 0 ? (unsigned)A.locked[in ? id[j] : 0] : 0u;
+            }
+            lk[u] = out ? out : (any ? 1u : 0u);
+        }
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
             if (rm[u]) continue;
@@ -111,24 +145,20 @@ __global__ __launch_bounds__(kBlock) void energy_partial_kernel(ReduceArgs A)
                     if (e > A.lim[j] && e <= A.lim[j + 1]) bk = j;
             }
 #pragma unroll
-            for (int k = 0; k < 11; ++k) p.buckets[k] += (bk == k) ? 1ull : 0ull;
-            // isTetLocked_ui (:1377-1384)
-            if (use_locks) {
-                const int4 t = tv[u];
-                if (t.x < 0 || t.x >= A.nv || t.y < 0 || t.y >= A.nv || t.z < 0 || t.z >= A.nv ||
-                    t.w < 0 || t.w >= A.nv) {
-                    p.bad++;
-                    continue;
-                }
-                if (A.locked[t.x] || A.locked[t.y] || A.locked[t.z] || A.locked[t.w]) continue;
-            }
+            for (int k = 0; k < 11; ++k) bucket[k] += (bk == k) ? 1u : 0u;
+            if (lk[u] & 2u) bad++;
+            if (lk[u]) continue;
             // getAvgMaxEnergy / getMaxEnergy (:605-635), getSecondMaxEnergy (:637-650)
             p.max = e > p.max ? e : p.max;
             if (e != kMaxEnergy) p.second = e > p.second ? e : p.second;
             p.sum += e;
-            p.count++;
+            count++;
         }
     }
+    p.count = count;
+    p.bad = bad;
+#pragma unroll
+    for (int k = 0; k < 11; ++k) p.buckets[k] = bucket[k];
     block_reduce(p, lds);
     if (threadIdx.x == 0) A.part[blockIdx.x] = p;
 }
@@ -136,7 +166,7 @@ __global__ __launch_bounds__(kBlock) void energy_partial_kernel(ReduceArgs A)
 __global__ __launch_bounds__(kBlock) void energy_final_kernel(Partial* part, int nblocks,
                                                               Partial* out)
 {
-    __shared__ Partial lds[kBlock];
+    __shared__ Partial lds[kBlock / 64];
     Partial p;
     p.sum = 0.0;
     p.max = 0.0;
@@ -175,16 +205,24 @@ extern "C" int twg_energy_stats(twg_ctx* ctx, const double* slim_energy, int64_t
     for (int j = 0; j <= 10; ++j) A.lim[j] = filter_energy_thres - 1 + std::pow(10.0, (double)j);
     if (int r = bind(ctx)) return r;
     const int nblocks = (int)std::max<int64_t>(1, std::min<int64_t>(grid_for(n), (int64_t)ctx->num_cus * 4));
-    if (int r = ensure_scratch(ctx, sizeof(Partial) * (size_t)(nblocks + 1))) return r;
-    A.part = static_cast<Partial*>(ctx->scratch);
-    Partial* dout = A.part + nblocks;
+    // the result goes to pinned host memory: no copy after the kernels, and one
+    // block is its own final pass
+    static_assert(sizeof(Partial) <= kHostOutBytes, "room for the result");
+    if (!ctx->host_out) TWG_HIP(hipHostMalloc(&ctx->host_out, kHostOutBytes, hipHostMallocDefault));
+    void* dout = nullptr;
+    TWG_HIP(hipHostGetDevicePointer(&dout, ctx->host_out, 0));
+    if (int r = ensure_scratch(ctx, sizeof(Partial) * (size_t)nblocks)) return r;
+    A.part = nblocks == 1 ? static_cast<Partial*>(dout) : static_cast<Partial*>(ctx->scratch);
     hipLaunchKernelGGL(energy_partial_kernel, dim3(nblocks), dim3(kBlock), 0, ctx->cur, A);
     TWG_LAUNCHED();
-    hipLaunchKernelGGL(energy_final_kernel, dim3(1), dim3(kBlock), 0, ctx->cur, A.part, nblocks, dout);
-    TWG_LAUNCHED();
-    Partial h;
-    TWG_HIP(hipMemcpyAsync(&h, dout, sizeof h, hipMemcpyDeviceToHost, ctx->cur));
+    if (nblocks > 1) {
+        hipLaunchKernelGGL(energy_final_kernel, dim3(1), dim3(kBlock), 0, ctx->cur, A.part, nblocks,
+                           static_cast<Partial*>(dout));
+        TWG_LAUNCHED();
+    }
     TWG_HIP(hipStreamSynchronize(ctx->cur));
+    Partial h;
+    std::memcpy(&h, ctx->host_out, sizeof h);
     TWG_REQUIRE(h.bad == 0, "twg_energy_stats: %llu tets with vertex ids outside [0, nv)",
                 (unsigned long long)h.bad);
     out->sum = h.sum;

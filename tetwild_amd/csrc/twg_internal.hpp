@@ -35,7 +35,10 @@ struct twg_ctx {
     // waves that tested their LDS facet list, waves that walked the tree
     unsigned long long* list_stats = nullptr;
     bool list_stats_on = false;
+    // pinned host memory a kernel writes a synchronous call's result to
+    void* host_out = nullptr;
 };
+constexpr size_t kHostOutBytes = 256;
 
 namespace twg {
 
