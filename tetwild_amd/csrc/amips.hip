@@ -8,8 +8,12 @@
 // transpose, so each
 // store instruction covers 64 consecutive elements and the kernel emits three
 // sequential write streams (planar outputs -- thirteen streams -- measured
-// ~35% slower on MI355X).  Vertex ids outside [0, nv) make the tet's outputs NaN (flip
-// test: flipped) instead of reading out of bounds.
+// ~35% slower on MI355X).  Blocks go to the XCDs in runs of 64
+// (xcd_run_block).  Reading the ids nontemporally on top of that takes 317 ->
+// 260 us on three meshes of 10.1 M tets in turn but 218 -> 265 on one evaluated
+// again and again, whose ids the last-level cache then loses: plain reads stay.
+// Vertex ids outside [0, nv) make the tet's outputs NaN (flip test: flipped)
+// instead of reading out of bounds.
 #include "twg_internal.hpp"
 #include "twg_math.hpp"
 
@@ -87,7 +91,7 @@ __global__ __launch_bounds__(kBlock) void amips_eval_kernel(
     double* __restrict__ G, double* __restrict__ H)
 {
     __shared__ double lds[kBlock * 9];
-    const int64_t base = xcd_block() * kBlock;
+    const int64_t base = xcd_run_block() * kBlock;
     const int64_t i = base + threadIdx.x;
     double e = 0.0, g[3] = {0.0, 0.0, 0.0}, h[9];
 #pragma unroll
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(kBlock) void amips_mixed_kernel(
     uint8_t* __restrict__ fallback)
 {
     __shared__ float lds[kBlock * 9];
-    const int64_t base = xcd_block() * kBlock;
+    const int64_t base = xcd_run_block() * kBlock;
     const int64_t i = base + threadIdx.x;
     float g[3] = {0.f, 0.f, 0.f}, h[9];
 #pragma unroll
@@ -288,7 +292,7 @@ __global__ __launch_bounds__(kBlock) void tet_quality_kernel(
     const double* __restrict__ y, const double* __restrict__ z, int64_t nv, float tol,
     double* __restrict__ out, uint8_t* __restrict__ fallback, Pending P)
 {
-    const int64_t i = xcd_block() * kBlock + threadIdx.x;
+    const int64_t i = xcd_run_block() * kBlock + threadIdx.x;
     if (i >= n) return;
     Tet T;
     uint8_t fb = 0;
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(kBlock) void tet_flip_kernel(const int32_t* __restr
                                                           const double* __restrict__ z, int64_t nv,
                                                           uint8_t* __restrict__ flipped, Pending P)
 {
-    const int64_t i = xcd_block() * kBlock + threadIdx.x;
+    const int64_t i = xcd_run_block() * kBlock + threadIdx.x;
     if (i >= n) return;
     Tet T;
     bool pend = false;

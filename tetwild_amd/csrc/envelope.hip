@@ -52,19 +52,6 @@ __global__ __launch_bounds__(kBlock) void points_kernel(BvhView B, const double*
     if (STATS) flush_stats(st, stats);
 }
 
-// xcd_block for work that is uneven along the items (sorted queries): each XCD
-// takes runs of 64 consecutive blocks in turn instead of a contiguous eighth,
-// so no XCD is left with a long eighth (3 M triangles 2187 -> 1812 us with the
-// one-wave blocks of faces_list_kernel: 31 % of the CU time had been idle).
-__device__ __forceinline__ int64_t xcd_run_block()
-{
-    const unsigned g = gridDim.x, b = blockIdx.x;
-    const unsigned whole = g / 512 * 512;
-    if (b >= whole) return b;
-    const unsigned k = b / 8;
-    return (int64_t)(k / 64) * 512 + (b % 8) * 64 + k % 64;
-}
-
 // Waves whose facets do not fit their list take their items in halves, down to
 // this many lanes.
 constexpr int kListSplit = 8;
