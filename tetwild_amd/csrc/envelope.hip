@@ -419,17 +419,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
 
 // A wave per triangle, its samples spread over the lanes (face_out_wave): for
 // small batches, so that few triangles with many samples each still fill the
-// machine.  Same outputs and pending queue as faces_kernel.  The tree is read
-// from global memory throughout (listing through an LDS copy of its top ran
+// machine.  Same outputs as faces_kernel; triangles the degeneracy filter cannot
+// settle are marked in out for faces_marked_kernel (a queue's counter would
+// take a launch of its own to clear).  The tree is read from global memory
+// throughout (listing through an LDS copy of its top ran
 // ~5 % slower here, and only lists that do not fit walk it).
+constexpr uint8_t kFacePending = 2;
 constexpr int kWaveListCap = 64;
 constexpr int kWaveListBytes = kWaveListCap * kCertEntryBytes;
 template <bool F32>
 __global__ __launch_bounds__(kBlock) void faces_wave_kernel(BvhView B, const double* __restrict__ tri9,
                                                             int64_t n, double eps2, double d,
                                                             double T, double sqrtT,
-                                                            uint8_t* __restrict__ out,
-                                                            unsigned* n_pending, int64_t* pending)
+                                                            uint8_t* __restrict__ out)
 {
     __shared__ __align__(16) unsigned char face_lists[(kBlock / 64) * kWaveListBytes];
     __shared__ double seg[(kBlock / 64) * kWaveSegBytes / 8];
@@ -439,10 +441,7 @@ __global__ __launch_bounds__(kBlock) void faces_wave_kernel(BvhView B, const dou
     if (i >= n) return;
     const double* t = tri9 + 9 * i;
     if (!certainly_not_collinear(t, t + 3, t + 6)) {
-        if (r == 0) {
-            unsigned k = atomicAdd(n_pending, 1u);
-            pending[k] = i;
-        }
+        if (r == 0) out[i] = kFacePending;
         return;
     }
     // the facets near the triangle, listed in the wave's LDS (the tree walk
@@ -475,6 +474,17 @@ __global__ __launch_bounds__(kBlock) void faces_wave_kernel(BvhView B, const dou
     const bool o = face_out_wave<F32>(W, ld3(t), ld3(t + 3), ld3(t + 6), eps2, d, T, sqrtT, r, lst, cert, F, nl,
                                       (LdsF64*)seg + (threadIdx.x / 64) * (kWaveSegBytes / 8));
     if (r == 0) out[i] = o ? 1 : 0;
+}
+
+template <bool F32>
+__global__ __launch_bounds__(kBlock) void faces_marked_kernel(BvhView B, const double* __restrict__ tri9,
+                                                              int64_t n, double eps2, double d, double T,
+                                                              double sqrtT, uint8_t* __restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n || out[i] != kFacePending) return;
+    Stats st;
+    out[i] = face_out<F32, false>(walk(B), tri9 + 9 * i, eps2, d, T, sqrtT, st) ? 1 : 0;
 }
 
 template <bool F32>
@@ -896,24 +906,32 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
                 "twg_envelope_faces: sampling_dist must be positive");
     if (n == 0) return TWG_OK;
     if (int r = bind(ctx)) return r;
-    if (int r = ensure_scratch(ctx, 256 + sizeof(int64_t) * (size_t)n)) return r;
-    unsigned* n_pending = (unsigned*)ctx->scratch;
-    int64_t* pending = (int64_t*)((char*)ctx->scratch + 256);
     double T = bvh_prune_threshold(B, eps2), sT = std::sqrt(T);
     dim3 g(grid_for(n)), b(kBlock);
     BvhView v = bvh_view(B);
+    if (n < kWaveMax && !stats) {
+        const dim3 gw(grid_for(n * 64));
+        if (precision == TWG_FP64) {
+            hipLaunchKernelGGL(faces_wave_kernel<false>, gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out);
+            TWG_LAUNCHED();
+            hipLaunchKernelGGL(faces_marked_kernel<false>, g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out);
+        } else {
+            hipLaunchKernelGGL(faces_wave_kernel<true>, gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out);
+            TWG_LAUNCHED();
+            hipLaunchKernelGGL(faces_marked_kernel<true>, g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out);
+        }
+        TWG_LAUNCHED();
+        return TWG_OK;
+    }
+    if (int r = ensure_scratch(ctx, 256 + sizeof(int64_t) * (size_t)n)) return r;
+    unsigned* n_pending = (unsigned*)ctx->scratch;
+    int64_t* pending = (int64_t*)((char*)ctx->scratch + 256);
     const int32_t* order = nullptr;
     if (n >= kSortMin)
         if (int r = morton_order(ctx, tri9, n, 9, B->lo, B->hi, &order)) return r;
     hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, ctx->cur, n_pending);
     TWG_LAUNCHED();
-    if (n < kWaveMax && !stats) {
-        dim3 gw(grid_for(n * 64));
-        if (precision == TWG_FP64)
-            hipLaunchKernelGGL(faces_wave_kernel<false>, gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending);
-        else
-            hipLaunchKernelGGL(faces_wave_kernel<true>, gw, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending);
-    } else if (order && !stats && n >= kFaceListDensity * B->nf) {
+    if (order && !stats && n >= kFaceListDensity * B->nf) {
         // (the list's boxes, and the few tree walks', are the FP32 ones in either precision)
         hipLaunchKernelGGL(faces_list_kernel<kFaceListCap>, dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
     } else if (precision == TWG_FP64) {

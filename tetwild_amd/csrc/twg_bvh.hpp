@@ -486,6 +486,9 @@ __device__ __forceinline__ double tri_d2(LdsF64c* t, V3<double> p)
                                        mk3(t[6], t[7], t[8]), cp);
 }
 
+// (in_envelope_list, face_list_mask's in_envelope_masked and face_out_listed are
+// the plain forms of in_envelope_cert's decision, without certificates; the
+// host checks reach them, no kernel does.)
 // in_envelope's decision for a point p of the box that a collect_facets list
 // was made for, with that box padded by at least sqrt(T) beyond every point
 // tested (then the list holds every facet the tree walk could accept): the
