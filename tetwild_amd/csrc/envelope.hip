@@ -985,7 +985,14 @@ int twg_nearest_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_t
     const dim3 b(kBlock);
     BvhView v = bvh_view(B);
     const int32_t* order = nullptr;
-    if (n >= kSortMin && n < (int64_t(1) << 31))
+    // (a captured graph would keep the address of the context's ordering memory,
+    // which a later call may grow: it walks the points as they come)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->cur, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusActive;
+    }
+    if (cap == hipStreamCaptureStatusNone && n >= kSortMin && n < (int64_t(1) << 31))
         if (int r = morton_order(ctx, p3, n, 3, B->lo, B->hi, &order)) return r;
     constexpr int64_t kPart = 1 << 26;  // a launch holds fewer than 2^32 threads
     for (int64_t at = 0; at < n; at += kPart) {
