@@ -401,8 +401,8 @@ int twg_collapse_plan_destroy(twg_collapse_plan* plan);
  * (:575-588, max over the group starting from 0), else max_q[g] = NaN.  The
  * evaluation step of EdgeRemover::removeAnEdge_32 / _44 / _56
  * (src/tetwild/EdgeRemover.cpp:138-174, 327-368, 501-575): one group per
- * configuration; the caller keeps the selection logic.  One thread per group:
- * meant for small groups (a few tets).  Identical to the CPU restatement. */
+ * configuration; the caller keeps the selection logic.  Meant for small groups
+ * (a few tets).  Identical to the CPU restatement. */
 int twg_tet_groups(twg_ctx* ctx, const int32_t* tets, const int32_t* group_off, int64_t n_groups,
                    int64_t n_tets, const double* x, const double* y, const double* z, int64_t nv,
                    uint8_t* flipped, double* max_q, double* q);

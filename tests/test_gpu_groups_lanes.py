@@ -58,3 +58,43 @@ def test_group_sizes(size):
     fl2 = ctx.tet_groups(dev[0], bad, *dev[2:], want_q=False)[0].cpu().numpy()
     assert (fl2[[2, 3, 8, 9]] == 2).all() and np.array_equal(np.delete(fl2, [2, 3, 8, 9]), np.delete(fl, [2, 3, 8, 9]))
     ctx.close()
+
+
+@pytest.mark.parametrize("n,lo,hi", [(1, 1, 6), (63, 4, 4), (64, 4, 4), (65, 4, 4), (257, 0, 9), (900, 2, 6),
+                                     (70, 28, 36), (40, 60, 70)])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_groups_of_a_wave(n, lo, hi, extra):
+    """Waves whose groups just fill their LDS, miss it by one tet, straddle the
+    batch's end or hold an offset out of range, groups of mixed sizes and empty
+    ones, flipped and coplanar tets among them"""
+    import torch
+
+    from oracle import oracle as O
+    from tetwild_amd import workloads as W
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    x, y, z, tets, _ = W.kuhn_lattice(6, seed=3)
+    r = np.random.default_rng(n * 100 + hi)
+    size = r.integers(lo, hi + 1, n)
+    size[n // 2] += extra
+    off = np.concatenate([[0], np.cumsum(size)]).astype(np.int32)
+    T = tets[r.integers(0, len(tets), off[-1])].copy()
+    flip = r.random(len(T)) < 0.3 / max(hi, 1)
+    T[flip] = T[flip][:, [0, 1, 3, 2]]
+    flat = r.random(len(T)) < 0.1 / max(hi, 1)
+    T[flat, 3] = T[flat, 2]
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0") for a in (T, off, x, y, z)]
+    fl, mq, q = (t.cpu().numpy() for t in ctx.tet_groups(*dev))
+    ofl, omq, oq = O.tet_groups(T, off, x, y, z)
+    fine = ofl == 0
+    own = np.repeat(np.arange(n), size)
+    assert np.array_equal(fl, ofl) and np.array_equal(mq[fine], omq[fine]) and np.isnan(mq[~fine]).all()
+    assert np.array_equal(q[fine[own]], oq[fine[own]])
+    for k, v in ((n // 3, -1), (n // 2, 2**31 - 1), (n, off[-1] + 1)):
+        bad = dev[1].clone()
+        bad[k] = v
+        fl2, mq2, _ = (t.cpu().numpy() for t in ctx.tet_groups(dev[0], bad, *dev[2:]))
+        hit = np.isin(np.arange(n), (k - 1, k))
+        assert (fl2[hit] == 2).all() and np.isnan(mq2[hit]).all()
+        assert np.array_equal(fl2[~hit], ofl[~hit]) and np.array_equal(mq2[fine & ~hit], omq[fine & ~hit])
+    ctx.close()
