@@ -380,8 +380,8 @@ int twg_collapse_batch(twg_ctx* ctx, const twg_collapse_desc* desc, int precisio
  * twg_collapse_batch would write them. */
 int twg_collapse_autotune(twg_ctx* ctx, const twg_collapse_desc* desc, int precision, int* tile,
                           int* chunk, float* ms);
-/* The batch's launches captured once into a hipGraph (queue reset, persistent
- * ring pass, exact ring pass, point, face, exact face and final passes) and
+/* The batch's launches captured once into a hipGraph (list reset, ring pass,
+ * exact ring pass, point, face, exact face and final passes) and
  * replayed by twg_collapse_plan_run on the context's stream.  The plan owns
  * its scratch; the descriptor's arrays must stay valid while the plan lives. */
 typedef struct twg_collapse_plan twg_collapse_plan;

@@ -273,3 +273,39 @@ def test_collapse_tiles_chunks_autotune_plan(ctx):
         plan.close()
     sf.close()
     bt.close()
+
+
+def test_more_candidates_than_a_launch_has_tiles(ctx):
+    """2^26 candidates and more on 64-lane tiles pass the 2^32 threads of one
+    launch: the ring pass takes several chunks a tile.  Empty rings, with the
+    rings of a small batch at both ends, against that batch's own codes."""
+    M, B = setup()
+    small = CollapseBatch(ctx, B)
+    m = small.n
+    dev = small.status.device
+    n = (1 << 26) + 5
+    half = m // 2
+    off = small.ring_off
+    cut = int(off[half])
+    big = CollapseBatch(ctx, B)
+    keep = [torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(2)]
+    for k, v in zip(keep, (small.v1, small.v2)):
+        k[:half], k[n - (m - half):] = v[:half], v[half:]
+    flags = torch.zeros(n, dtype=torch.uint8, device=dev)
+    flags[:half], flags[n - (m - half):] = small.flags[:half], small.flags[half:]
+    ring_off = torch.full((n + 1,), cut, dtype=torch.int32, device=dev)
+    ring_off[:half], ring_off[n - (m - half):] = off[:half], off[half:]
+    big.status = torch.full((n,), 99, dtype=torch.uint8, device=dev)
+    d = big.desc
+    d.n, d.n_tri, d.check_eps = n, 0, 0
+    d.v1, d.v2, d.flags = keep[0].data_ptr(), keep[1].data_ptr(), flags.data_ptr()
+    d.ring_off, d.status = ring_off.data_ptr(), big.status.data_ptr()
+    small.desc.n_tri, small.desc.check_eps = 0, 0
+    ref, nref = small.run(C.TWG_FP64, tile=64, chunk=1)
+    big.n = n
+    st, nq = big.run(C.TWG_FP64, tile=64, chunk=1)
+    torch.cuda.synchronize()
+    assert torch.equal(st[:half], ref[:half]) and torch.equal(st[n - (m - half):], ref[half:])
+    assert torch.equal(nq.view(torch.int64), nref.view(torch.int64))
+    mid = st[half:n - (m - half)]
+    assert int(mid.min()) == int(mid.max()) != 99

@@ -322,15 +322,20 @@ __device__ void ring_candidate(const CollapseArgs& A, int64_t c, int tl, int wba
 // of its gathers (candidate -> ring ids -> vertices), so the more waves wait
 // the better.  (Persistent tiles popping candidates from one atomic counter
 // ran at the counter's rate, ~6 ns per pop: 200k candidates of 24-tet rings,
-// chunk 1: 1446 us for the whole batch, 360 us this way.)
+// chunk 1: 1446 us for the whole batch, 360 us this way.)  A launch holds fewer
+// than 2^32 threads, 2^26 candidates on 64-lane tiles: from kRingBlocks blocks on
+// a tile takes more than one chunk.
+constexpr int64_t kRingBlocks = 1 << 22;
 template <int TILE>
 __global__ __launch_bounds__(kBlock) void collapse_ring_kernel(CollapseArgs A)
 {
     const int tl = threadIdx.x % TILE;
     const int wbase = (threadIdx.x % 64) - tl;
-    const int64_t c0 = (xcd_block() * (int64_t)(kBlock / TILE) + threadIdx.x / TILE) * A.chunk;
-    const int64_t c1 = c0 + A.chunk < A.n ? c0 + A.chunk : A.n;
-    for (int64_t c = c0; c < c1; ++c) ring_candidate<TILE, false>(A, c, tl, wbase);
+    const int64_t step = (int64_t)gridDim.x * (kBlock / TILE) * A.chunk;
+    for (int64_t c0 = (xcd_block() * (int64_t)(kBlock / TILE) + threadIdx.x / TILE) * A.chunk; c0 < A.n; c0 += step) {
+        const int64_t c1 = c0 + A.chunk < A.n ? c0 + A.chunk : A.n;
+        for (int64_t c = c0; c < c1; ++c) ring_candidate<TILE, false>(A, c, tl, wbase);
+    }
 }
 
 // the candidates the filter pass listed, with the exact predicate; a tile per
@@ -563,7 +568,7 @@ int enqueue(twg_ctx* ctx, const CollapseArgs& A, int tile, bool f32, hipStream_t
 {
     RingFn ring = ring_fn(tile, false);
     const int64_t per = (int64_t)(kBlock / tile) * A.chunk;  // candidates per block
-    const unsigned gring = (unsigned)((A.n + per - 1) / per);
+    const unsigned gring = (unsigned)std::min<int64_t>((A.n + per - 1) / per, kRingBlocks);
     const int64_t need = (A.n * tile + kBlock - 1) / kBlock;
     const unsigned gexact = (unsigned)std::min<int64_t>(std::max<int64_t>(need, 1), 2048);
     hipLaunchKernelGGL(reset_list, dim3(1), dim3(1), 0, s, A.counter);
