@@ -64,7 +64,11 @@ int twg_ctx_destroy(twg_ctx* ctx);
  * context's own).  The context's scratch is shared by all its calls, so the
  * new stream is made to wait (an event, no host wait) for the work already
  * enqueued on the old one -- unless either stream is capturing a graph, in
- * which case ordering the two is the caller's. */
+ * which case ordering the two is the caller's.  A call captured into a graph
+ * keeps its scratch while the context lives, whatever later calls need; the
+ * scratch has to be there before the capture where that forbids allocations
+ * (make the call once outside it), and replays are ordered against the
+ * context's other calls by the caller. */
 int twg_ctx_set_stream(twg_ctx* ctx, void* hip_stream);
 void* twg_ctx_stream(twg_ctx* ctx);
 int twg_ctx_sync(twg_ctx* ctx);

@@ -146,3 +146,60 @@ def test_rows_per_wave(rows):
         out = ctx.envelope_faces(surf, torch.from_numpy(Q).to("cuda:0"), eps * eps, d, precision=prec)
         assert np.array_equal(out.cpu().numpy(), ref), prec
     ctx.close()
+
+
+@pytest.mark.parametrize("what", ["faces", "sparse_faces", "points", "nearest"])
+def test_captured_batch_outlives_larger_calls(what):
+    """A captured batch keeps its ordering and queue memory when larger eager
+    calls on the context outgrow it: replays between such calls, each against
+    the eager result, on inputs that change in place"""
+    import torch
+
+    from tetwild_amd import workloads as W
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    V, F = W.bumpy_sphere(freq=70 if what == "sparse_faces" else 24, seed=2)
+    surf = ctx.surface(V, F)
+    eps, n = 2e-3, 70001
+    sets = [torch.from_numpy(W.query_triangles(V, F, n, eps=eps, edge=0.004, seed=s)).to("cuda:0") for s in (1, 2, 3)]
+    for t in sets:
+        t[5, 3:6] = t[5, 0:3]  # degenerate: the queue is used
+    more = sets[0].repeat(4, 1)
+    q = sets[0].clone()
+    p3 = q[:, :3].contiguous()
+    big3 = more[:, :3].contiguous()
+    if what == "nearest":
+        def call(t, p):
+            return list(ctx.nearest(surf, p))
+    elif what == "points":
+        def call(t, p):
+            return [ctx.envelope_points(surf, p, eps * eps)]
+    else:
+        def call(t, p):
+            return [ctx.envelope_faces(surf, t, eps * eps, eps)]
+    refs = [[r.clone() for r in call(t, t[:, :3].contiguous())] for t in sets]
+    assert not all(torch.equal(a, b) for a, b in zip(refs[0], refs[1]))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(q, p3)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        out = call(q, p3)
+    for k in range(6):
+        q.copy_(sets[k % 3])
+        p3.copy_(sets[k % 3][:, :3])
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, refs[k % 3])), (what, k)
+        if k == 1:
+            ctx.nearest(surf, big3)
+        if k == 2:
+            ctx.envelope_points(surf, big3, eps * eps)
+            ctx.envelope_faces(surf, more, eps * eps, eps)
+        if k == 3:
+            ctx.envelope_faces(surf, more.repeat(2, 1), eps * eps, eps)
+        torch.cuda.synchronize()
+    ctx.close()

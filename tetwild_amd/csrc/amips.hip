@@ -387,8 +387,8 @@ __global__ void zero_count(unsigned* c) { *c = 0u; }
 int pending_slot(twg_ctx* ctx, Pending& P)
 {
     if (int r = ensure_slot(ctx, 0, 256 + sizeof(int64_t) * kPendingCap)) return r;
-    P.count = static_cast<unsigned*>(ctx->slot[0]);
-    P.list = reinterpret_cast<int64_t*>(static_cast<char*>(ctx->slot[0]) + 256);
+    P.count = static_cast<unsigned*>(ctx->slot[0].p);
+    P.list = reinterpret_cast<int64_t*>(static_cast<char*>(ctx->slot[0].p) + 256);
     return TWG_OK;
 }
 

@@ -1,6 +1,7 @@
 // capi.hip -- context management and memory helpers of the C-ABI.
 #include <cstdarg>
 #include <cstring>
+#include <new>
 
 #include "twg_internal.hpp"
 
@@ -30,35 +31,40 @@ int bind(twg_ctx* ctx)
     return TWG_OK;
 }
 
-int ensure_scratch(twg_ctx* ctx, size_t bytes)
+// Memory of at least `bytes` in block m.  A block that a captured graph may
+// hold the address of is never freed while the context lives.
+static int ensure(twg_ctx* ctx, twg_ctx::Block& m, size_t bytes)
 {
-    if (bytes <= ctx->scratch_bytes) return TWG_OK;
-    if (ctx->scratch) {
-        TWG_HIP(hipStreamSynchronize(ctx->cur));
-        TWG_HIP(hipFree(ctx->scratch));
-        ctx->scratch = nullptr;
-        ctx->scratch_bytes = 0;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->cur, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusActive;  // the null stream beside a capturing one
     }
-    size_t want = bytes + bytes / 4;
-    TWG_HIP(hipMalloc(&ctx->scratch, want));
-    ctx->scratch_bytes = want;
+    const bool capturing = cap != hipStreamCaptureStatusNone;
+    if (bytes > m.bytes) {
+        if (m.p && (m.in_graph || capturing)) {
+            twg_ctx::Retired* r = new (std::nothrow) twg_ctx::Retired{m.p, ctx->retired};
+            if (!r) {
+                set_error("out of host memory");
+                return TWG_ENOMEM;
+            }
+            ctx->retired = r;
+        } else if (m.p) {
+            TWG_HIP(hipStreamSynchronize(ctx->cur));
+            TWG_HIP(hipFree(m.p));
+        }
+        m = twg_ctx::Block();
+        const size_t want = bytes + bytes / 4;
+        TWG_HIP(hipMalloc(&m.p, want));
+        m.bytes = want;
+    }
+    m.in_graph = m.in_graph || capturing;
     return TWG_OK;
 }
 
-int ensure_slot(twg_ctx* ctx, int i, size_t bytes)
-{
-    if (bytes <= ctx->slot_bytes[i]) return TWG_OK;
-    if (ctx->slot[i]) {
-        TWG_HIP(hipStreamSynchronize(ctx->cur));
-        TWG_HIP(hipFree(ctx->slot[i]));
-        ctx->slot[i] = nullptr;
-        ctx->slot_bytes[i] = 0;
-    }
-    size_t want = bytes + bytes / 4;
-    TWG_HIP(hipMalloc(&ctx->slot[i], want));
-    ctx->slot_bytes[i] = want;
-    return TWG_OK;
-}
+int ensure_scratch(twg_ctx* ctx, size_t bytes) { return ensure(ctx, ctx->scratch, bytes); }
+
+int ensure_slot(twg_ctx* ctx, int i, size_t bytes) { return ensure(ctx, ctx->slot[i], bytes); }
 
 }  // namespace twg
 
@@ -101,9 +107,14 @@ int twg_ctx_destroy(twg_ctx* ctx)
     if (!ctx) return TWG_OK;
     (void)hipSetDevice(ctx->device);
     if (ctx->cur) (void)hipStreamSynchronize(ctx->cur);
-    if (ctx->scratch) (void)hipFree(ctx->scratch);
-    for (int i = 0; i < 4; ++i)
-        if (ctx->slot[i]) (void)hipFree(ctx->slot[i]);
+    if (ctx->scratch.p) (void)hipFree(ctx->scratch.p);
+    for (twg_ctx::Block& m : ctx->slot)
+        if (m.p) (void)hipFree(m.p);
+    while (twg_ctx::Retired* r = ctx->retired) {
+        ctx->retired = r->next;
+        (void)hipFree(r->p);
+        delete r;
+    }
     if (ctx->host_out) (void)hipHostFree(ctx->host_out);
     if (ctx->list_stats) (void)hipFree(ctx->list_stats);
     if (ctx->order) (void)hipEventDestroy(ctx->order);

@@ -654,7 +654,7 @@ int twg_collapse_batch(twg_ctx* ctx, const twg_collapse_desc* d, int precision, 
     if (A.n == 0) return TWG_OK;
     if ((r = bind(ctx))) return r;
     if ((r = ensure_scratch(ctx, scratch_bytes(A)))) return r;
-    bind_scratch(A, ctx->scratch);
+    bind_scratch(A, ctx->scratch.p);
     const bool f32 = precision == TWG_MIXED;
     int t;
     pick(ctx, A, f32, tile, chunk, t, A.chunk);
@@ -671,7 +671,7 @@ int twg_collapse_autotune(twg_ctx* ctx, const twg_collapse_desc* d, int precisio
     if (r) return r;
     if ((r = bind(ctx))) return r;
     if ((r = ensure_scratch(ctx, scratch_bytes(A)))) return r;
-    bind_scratch(A, ctx->scratch);
+    bind_scratch(A, ctx->scratch.p);
     const bool f32 = precision == TWG_MIXED;
     const int tiles[3] = {16, 32, 64};
     const unsigned chunks[3] = {1, 4, 16};

@@ -876,7 +876,7 @@ int twg_envelope_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_
     const bool group = !stats && (n < kSortMin || (n < kPointGroupMax && n < kPointGroupDensity * B->nf));
     const int32_t* order = nullptr;
     if (n >= kSortMin && !group)
-        if (int r = morton_order(ctx, p3, n, 3, B->lo, B->hi, &order)) return r;
+        if (int r = morton_order(ctx, 1, p3, n, 3, B->lo, B->hi, &order)) return r;
     if (group) {
         const dim3 gg(grid_for(n * kPointGroup));
         if (precision == TWG_FP64) hipLaunchKernelGGL(points_group_kernel<false>, gg, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out);
@@ -924,11 +924,11 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
         return TWG_OK;
     }
     if (int r = ensure_scratch(ctx, 256 + sizeof(int64_t) * (size_t)n)) return r;
-    unsigned* n_pending = (unsigned*)ctx->scratch;
-    int64_t* pending = (int64_t*)((char*)ctx->scratch + 256);
+    unsigned* n_pending = (unsigned*)ctx->scratch.p;
+    int64_t* pending = (int64_t*)((char*)ctx->scratch.p + 256);
     const int32_t* order = nullptr;
     if (n >= kSortMin)
-        if (int r = morton_order(ctx, tri9, n, 9, B->lo, B->hi, &order)) return r;
+        if (int r = morton_order(ctx, 1, tri9, n, 9, B->lo, B->hi, &order)) return r;
     hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, ctx->cur, n_pending);
     TWG_LAUNCHED();
     if (order && !stats && n >= kFaceListDensity * B->nf) {
@@ -985,15 +985,14 @@ int twg_nearest_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_t
     const dim3 b(kBlock);
     BvhView v = bvh_view(B);
     const int32_t* order = nullptr;
-    // (a captured graph would keep the address of the context's ordering memory,
-    // which a later call may grow: it walks the points as they come)
+    // (no ordering memory for a captured graph: it walks the points as they come)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->cur, &cap) != hipSuccess) {
         (void)hipGetLastError();
         cap = hipStreamCaptureStatusActive;
     }
     if (cap == hipStreamCaptureStatusNone && n >= kSortMin && n < (int64_t(1) << 31))
-        if (int r = morton_order(ctx, p3, n, 3, B->lo, B->hi, &order)) return r;
+        if (int r = morton_order(ctx, 2, p3, n, 3, B->lo, B->hi, &order)) return r;
     constexpr int64_t kPart = 1 << 26;  // a launch holds fewer than 2^32 threads
     for (int64_t at = 0; at < n; at += kPart) {
         const dim3 g(grid_for(std::min(n - at, kPart) * kNearestGroup));

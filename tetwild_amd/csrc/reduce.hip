@@ -212,7 +212,7 @@ extern "C" int twg_energy_stats(twg_ctx* ctx, const double* slim_energy, int64_t
     void* dout = nullptr;
     TWG_HIP(hipHostGetDevicePointer(&dout, ctx->host_out, 0));
     if (int r = ensure_scratch(ctx, sizeof(Partial) * (size_t)nblocks)) return r;
-    A.part = nblocks == 1 ? static_cast<Partial*>(dout) : static_cast<Partial*>(ctx->scratch);
+    A.part = nblocks == 1 ? static_cast<Partial*>(dout) : static_cast<Partial*>(ctx->scratch.p);
     hipLaunchKernelGGL(energy_partial_kernel, dim3(nblocks), dim3(kBlock), 0, ctx->cur, A);
     TWG_LAUNCHED();
     if (nblocks > 1) {

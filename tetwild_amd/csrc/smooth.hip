@@ -1435,7 +1435,7 @@ int twg_smooth_autotune(twg_ctx* ctx, const twg_smooth_desc* d, int precision, i
     if (int r = bind(ctx)) return r;
     if (int r = ensure_scratch(ctx, 256)) return r;
     SmoothArgs A;
-    if (int r = make_args(ctx, d, (unsigned*)ctx->scratch, 1, A)) return r;
+    if (int r = make_args(ctx, d, (unsigned*)ctx->scratch.p, 1, A)) return r;
     const int tiles[4] = {16, 32, 64, TWG_SMOOTH_TILE_SPLIT};
     const unsigned chunks[3] = {1, 4, 16};
     EventPair ev;
@@ -1484,7 +1484,7 @@ int twg_smooth_batch(twg_ctx* ctx, const twg_smooth_desc* d, int precision, int 
     int t = tile ? tile : tt;
     unsigned ch = chunk ? (unsigned)chunk : tc;
     SmoothArgs A;
-    if (int r = make_args(ctx, d, (unsigned*)ctx->scratch, ch, A)) return r;
+    if (int r = make_args(ctx, d, (unsigned*)ctx->scratch.p, ch, A)) return r;
     return enqueue(ctx, A, t, precision == TWG_MIXED, ctx->cur);
 }
 

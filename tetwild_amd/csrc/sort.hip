@@ -271,20 +271,19 @@ int sort_pairs(ulonglong2* kv[2], int64_t n, int bits, void* work, hipStream_t s
     return TWG_OK;
 }
 
-int morton_order(twg_ctx* ctx, const double* items, int64_t n, int stride, const double* lo,
+int morton_order(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const double* lo,
                  const double* hi, const int32_t** order)
 {
     TWG_REQUIRE(n < (int64_t(1) << 31), "morton_order: too many items");
     const size_t nb = (size_t)((n + kSortTile - 1) / kSortTile);
-    // slot 1: the box, the digits' totals, two buffers of (key, item), the order
-    if (int r = ensure_slot(ctx, 1, 4096 + (size_t)n * (8 + 8 + 4))) return r;
-    if (int r = ensure_slot(ctx, 2, nb * kDigits * 4)) return r;
-    char* base = (char*)ctx->slot[1];
+    // the box, the digits' totals, two buffers of (key, item), the order, the counts
+    if (int r = ensure_slot(ctx, slot, 4096 + (size_t)n * (8 + 8 + 4) + nb * kDigits * 4)) return r;
+    char* base = (char*)ctx->slot[slot].p;
     double* box = (double*)base;
     unsigned* total = (unsigned*)(base + 1024);
     uint2* kv[2] = {(uint2*)(base + 4096), (uint2*)(base + 4096) + n};
     int32_t* out = (int32_t*)(kv[1] + n);
-    unsigned* count = (unsigned*)ctx->slot[2];
+    unsigned* count = (unsigned*)(out + n);
     static_assert(kDigits * 4 <= 4096 - 1024, "room for the totals");
     Box6 tree;
     for (int k = 0; k < 3; ++k) {

@@ -21,13 +21,26 @@ struct twg_ctx {
     // the new one starts after the old one's use of the shared scratch
     hipEvent_t order = nullptr;
     int num_cus = 256;
-    // growable device scratch owned by the context
-    void* scratch = nullptr;
-    size_t scratch_bytes = 0;
-    // further growable slots: 0 the queue of tets the orientation filter left
-    // undecided, 1 query ordering keys and values, 2 its digit counts
-    void* slot[4] = {nullptr, nullptr, nullptr, nullptr};
-    size_t slot_bytes[4] = {0, 0, 0, 0};
+    // growable device memory owned by the context.  in_graph: a stream was
+    // capturing when a call took it, so a graph may hold its address
+    struct Block {
+        void* p = nullptr;
+        size_t bytes = 0;
+        bool in_graph = false;
+    };
+    Block scratch;
+    // further blocks: 0 the queue of tets the orientation filter left
+    // undecided, 1 the envelope batches' query order, 2 the nearest queries'
+    // (which take none under capture, so they never write to a graph's)
+    Block slot[3];
+    // outgrown blocks that a graph may still use, freed with the context (a
+    // block grows by a quarter at least, so they come to less than five times
+    // the one in use)
+    struct Retired {
+        void* p;
+        Retired* next;
+    };
+    Retired* retired = nullptr;
     // device address of smooth.hip's file-scope scratch array on this
     // context's device (twg_smooth_batch_noalloc), looked up at creation
     void* noalloc_scratch = nullptr;
@@ -52,9 +65,9 @@ int ensure_slot(twg_ctx* ctx, int i, size_t bytes);
 
 // Morton order of n query items (points: stride 3, triangles: stride 9,
 // keyed by their first three coordinates' centroid) inside the box [lo, hi]:
-// writes a permutation (int32, device) into *order (a context slot).  The
-// order only affects speed: every query's result is independent of it.
-int morton_order(twg_ctx* ctx, const double* items, int64_t n, int stride, const double* lo,
+// writes a permutation (int32, device) into *order (in the context's `slot`).
+// The order only affects speed: every query's result is independent of it.
+int morton_order(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const double* lo,
                  const double* hi, const int32_t** order);
 
 // Stable sort of n (key, value) pairs by the low `bits` bits of their keys:
