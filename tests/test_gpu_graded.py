@@ -1,0 +1,55 @@
+"""Surfaces whose facets shrink towards one side: the query order that such a
+surface takes (as many bits as keep crowded cells rare)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def graded_sphere(freq, k):
+    """a geodesic sphere drawn k-fold together towards its south pole (a
+    conformal map, so the facets keep their shapes)"""
+    from tetwild_amd import workloads as W
+    V, F = W.geodesic_sphere(freq)
+    x, y, z = V.T
+    X, Y = (a / (1 - z + 1e-9) / k for a in (x, y))
+    s = X * X + Y * Y
+    return np.ascontiguousarray(np.stack([2 * X / (1 + s), 2 * Y / (1 + s), (s - 1) / (1 + s)], 1)), F
+
+
+def facet_queries(V, F, n, eps, seed):
+    """triangles on facets drawn one by one, their size at most 2.5e-3, offset
+    by up to 2 eps"""
+    r = np.random.default_rng(seed)
+    T = V[F[r.integers(0, len(F), n)]]
+    c = T.mean(1, keepdims=True)
+    N = np.cross(T[:, 1] - T[:, 0], T[:, 2] - T[:, 0])
+    N /= np.linalg.norm(N, axis=1, keepdims=True)
+    size = np.linalg.norm(T - np.roll(T, 1, axis=1), axis=2).max(1)
+    Q = c + (T - c) * np.minimum(1.0, 2.5e-3 / size)[:, None, None] + (r.uniform(-2, 2, n) * eps)[:, None, None] * N[:, None]
+    return np.ascontiguousarray(Q.reshape(n, 9))
+
+
+@pytest.mark.parametrize("freq,k", [(40, 30), (60, 30), (60, 300)])
+def test_order_resolves_the_small_facets(freq, k):
+    """Where all queries of the small side fell into a few cells of the order, a
+    wave's 64 queries lay apart and most lists overflowed"""
+    import torch
+
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    V, F = graded_sphere(freq, k)
+    surf = ctx.surface(V, F)
+    eps = 0.1 / 60 / k
+    tq = torch.from_numpy(facet_queries(V, F, 12 * len(F), eps, k)).to("cuda:0")
+    p3 = tq[:, :3].contiguous()
+    tq = tq[:6 * len(F)]
+    for q, call in ((tq, lambda: ctx.envelope_faces(surf, tq, eps * eps, 1e-3)),
+                    (p3, lambda: ctx.envelope_points(surf, p3, eps * eps))):
+        ctx.list_stats(True)
+        call()
+        listed, walked = ctx.list_stats(False)
+        print(freq, k, listed, walked)
+        assert listed + walked == -(-len(q) // 256) * 4
+        assert walked < 0.2 * listed
+    ctx.close()

@@ -20,6 +20,7 @@ struct BuildScalars {
     unsigned long long lo[3], hi[3];  // of the centroids
     unsigned long long rmax;          // bits of the longest edge
     unsigned long long bad;           // first corner with an id out of range
+    unsigned crowded[2 * kCrowdLevels];  // facets by crowd_level to the kCrowd-th after them
 };
 
 __device__ __forceinline__ unsigned long long ordered(double x)
@@ -27,7 +28,7 @@ __device__ __forceinline__ unsigned long long ordered(double x)
     const unsigned long long b = f2u(x);
     return b >> 63 ? ~b : b | 0x8000000000000000ull;
 }
-__device__ __forceinline__ double unordered(unsigned long long u)
+TWG_HD double unordered(unsigned long long u)
 {
     return u2f(u >> 63 ? u & 0x7FFFFFFFFFFFFFFFull : ~u);
 }
@@ -56,6 +57,7 @@ __global__ void build_init(BuildArgs A)
     }
     A.sc->rmax = 0ull;
     A.sc->bad = ~0ull;
+    for (int k = 0; k < 2 * kCrowdLevels; ++k) A.sc->crowded[k] = 0u;
 }
 
 __device__ __forceinline__ double centroid(const BuildArgs& A, int64_t f, int c)
@@ -134,6 +136,21 @@ __global__ __launch_bounds__(kBlock) void build_keys(BuildArgs A, ulonglong2* __
     r.x = key;
     r.y = (unsigned long long)f;
     kv[f] = r;
+}
+
+// twg_bvh::crowded by level, not summed yet
+__global__ __launch_bounds__(kBlock) void build_crowded(BuildArgs A, const ulonglong2* __restrict__ sorted)
+{
+    __shared__ unsigned n[2 * kCrowdLevels];
+    if (threadIdx.x < 2 * kCrowdLevels) n[threadIdx.x] = 0u;
+    __syncthreads();
+    for (int64_t b = (int64_t)blockIdx.x * kBlock + threadIdx.x; b < A.nf; b += (int64_t)gridDim.x * kBlock)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            if (b + kCrowd[j] < A.nf)
+                atomicAdd(&n[j * kCrowdLevels + crowd_level(sorted[b].x, sorted[b + kCrowd[j]].x)], 1u);
+    __syncthreads();
+    if (threadIdx.x < 2 * kCrowdLevels && n[threadIdx.x]) atomicAdd(&A.sc->crowded[threadIdx.x], n[threadIdx.x]);
 }
 
 // tree position b: the facet's corners, its order entry, its longest edge
@@ -306,6 +323,8 @@ int bvh_build_device(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F
     hipLaunchKernelGGL(build_keys, gf, b, 0, s, A, kv[0]);
     TWG_LAUNCHED();
     if (int r = sort_pairs(kv, nf, 63, work, s)) return r;
+    hipLaunchKernelGGL(build_crowded, dim3(std::min<unsigned>(grid_for(nf), kCheckBlocks)), b, 0, s, A, kv[0]);
+    TWG_LAUNCHED();
     hipLaunchKernelGGL(build_facets, gf, b, 0, s, A, kv[0]);
     TWG_LAUNCHED();
     for (int bottom = depth;;) {
@@ -324,6 +343,11 @@ int bvh_build_device(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F
     TWG_HIP(hipStreamSynchronize(s));
     *bad = h.bad == ~0ull ? -1 : (int64_t)h.bad;
     B->rmax = u2f(h.rmax);
+    for (int c = 0; c < 3; ++c) B->side = std::max(B->side, unordered(h.hi[c]) - unordered(h.lo[c]));
+    for (int j = 0; j < 2; ++j) {
+        int64_t n = 0;
+        for (int l = kCrowdLevels - 1; l >= 0; --l) B->crowded[j][l] = n += h.crowded[j * kCrowdLevels + l];
+    }
     for (int c = 0; c < 3; ++c) {
         B->lo[c] = root.lo[c];
         B->hi[c] = root.hi[c];

@@ -766,6 +766,10 @@ int twg_bvh_build(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F, i
         }
     }
     B->rmax = rmax;
+    for (int c = 0; c < 3; ++c) B->side = std::max(B->side, hi[c] - lo[c]);
+    for (int j = 0; j < 2; ++j)
+        for (int64_t b = 0; b + kCrowd[j] < nf; ++b)
+            for (int l = crowd_level(key[b].first, key[b + kCrowd[j]].first); l >= 0; --l) B->crowded[j][l]++;
     B->nnode = max_node(1, 0, nf) + 1;
     std::vector<BvhNode64> nodes(B->nnode);
     for (auto& N : nodes) {
@@ -876,7 +880,7 @@ int twg_envelope_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_
     const bool group = !stats && (n < kSortMin || (n < kPointGroupMax && n < kPointGroupDensity * B->nf));
     const int32_t* order = nullptr;
     if (n >= kSortMin && !group)
-        if (int r = morton_order(ctx, 1, p3, n, 3, B->lo, B->hi, &order)) return r;
+        if (int r = morton_order(ctx, 1, p3, n, 3, B, &order)) return r;
     if (group) {
         const dim3 gg(grid_for(n * kPointGroup));
         if (precision == TWG_FP64) hipLaunchKernelGGL(points_group_kernel<false>, gg, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out);
@@ -928,7 +932,7 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
     int64_t* pending = (int64_t*)((char*)ctx->scratch.p + 256);
     const int32_t* order = nullptr;
     if (n >= kSortMin)
-        if (int r = morton_order(ctx, 1, tri9, n, 9, B->lo, B->hi, &order)) return r;
+        if (int r = morton_order(ctx, 1, tri9, n, 9, B, &order)) return r;
     hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, ctx->cur, n_pending);
     TWG_LAUNCHED();
     if (order && !stats && n >= kFaceListDensity * B->nf) {
@@ -992,7 +996,7 @@ int twg_nearest_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_t
         cap = hipStreamCaptureStatusActive;
     }
     if (cap == hipStreamCaptureStatusNone && n >= kSortMin && n < (int64_t(1) << 31))
-        if (int r = morton_order(ctx, 2, p3, n, 3, B->lo, B->hi, &order)) return r;
+        if (int r = morton_order(ctx, 2, p3, n, 3, B, &order)) return r;
     constexpr int64_t kPart = 1 << 26;  // a launch holds fewer than 2^32 threads
     for (int64_t at = 0; at < n; at += kPart) {
         const dim3 g(grid_for(std::min(n - at, kPart) * kNearestGroup));

@@ -5,8 +5,8 @@
 #include <cmath>
 #include <utility>
 
+#include "twg_bvh.hpp"
 #include "twg_internal.hpp"
-#include "twg_math.hpp"
 
 namespace twg {
 namespace {
@@ -72,7 +72,8 @@ __global__ __launch_bounds__(kBoxThreads) void query_box(const double* __restric
 // the first pass counts as it makes the keys), a block per digit scans its row
 // and leaves the digit's total, and the items go to their places.  Nothing
 // waits on another block.  27 bits, nine an axis, order 3 M items into cells of
-// about four along a closed surface; below kTwoPassMax items 18 bits do.  Bound
+// about four along a closed surface; below kTwoPassMax items 18 bits do, and a
+// graded surface takes more (morton_bits).  Bound
 // by its launches up to about 1 M items, by the scattered 8-byte writes
 // beyond.  A library radix sort of 63-bit keys, with seventeen memory fills
 // among its launches, took 440 us for 3 M triangles and 200 us for 1 M points;
@@ -84,7 +85,7 @@ constexpr int kSortTile = kBlock * kSortItems;
 constexpr int64_t kTwoPassMax = 1 << 18;
 
 // the item's sort key: the leading `bits` bits of its 63-bit Morton code in the box
-__device__ __forceinline__ uint32_t morton_key(const double* __restrict__ p, int stride,
+__device__ __forceinline__ uint64_t morton_key(const double* __restrict__ p, int stride,
                                                const double* __restrict__ box, int bits)
 {
     double c[3];
@@ -95,7 +96,7 @@ __device__ __forceinline__ uint32_t morton_key(const double* __restrict__ p, int
         const uint64_t qi = !(q > 0.0) ? 0 : (q >= 2097151.0 ? 2097151 : (uint64_t)q);
         key |= spread3d(qi) << k;
     }
-    return (uint32_t)(key >> (63 - bits));
+    return key >> (63 - bits);
 }
 
 // keys (first pass) and the block's digit counts; KV: a (key, item) pair
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(kBlock) void digit_count(const double* __restrict__
         if (i >= n) break;
         KV v;
         if (FIRST) {
-            v.x = morton_key(items + (int64_t)stride * i, stride, box, bits);
+            v.x = (decltype(v.x))morton_key(items + (int64_t)stride * i, stride, box, bits);
             v.y = (uint32_t)i;
             kv[i] = v;
         } else {
@@ -271,44 +272,69 @@ int sort_pairs(ulonglong2* kv[2], int64_t n, int bits, void* work, hipStream_t s
     return TWG_OK;
 }
 
-int morton_order(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const double* lo,
-                 const double* hi, const int32_t** order)
+// Bits of the query order.  Two passes of the sort up to kTwoPassMax items,
+// three beyond, and more where the surface is graded: as many as leave no more
+// than one facet in kCrowdShare in a crowded cell.  (3 M triangles on 246 k
+// facets, 30 and 300 times smaller towards one side: with 27 bits the facets of a
+// wave's queries overflow its list, 8452 and 10780 us a call, with 36 and 45 bits
+// 1414 and 1484.)
+constexpr int64_t kCrowdShare = 64;
+static int morton_bits(const twg_bvh* B, int64_t n)
 {
-    TWG_REQUIRE(n < (int64_t(1) << 31), "morton_order: too many items");
+    constexpr int kLevels = kDigitBits / 3;  // a pass
+    int passes = n < kTwoPassMax ? 2 : 3;
+    while (passes * kLevels < kCrowdLevels - 1 && B->crowded[0][passes * kLevels] * kCrowdShare > B->nf) ++passes;
+    return passes * kDigitBits;
+}
+
+// KV: a (key, item) pair that holds the key's bits
+template <class KV>
+static int order_items(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const Box6& tree,
+                       int bits, const int32_t** order)
+{
     const size_t nb = (size_t)((n + kSortTile - 1) / kSortTile);
     // the box, the digits' totals, two buffers of (key, item), the order, the counts
-    if (int r = ensure_slot(ctx, slot, 4096 + (size_t)n * (8 + 8 + 4) + nb * kDigits * 4)) return r;
+    if (int r = ensure_slot(ctx, slot, 4096 + (size_t)n * (2 * sizeof(KV) + 4) + nb * kDigits * 4)) return r;
     char* base = (char*)ctx->slot[slot].p;
     double* box = (double*)base;
     unsigned* total = (unsigned*)(base + 1024);
-    uint2* kv[2] = {(uint2*)(base + 4096), (uint2*)(base + 4096) + n};
+    KV* kv[2] = {(KV*)(base + 4096), (KV*)(base + 4096) + n};
     int32_t* out = (int32_t*)(kv[1] + n);
     unsigned* count = (unsigned*)(out + n);
     static_assert(kDigits * 4 <= 4096 - 1024, "room for the totals");
-    Box6 tree;
-    for (int k = 0; k < 3; ++k) {
-        tree.lo[k] = lo[k];
-        tree.hi[k] = hi[k];
-    }
     hipStream_t s = ctx->cur;
     hipLaunchKernelGGL(query_box, dim3(1), dim3(kBoxThreads), 0, s, items, n, stride, tree, box);
     TWG_LAUNCHED();
-    const int passes = n < kTwoPassMax ? 2 : 3, bits = passes * kDigitBits;
+    const int passes = bits / kDigitBits;
     const dim3 g((unsigned)nb), b(kBlock);
     for (int p = 0; p < passes; ++p) {
-        uint2 *from = kv[p % 2], *to = kv[1 - p % 2];
+        KV *from = kv[p % 2], *to = kv[1 - p % 2];
         const int shift = p * kDigitBits;
-        if (p == 0) hipLaunchKernelGGL((digit_count<uint2, true>), g, b, 0, s, items, n, stride, box, bits, shift, from, count);
-        else hipLaunchKernelGGL((digit_count<uint2, false>), g, b, 0, s, items, n, stride, box, bits, shift, from, count);
+        if (p == 0) hipLaunchKernelGGL((digit_count<KV, true>), g, b, 0, s, items, n, stride, box, bits, shift, from, count);
+        else hipLaunchKernelGGL((digit_count<KV, false>), g, b, 0, s, items, n, stride, box, bits, shift, from, count);
         TWG_LAUNCHED();
         hipLaunchKernelGGL(digit_scan, dim3(kDigits), b, 0, s, count, (int)nb, total);
         TWG_LAUNCHED();
-        if (p + 1 < passes) hipLaunchKernelGGL((digit_place<uint2, false>), g, b, 0, s, from, n, shift, count, total, to, out);
-        else hipLaunchKernelGGL((digit_place<uint2, true>), g, b, 0, s, from, n, shift, count, total, to, out);
+        if (p + 1 < passes) hipLaunchKernelGGL((digit_place<KV, false>), g, b, 0, s, from, n, shift, count, total, to, out);
+        else hipLaunchKernelGGL((digit_place<KV, true>), g, b, 0, s, from, n, shift, count, total, to, out);
         TWG_LAUNCHED();
     }
     *order = out;
     return TWG_OK;
+}
+
+int morton_order(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const twg_bvh* B,
+                 const int32_t** order)
+{
+    TWG_REQUIRE(n < (int64_t(1) << 31), "morton_order: too many items");
+    Box6 tree;
+    for (int k = 0; k < 3; ++k) {
+        tree.lo[k] = B->lo[k];
+        tree.hi[k] = B->hi[k];
+    }
+    const int bits = morton_bits(B, n);
+    return bits <= 32 ? order_items<uint2>(ctx, slot, items, n, stride, tree, bits, order)
+                      : order_items<ulonglong2>(ctx, slot, items, n, stride, tree, bits, order);
 }
 
 }  // namespace twg

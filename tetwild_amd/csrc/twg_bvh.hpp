@@ -37,12 +37,25 @@ struct BvhNode32 {
 static_assert(sizeof(BvhNode64) == 64, "node64");
 static_assert(sizeof(BvhNode32) == 32, "node32");
 
+// How the facets crowd, from their 63-bit Morton codes: the dispatch of query
+// batches reads it (morton_bits); results never depend on it
+constexpr int kCrowdLevels = 22;
+constexpr int kCrowd[2] = {32, 64};
+
+// levels at which two codes fall into the same cell
+TWG_HD int crowd_level(uint64_t a, uint64_t b) { return a == b ? kCrowdLevels - 1 : (__builtin_clzll(a ^ b) - 1) / 3; }
+
 struct twg_bvh {
     int device = 0;
     double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // root box
     int64_t nf = 0, nnode = 0;
     int depth = 0;
     double rmax = 0.0;
+    // crowded[j][l]: facets past the first kCrowd[j] of their cell l times
+    // halved, the cell of 0 halvings being the cube of side `side` about the
+    // facets' centroids
+    int64_t crowded[2][kCrowdLevels] = {};
+    double side = 0.0;
     BvhNode64* node64 = nullptr;
     BvhNode32* node32 = nullptr;
     double* tri = nullptr;  // nf x 9, tree order

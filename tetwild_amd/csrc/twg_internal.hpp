@@ -64,11 +64,11 @@ int ensure_scratch(twg_ctx* ctx, size_t bytes);
 int ensure_slot(twg_ctx* ctx, int i, size_t bytes);
 
 // Morton order of n query items (points: stride 3, triangles: stride 9,
-// keyed by their first three coordinates' centroid) inside the box [lo, hi]:
-// writes a permutation (int32, device) into *order (in the context's `slot`).
-// The order only affects speed: every query's result is independent of it.
-int morton_order(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const double* lo,
-                 const double* hi, const int32_t** order);
+// keyed by their centroids) near tree B: writes a permutation (int32, device)
+// into *order (in the context's `slot`).  The order only affects speed: every
+// query's result is independent of it.
+int morton_order(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const twg_bvh* B,
+                 const int32_t** order);
 
 // Stable sort of n (key, value) pairs by the low `bits` bits of their keys:
 // kv[0] in and, after the call, out; kv[1] as large; work: sort_pairs_bytes(n).
