@@ -1,5 +1,7 @@
-"""Surfaces whose facets shrink towards one side: the query order that such a
-surface takes (as many bits as keep crowded cells rare)."""
+"""Surfaces whose facets shrink towards one side, and envelopes wider than the
+facets: the query order that such a surface takes (as many bits as keep crowded
+cells rare), wave lists that overflow, and the batches that leave the list and
+lanes-per-point kernels, against the per-query tree walk (the statistics path)."""
 import numpy as np
 import pytest
 
@@ -52,4 +54,33 @@ def test_order_resolves_the_small_facets(freq, k):
         print(freq, k, listed, walked)
         assert listed + walked == -(-len(q) // 256) * 4
         assert walked < 0.2 * listed
+    ctx.close()
+
+
+@pytest.mark.parametrize("k", [1, 10, 300])
+@pytest.mark.parametrize("n", [32767, 32768, 70001, 300000])
+@pytest.mark.parametrize("eps", [1e-5, 1e-3, 0.05])
+def test_decisions(k, n, eps):
+    """Both sides of every rule, coordinates that are not finite in many waves"""
+    import torch
+
+    from tetwild_amd.ops import Context
+    ctx = Context(0)
+    V, F = graded_sphere(34, k)
+    Q = facet_queries(V, F, n, eps, n)
+    Q[7::61, 4] = np.nan
+    Q[11::173, 1] = np.inf
+    Q[13::977] = -np.inf
+    tq = torch.from_numpy(Q).to("cuda:0")
+    p3 = tq[:, :3].contiguous()
+    for nf in (len(F), 500):  # (500: built on the host)
+        surf = ctx.surface(V, F[:nf])
+        for prec in (0, 1):
+            out = ctx.envelope_faces(surf, tq, eps * eps, 1e-3, precision=prec)
+            walk, _ = ctx.envelope_faces(surf, tq, eps * eps, 1e-3, precision=prec, stats=True)
+            assert torch.equal(out, walk), (nf, prec, int((out != walk).sum()))
+            out = ctx.envelope_points(surf, p3, eps * eps, precision=prec)
+            walk, _ = ctx.envelope_points(surf, p3, eps * eps, precision=prec, stats=True)
+            assert torch.equal(out, walk), (nf, prec, int((out != walk).sum()))
+        surf.close()
     ctx.close()

@@ -55,18 +55,36 @@ __global__ __launch_bounds__(kBlock) void points_kernel(BvhView B, const double*
 // Waves whose facets do not fit their list take their items in halves, down to
 // this many lanes.
 constexpr int kListSplit = 8;
+// ... and only while the box is so many times as wide as one query's (`one`: its
+// own extent and the envelope's on both sides): where the envelope is about as
+// wide as the box, a half meets nearly the same facets.  Lanes may hold different
+// boxes where a coordinate is not finite: one answer for the wave.  (Points, 3 M and 1 M of
+// them with an envelope of two facets and 1 M of three: 1849, 1323 and 1774 us a
+// call at 1.5, 2475, 1370 and 1666 at 2.0.  Triangles, 2 M with an envelope of one
+// and a half facets and 106 k with 0.6: 4323 and 1300 us at 2.0, 5243 and 1396 at
+// 1.5.)
+constexpr double kHalvePoints = 1.5, kHalveFaces = 2.0;
+__device__ __forceinline__ bool halves_help(const double lo[3], const double hi[3], double one)
+{
+    return __ballot(fmax(hi[0] - lo[0], fmax(hi[1] - lo[1], hi[2] - lo[2])) >= one) != 0ull;
+}
 
 // points_kernel for small batches: sixteen lanes per point, which list the
 // facets within reach (collect_facets) and test one each -- a chain of a few
 // reads instead of a walk's, with lanes to spare, in the caller's order.  On
 // 246 k facets 4,096 points 143 -> 17 us, 65 k 169 -> 53, 400 k 282 -> 240, but
 // 1 M 451 -> 563 (there the sort pays, and from two points a facet on the wave
-// lists).  Dense batches of 65 k points and more keep the wave lists too.
+// lists).  Dense batches of 65 k points and more keep the wave lists too, and
+// where the envelope is wide (reach_wide) most lists overflow and sixteen lanes
+// walk one point's way: an envelope of three facets, 5 k points 445 -> 222 us, but
+// 60 k 443 -> 670 and 450 k 1003 -> 3965, so from kPointGroupWide points on those
+// keep points_kernel.
 // (Eight and thirty-two lanes: 58 and 61 us for 65 k.)
 constexpr int kPointGroup = 16;
 constexpr int kPointGroupCap = 32;
 constexpr int64_t kPointGroupMax = 1 << 19;
 constexpr int64_t kPointGroupDensity = 8;
+constexpr int64_t kPointGroupWide = 1 << 15;
 template <bool F32>
 __global__ __launch_bounds__(kBlock) void points_group_kernel(BvhView B, const double* __restrict__ p3,
                                                               int64_t n, double eps2, double T,
@@ -104,7 +122,7 @@ __global__ __launch_bounds__(kBlock) void points_group_kernel(BvhView B, const d
 // points padded by more than sqrt(T), with their certificates, and each lane
 // tests its point against the list (in_envelope_cert).  Blocks of one wave and
 // split waves as faces_list_kernel; lanes that no list serves, or that hold a
-// coordinate that is not finite, walk the tree.
+// coordinate that is not finite, walk the tree, all at once at the end.
 template <bool F32, int CAP>
 __global__ __launch_bounds__(64) void points_list_kernel(BvhView B, const double* __restrict__ p3,
                                                          int64_t n, double eps2, double T,
@@ -126,7 +144,7 @@ __global__ __launch_bounds__(64) void points_list_kernel(BvhView B, const double
         p = ld3(p3 + 3 * i);
     }
     const bool fin = is_finite(p.x) && is_finite(p.y) && is_finite(p.z);
-    bool walked = false;
+    bool rest = false;
     for (int s = 0, w = 64; s < 64;) {
         const bool act = have && lane >= s && lane < s + w;
         if (__ballot(act)) {
@@ -162,22 +180,25 @@ __global__ __launch_bounds__(64) void points_list_kernel(BvhView B, const double
                     out[i] = in_envelope_cert(W, lst, cert, nl, mk, p, F, eps2, hl, sure) ? 0 : 1;
                 }
                 wave_sync();  // the list's last reads
-            } else if (w > kListSplit) {
+            } else if (w > kListSplit && halves_help(lo, hi, kHalvePoints * 2.0 * pad)) {
                 w /= 2;
                 continue;
             } else {
-                walked = true;
-                if (act) {
-                    int hint = -1;
-                    Stats st;
-                    out[i] = in_envelope<F32, false>(W, p, eps2, T, sqrtT, hint, st) ? 0 : 1;
-                }
+                rest = rest || act;
             }
         }
         s += w;
         w = s & -s;
     }
-    if (lstat && lane == 0) atomicAdd(lstat + (walked ? 1 : 0), 1ull);
+    if (rest) {
+        int hint = -1;
+        Stats st;
+        out[i] = in_envelope<F32, false>(W, p, eps2, T, sqrtT, hint, st) ? 0 : 1;
+    }
+    if (lstat) {
+        const bool any = __ballot(rest) != 0ull;
+        if (lane == 0) atomicAdd(lstat + (any ? 1 : 0), 1ull);
+    }
 }
 
 // Triangles the degeneracy filter cannot settle are queued (pending[],
@@ -301,10 +322,11 @@ __device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double ep
 // rounds of collect_facets, the rows through LDS, the split waves, the short
 // blocks and the open triangles on their own lanes; the VALU is busy for some
 // 40 % of it, the rest waits for the list's chain of reads.
-template <int CAP>
+template <bool F32, int CAP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void faces_list_kernel(
-    BvhView B, const double* __restrict__ tri9, int64_t n, double eps2, double d, double T_, double sqrtT, uint8_t* __restrict__ out, unsigned* n_pending, int64_t* pending,
-    const int32_t* __restrict__ order, unsigned long long* lstat)
+    BvhView B, const double* __restrict__ tri9, int64_t n, double eps2, double d, double T_, double sqrtT,
+    uint8_t* __restrict__ out, unsigned* n_pending, int64_t* pending, const int32_t* __restrict__ order,
+    unsigned long long* lstat)
 {
     constexpr int kWaveBytes = CAP * kCertEntryBytes;
     static_assert(CAP <= 128, "two list-mask words");
@@ -351,9 +373,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
     }
     // The lanes [s, s + w) at a time: all 64, unless their facets do not fit the
     // list -- the Morton order jumps inside the wave, say -- then its halves, down
-    // to kListSplit lanes, which walk the tree.  (Whole waves walking it, 5.8 %
-    // of them, ran on alone for half of the kernel's time.)
-    bool walked = false;
+    // to kListSplit lanes; the lanes whose facets do not fit then walk the tree,
+    // all at once at the end.  (Whole waves walking it, 5.8 % of them, ran on
+    // alone for half of the kernel's time.  Each last split walking it by itself
+    // before the next took 7.7 ms for 1 M triangles whose envelope is three facets
+    // wide, this 2.9; a kernel of its own for the lanes left, after this one,
+    // costs the ordinary batch its tail: 3 M triangles 1386 -> 1646 us.)
+    bool rest = false;
     for (int s = 0, w = 64; s < 64;) {
         WaveFace U = T;
         U.act = T.act && lane >= s && lane < s + w;
@@ -401,20 +427,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                 const bool o = faces_wave_listed(W, U, eps2, d, lst, cert, nl, F);
                 if (U.act) out[i] = o ? 1 : 0;
                 wave_sync();  // the list's last reads
-            } else if (w > kListSplit) {
-                w /= 2;
-                continue;
             } else {
-                // (left to the exact pass: 1551 -> 1685 us)
-                walked = true;
-                Stats st;
-                if (U.act) out[i] = face_out_sampled<true, false>(W, T.t9, eps2, d, T_, sqrtT, st) ? 1 : 0;
+                bool halve = w > kListSplit;
+                if (halve) {
+                    double one = U.act ? fmax(h3.x - l3.x, fmax(h3.y - l3.y, h3.z - l3.z)) : 0.0;
+                    for (int off = 32; off > 0; off >>= 1) one = fmax(one, __shfl_xor(one, off, 64));
+                    halve = halves_help(lo, hi, kHalveFaces * (one + 2.0 * pad));
+                }
+                if (halve) {
+                    w /= 2;
+                    continue;
+                }
+                rest = rest || U.act;
             }
         }
         s += w;
         w = s & -s;
     }
-    if (lstat && lane == 0) atomicAdd(lstat + (walked ? 1 : 0), 1ull);
+    if (rest) {
+        Stats st;
+        out[i] = face_out_sampled<F32, false>(W, T.t9, eps2, d, T_, sqrtT, st) ? 1 : 0;
+    }
+    if (lstat) {
+        const bool any = __ballot(rest) != 0ull;
+        if (lane == 0) atomicAdd(lstat + (any ? 1 : 0), 1ull);
+    }
 }
 
 // A wave per triangle, its samples spread over the lanes (face_out_wave): for
@@ -518,11 +555,16 @@ constexpr int64_t kWaveMax = 1 << 16;
 // which a wave's 64 triangles (about 64 / density facets apart) fit it whole or
 // in halves.  Measured against faces_kernel: 800 k triangles on 246 k facets
 // (3.2 a facet) 1629 -> 1027 us with the lists, 200 k on 512 k (0.4) 1082 ->
-// 2153, so sparser batches keep faces_kernel.
+// 2153, so sparser batches keep faces_kernel.  So do wide envelopes (reach_wide),
+// and below kWideDensity queries a facet those half as wide: eps two facets,
+// 2 M triangles (8 a facet) 4156 us without lists and 4356 with them; eps one
+// facet, 560 k (2.3) 1372 and 1779, 2 M (8) 3509 and 3478.
 constexpr int kFaceListCap = 80;
-constexpr int64_t kFaceListDensity = 2;
+constexpr int64_t kFaceListDensity = 2, kWideDensity = 8;
 // the same for points_list_kernel: 1 M points on 246 k facets (4 a facet) 593
-// -> 576 us, 4 M on 72 k (56) 980 -> 829, but 300 k on 512 k (0.6) 418 -> 822
+// -> 576 us, 4 M on 72 k (56) 980 -> 829, but 300 k on 512 k (0.6) 418 -> 822;
+// eps three facets, 1 M points (4 a facet) 1562 us without lists and 1774 with
+// them, eps two facets, 3 M (12) 3033 and 1849
 constexpr int kPointListCap = 64;
 constexpr int64_t kPointListDensity = 2;
 
@@ -877,7 +919,9 @@ int twg_envelope_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_
     double T = bvh_prune_threshold(B, eps2), sT = std::sqrt(T);
     dim3 g(grid_for(n)), b(kBlock);
     BvhView v = bvh_view(B);
-    const bool group = !stats && (n < kSortMin || (n < kPointGroupMax && n < kPointGroupDensity * B->nf));
+    const bool wide = reach_wide(B, 2.0 * sT);
+    const bool group = !stats && (n < kSortMin || (n < kPointGroupMax && n < kPointGroupDensity * B->nf)) &&
+                       (n < kPointGroupWide || !wide);
     const int32_t* order = nullptr;
     if (n >= kSortMin && !group)
         if (int r = morton_order(ctx, 1, p3, n, 3, B, &order)) return r;
@@ -885,7 +929,7 @@ int twg_envelope_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_
         const dim3 gg(grid_for(n * kPointGroup));
         if (precision == TWG_FP64) hipLaunchKernelGGL(points_group_kernel<false>, gg, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out);
         else hipLaunchKernelGGL(points_group_kernel<true>, gg, b, 0, ctx->cur, v, p3, n, eps2, T, sT, out);
-    } else if (order && !stats && n >= kPointListDensity * B->nf) {
+    } else if (order && !stats && n >= (wide ? kWideDensity : kPointListDensity) * B->nf) {
         if (precision == TWG_FP64)
             hipLaunchKernelGGL((points_list_kernel<false, kPointListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, p3, n, eps2, T, sT, out, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
         else
@@ -935,9 +979,12 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
         if (int r = morton_order(ctx, 1, tri9, n, 9, B, &order)) return r;
     hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, ctx->cur, n_pending);
     TWG_LAUNCHED();
-    if (order && !stats && n >= kFaceListDensity * B->nf) {
-        // (the list's boxes, and the few tree walks', are the FP32 ones in either precision)
-        hipLaunchKernelGGL(faces_list_kernel<kFaceListCap>, dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
+    const bool wide = reach_wide(B, (n < kWideDensity * B->nf ? 4.0 : 2.0) * sT);
+    if (order && !stats && !wide && n >= kFaceListDensity * B->nf) {
+        if (precision == TWG_FP64)
+            hipLaunchKernelGGL((faces_list_kernel<false, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
+        else
+            hipLaunchKernelGGL((faces_list_kernel<true, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
     } else if (precision == TWG_FP64) {
         if (stats) hipLaunchKernelGGL((faces_kernel<false, true>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, stats, n_pending, pending, order);
         else hipLaunchKernelGGL((faces_kernel<false, false>), g, b, 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, stats, n_pending, pending, order);

@@ -38,7 +38,7 @@ static_assert(sizeof(BvhNode64) == 64, "node64");
 static_assert(sizeof(BvhNode32) == 32, "node32");
 
 // How the facets crowd, from their 63-bit Morton codes: the dispatch of query
-// batches reads it (morton_bits); results never depend on it
+// batches reads it (morton_bits, reach_wide); results never depend on it
 constexpr int kCrowdLevels = 22;
 constexpr int kCrowd[2] = {32, 64};
 
@@ -1359,6 +1359,20 @@ inline BvhView no_bvh()
 {
     BvhView v = {nullptr, nullptr, nullptr, 0, 0};
     return v;
+}
+
+// Whether a box of side `reach` about a facet holds more than some 24 facets
+// (16 to 32: kCrowd at the level whose cells are up to twice as wide) for a
+// quarter of them
+inline bool reach_wide(const twg_bvh* b, double reach)
+{
+    int l = 0;
+    double s = b->side;
+    while (l + 1 < kCrowdLevels && 0.5 * s >= reach) {
+        s *= 0.5;
+        ++l;
+    }
+    return 4 * b->crowded[s * s >= 2.0 * reach * reach][l] > b->nf;
 }
 
 inline double bvh_prune_threshold(const twg_bvh* b, double eps2)
