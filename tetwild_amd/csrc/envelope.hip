@@ -556,7 +556,7 @@ constexpr int64_t kWaveMax = 1 << 16;
 // in halves.  Measured against faces_kernel: 800 k triangles on 246 k facets
 // (3.2 a facet) 1629 -> 1027 us with the lists, 200 k on 512 k (0.4) 1082 ->
 // 2153, so sparser batches keep faces_kernel.  So do wide envelopes (reach_wide),
-// and below kWideDensity queries a facet those half as wide: eps two facets,
+// and below kWideDensity queries a facet those 2.5 times less wide: eps two facets,
 // 2 M triangles (8 a facet) 4156 us without lists and 4356 with them; eps one
 // facet, 560 k (2.3) 1372 and 1779, 2 M (8) 3509 and 3478.
 constexpr int kFaceListCap = 80;
@@ -979,7 +979,7 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
         if (int r = morton_order(ctx, 1, tri9, n, 9, B, &order)) return r;
     hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, ctx->cur, n_pending);
     TWG_LAUNCHED();
-    const bool wide = reach_wide(B, (n < kWideDensity * B->nf ? 4.0 : 2.0) * sT);
+    const bool wide = reach_wide(B, (n < kWideDensity * B->nf ? 5.0 : 2.0) * sT);
     if (order && !stats && !wide && n >= kFaceListDensity * B->nf) {
         if (precision == TWG_FP64)
             hipLaunchKernelGGL((faces_list_kernel<false, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);

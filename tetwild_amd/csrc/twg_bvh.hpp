@@ -40,7 +40,7 @@ static_assert(sizeof(BvhNode32) == 32, "node32");
 // How the facets crowd, from their 63-bit Morton codes: the dispatch of query
 // batches reads it (morton_bits, reach_wide); results never depend on it
 constexpr int kCrowdLevels = 22;
-constexpr int kCrowd[2] = {32, 64};
+constexpr int kCrowd[2] = {24, 48};
 
 // levels at which two codes fall into the same cell
 TWG_HD int crowd_level(uint64_t a, uint64_t b) { return a == b ? kCrowdLevels - 1 : (__builtin_clzll(a ^ b) - 1) / 3; }
@@ -1361,9 +1361,10 @@ inline BvhView no_bvh()
     return v;
 }
 
-// Whether a box of side `reach` about a facet holds more than some 24 facets
-// (16 to 32: kCrowd at the level whose cells are up to twice as wide) for a
-// quarter of them
+// Whether a quarter of the facets have more than some 36 others in a box of side
+// `reach` about them.  Read off the level whose cells are up to twice as wide,
+// with the kCrowd for its width; a cell holds about two thirds of what a box of
+// its size about a facet does, so the line lies between 24 and 48 facets.
 inline bool reach_wide(const twg_bvh* b, double reach)
 {
     int l = 0;
