@@ -105,7 +105,8 @@ static bool inside_box(const Setup& S, V3<double> p)
 
 int main()
 {
-    long n = 0, in = 0, out = 0, plain = 0, plain_sure = 0, tris = 0, runs = 0, run_samples = 0, lists = 0;
+    long n = 0, in = 0, out = 0, plain = 0, plain_sure = 0, tris = 0, runs = 0, run_samples = 0, lists = 0, past = 0, past_hint = 0,
+         ends = 0;
     for (int s = 0; s < 4000; ++s) {
         const double scale = s % 5 == 0 ? LU(1e-12, 1e9) : 1.0;
         const Setup S = setup(scale, s % 3 == 0 ? scale * LU(1, 1e9) : scale * U(0, 2));
@@ -134,31 +135,58 @@ int main()
                     plain_sure += r != 0;
                 }
             }
-        // the whole list's decision, with and without a hint and a mask word's end
+        // the whole list's decision, with and without a hint, on lists up to
+        // the masks' end: few facets hold p, on either side of position 64
+        const int lens[] = {1 + (int)(rng() % 12), 63, 64, 65, 80, 92, 128};
+        const int nl = lens[s % 7];
         struct Node { int32_t leaf, pad; };
-        std::vector<Node> L(12);
-        for (int f = 0; f < 12; ++f) L[f] = {f, -1};
+        std::vector<Node> L(nl);
+        std::vector<double> LT(9 * nl);
+        std::vector<float> LC(kCertFloats * nl);
+        for (int f = 0; f < nl; ++f) {
+            L[f] = {f, 0};
+            if (f < 12) std::memcpy(&LT[9 * f], &T[9 * f], 72);
+            else facet(S, &LT[9 * f]);
+        }
+        for (int f = 0; f < nl; ++f)  // the twelve the points lie about at places of the whole list
+            if (f < 12) {
+                const int g = (int)(rng() % nl);
+                for (int q = 0; q < 9; ++q) std::swap(LT[9 * f + q], LT[9 * g + q]);
+            }
+        for (int f = 0; f < nl; ++f) cert_write(&LC[kCertFloats * f], &LT[9 * f], S.F, S.eps2);
         BvhWalk W;
         std::memset(&W, 0, sizeof W);
-        W.tri = T.data();
+        W.tri = LT.data();
         for (int k = 0; k < 60; ++k) {
             V3<double> p = near_point(S, &T[9 * (rng() % 12)]);
             if (!inside_box(S, p)) continue;
-            bool ref = false;
+            bool ref = false, low = false, high = false;
             uint64_t mask[2] = {0, 0};
-            const int nl = 1 + (int)(rng() % 12);
             for (int f = 0; f < nl; ++f)
                 if (rng() % 8) {
-                    mask[0] |= 1ull << f;
-                    ref = ref || d2(&T[9 * f], p) <= S.eps2;
+                    mask[f / 64] |= 1ull << (f % 64);
+                    const bool holds = d2(&LT[9 * f], p) <= S.eps2;
+                    ref = ref || holds;
+                    (f < 64 ? low : high) |= holds;
                 }
             int hl = -1;
-            if (mask[0] && rng() % 2) hl = __builtin_ctzll(mask[0]);
+            if (rng() % 2) hl = (int)(rng() % nl);  // (a hint counts outside the mask too)
+            const int hint = hl;
+            ref = ref || (hint >= 0 && d2(&LT[9 * hint], p) <= S.eps2);
             bool sure = false;
-            const bool got = in_envelope_cert(W, L.data(), C.data(), nl, mask, p, S.F, S.eps2, hl, sure);
-            CHECK(got == ref, "set %d: list decision %d, FP64 %d\n", s, got, ref);
-            CHECK(!got || (hl >= 0 && d2(&T[9 * hl], p) <= S.eps2), "set %d: the facet left does not hold p\n", s);
+            const bool got = in_envelope_cert(W, L.data(), LC.data(), nl, mask, p, S.F, S.eps2, hl, sure);
+            CHECK(got == ref, "set %d: list of %d, decision %d, FP64 %d\n", s, nl, got, ref);
+            CHECK(!got || (hl >= 0 && hl < nl && d2(&LT[9 * hl], p) <= S.eps2), "set %d: the facet left does not hold p\n", s);
             ++lists;
+            past += high && !low;
+            past_hint += hint >= 64;
+            if (nl == 64) {  // the word past the list's end is not read
+                mask[1] = ~0ull;
+                int h2 = hint;
+                CHECK(in_envelope_cert(W, L.data(), LC.data(), nl, mask, p, S.F, S.eps2, h2, sure) == ref,
+                      "set %d: a list that ends a word reads past it\n", s);
+                ++ends;
+            }
         }
         if (!S.F.runs) continue;
         // triangles near the facets, their samples between certified ones
@@ -217,10 +245,10 @@ int main()
             }
         }
     }
-    printf("%ld facet decisions (%ld certified in, %ld out), %ld lists, %ld certified triangles, %ld runs (%ld "
+    printf("%ld facet decisions (%ld certified in, %ld out), %ld lists (%ld held past position 64 alone, %ld hints past it, %ld at a word's end), %ld certified triangles, %ld runs (%ld "
            "samples); ordinary facets off the limit: %ld of %ld certified\n",
-           n, in, out, lists, tris, runs, run_samples, plain_sure, plain);
-    CHECK(in > 100000 && out > 100000 && tris > 500 && runs > 5000 && lists > 50000, "too few cases\n");
+           n, in, out, lists, past, past_hint, ends, tris, runs, run_samples, plain_sure, plain);
+    CHECK(in > 100000 && out > 100000 && tris > 500 && runs > 5000 && lists > 50000 && past > 5000 && past_hint > 5000 && ends > 5000, "too few cases\n");
     CHECK(plain_sure > 0.8 * plain && plain > 10000, "certificates miss ordinary cases\n");
     printf("%ld failures\n", failures);
     return failures ? 1 : 0;

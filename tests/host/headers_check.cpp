@@ -7,12 +7,14 @@
 //   2. in_envelope -- global walker and LDS walker over the top levels, FP64
 //      and FP32 boxes -- against the brute-force minimum over all facets, on
 //      trees of 1..50k facets (the tree built by the library's own host code);
-//   3. face_out_group's block split (G lanes emulated one after another, the
+//   3. face_out_wave's block split (G lanes emulated one after another, the
 //      ballot as the OR of the lanes' step results) against face_out_sampled,
 //      and that every sample of an inside triangle is tested exactly once;
 //   4. collect_facets (one-lane group) against the facets whose boxes meet
-//      the query box, in_envelope_list on its lists against brute force, and
-//      in_envelope_masked with face_list_mask against in_envelope_list;
+//      the query box; on its lists in_envelope_cert with point_list_mask and
+//      with face_list_mask, and faces_wave_listed's decision of a whole
+//      triangle, against brute force and the tree walk, with lists past the
+//      masks' first word among them;
 //   5. nearest_facet_group (one-lane group) against nearest_facet, bit for
 //      bit, with queries above shared grid edges and vertices (ties);
 //   6. point_tri_d2 (squared distance and closest point) against the
@@ -21,6 +23,7 @@
 // Exit status 0 when every check passes.
 #include "twg_bvh.hpp"
 
+#include <algorithm>
 #include <cstdio>
 #include <cmath>
 #include <cstring>
@@ -321,7 +324,7 @@ static void check_lists(std::mt19937_64& rng)
 {
     std::uniform_real_distribution<double> U(0, 1);
     std::vector<unsigned char> cache(kTreeCacheBytes);
-    long lists = 0, points = 0, overflow = 0, masked = 0, listed_faces = 0;
+    long lists = 0, points = 0, overflow = 0, masked = 0, listed_faces = 0, word1 = 0, past = 0, settled = 0;
     for (int nf : {2, 3, 7, 100, 1000, 3001, 20001}) {
         Tree T;
         build(T, nf, rng, 0.02);
@@ -334,9 +337,16 @@ static void check_lists(std::mt19937_64& rng)
                 const int cap = q % 5 == 0 ? 16 : 4096;
                 std::vector<BvhNode32> lst(cap);
                 std::vector<uint32_t> fr(2 * cap);
-                const double cx = U(rng), cy = U(rng), s = (q % 3 == 0) ? 0.3 : 0.04 * U(rng);
+                const bool hundred = q % 4 == 1 && nf >= 1000;
+                const double s = hundred ? sqrt(95.0 / nf) - 0.04 : (q % 3 == 0) ? 0.3 : 0.04 * U(rng);
+                const double cx = U(rng) * (hundred ? 1 - s : 1), cy = U(rng) * (hundred ? 1 - s : 1);
                 double lo[3] = {cx, cy, 0.05 * sin(7 * cx) * cos(5 * cy) - 0.01};
                 double hi[3] = {cx + s * U(rng), cy + s * U(rng), lo[2] + 0.02 + 0.03 * U(rng)};
+                if (hundred) {  // about as many facets, the height of the sheet there
+                    hi[0] = cx + s;
+                    hi[1] = cy + s;
+                    hi[2] = lo[2] + 0.06;
+                }
                 const double pad = 1.0001 * sqrtT + 1e-9;
                 for (int k = 0; k < 3; ++k) {
                     lo[k] -= pad;
@@ -369,89 +379,100 @@ static void check_lists(std::mt19937_64& rng)
                 for (int f = 0; f < nf; ++f) ok = ok && (!exact[f] || in_list[f]);
                 CHECK(ok, "lists: %d facets, mode %d, query %d: list differs from the box query\n", nf, mode, q);
                 lists++;
-                // half the lists record edge neighbours for in_envelope_list's
-                // second try (any list positions: a facet within eps decides
-                // "in" whichever facet it is, so arbitrary ones must not change
-                // a decision)
-                if (q % 2 == 1 && n < 256)
-                    for (int j = 0; j < n; ++j) {
-                        uint32_t pk = 0xff000000u;
-                        for (int k = 0; k < 3; ++k) {
-                            const uint32_t v = rng() % 4 == 0 ? 0xffu : (uint32_t)(rng() % n);
-                            pk |= v << (8 * k);
-                        }
-                        lst[j].pad = (int32_t)pk;
-                    }
+                if (n > 128) continue;  // (no kernel's list is longer)
+                word1 += n > 64;
+                const double d = 0.004;
+                double amax = 0.0;
+                for (int k = 0; k < 3; ++k) amax = std::max({amax, fabs(lo[k] + pad), fabs(hi[k] - pad)});
+                const CertFrame F = cert_frame(lo, hi, amax, eps2, d);
+                std::vector<float> cert(kCertFloats * (size_t)std::max(n, 1));
+                cert_list<1>(W, lst.data(), cert.data(), n, F, eps2, 0);
                 // points of the unpadded box against brute force
-                std::vector<double> tri(9 * (size_t)std::max(n, 1));
-                for (int j = 0; j < n; ++j)
-                    for (int k = 0; k < 9; ++k) tri[9 * j + k] = T.tri[9 * (size_t)lst[j].leaf + k];
+                auto in_box = [&](V3<double>& p) {
+                    double* pc[3] = {&p.x, &p.y, &p.z};
+                    for (int k = 0; k < 3; ++k) *pc[k] = lo[k] + pad + (hi[k] - lo[k] - 2 * pad) * U(rng);
+                };
+                // ... about a listed facet, from the last one down
+                auto near_facet = [&](V3<double>& p, int r) {
+                    in_box(p);
+                    if (n == 0) return;
+                    const double* t = &T.tri[9 * (size_t)lst[(n - 1 - r % n)].leaf];
+                    double* pc[3] = {&p.x, &p.y, &p.z};
+                    for (int k = 0; k < 3; ++k) {
+                        const double c = (t[k] + t[3 + k] + t[6 + k]) / 3 + eps * (2 * U(rng) - 1);
+                        *pc[k] = std::min(std::max(c, lo[k] + pad), hi[k] - pad);
+                    }
+                };
+                auto brute = [&](V3<double> p) {
+                    double best = INFINITY;
+                    for (int f = 0; f < nf; ++f) best = std::min(best, facet_d2(W, f, p));
+                    return best <= eps2;
+                };
+                uint64_t mk[2];
+                bool sure;
                 int hl = -1;
                 for (int r = 0; r < 16; ++r) {
                     V3<double> p;
-                    double* pc[3] = {&p.x, &p.y, &p.z};
-                    for (int k = 0; k < 3; ++k) *pc[k] = lo[k] + pad + (hi[k] - lo[k] - 2 * pad) * U(rng);
-                    double best = INFINITY;
-                    for (int f = 0; f < nf; ++f) best = std::min(best, facet_d2(W, f, p));
-                    const bool got = q % 2 == 1
-                                         ? in_envelope_list<true>(lst.data(), tri.data(), n, p, eps2, sqrtT, hl)
-                                         : in_envelope_list(lst.data(), tri.data(), n, p, eps2, sqrtT, hl);
-                    CHECK(got == (best <= eps2), "lists: %d facets, mode %d, query %d, point %d\n", nf, mode, q, r);
+                    if (r % 2) near_facet(p, r);
+                    else in_box(p);
+                    point_list_mask(lst.data(), n, p, sqrtT, mk);
+                    const bool got = in_envelope_cert(W, lst.data(), cert.data(), n, mk, p, F, eps2, hl, sure);
+                    CHECK(got == brute(p) && (!got || facet_d2(W, lst[hl].leaf, p) <= eps2),
+                          "lists: %d facets, mode %d, query %d, point %d\n", nf, mode, q, r);
+                    past += got && hl >= 64;
                     if (r % 7 == 0) hl = -1;
                     points++;
                 }
-                // a face inside the box, its samples tested through the face's
-                // list mask: the decision and the facet left in the hint are
-                // in_envelope_list's (the mask leaves out only facets farther
-                // than sqrt(T) from the face)
-                if (n >= 0 && n <= 128) {
-                    V3<double> fv[3];
-                    for (int j = 0; j < 3; ++j) {
-                        double* pc[3] = {&fv[j].x, &fv[j].y, &fv[j].z};
-                        for (int k = 0; k < 3; ++k) *pc[k] = lo[k] + pad + (hi[k] - lo[k] - 2 * pad) * U(rng);
+                // triangles of the box: every sample through the triangle's
+                // list mask, and the decision of the whole
+                for (int r = 0; r < 4; ++r) {
+                    V3<double> v[3];
+                    near_facet(v[0], r);
+                    for (int j = 1; j < 3; ++j) {
+                        in_box(v[j]);
+                        if (r) v[j] = v[0] + mulv(v[j] - v[0], r == 1 ? 0.2 : 0.03);
                     }
-                    uint64_t mk[2];
-                    face_list_mask(lst.data(), n, fv[0], fv[1], fv[2], sqrtT, mk);
-                    int hm = -1, hu = -1;
-                    const bool nbr = q % 2 == 1;  // these lists carry neighbour positions
-                    for_each_sample(fv[0], fv[1], fv[2], 0.004, [&](V3<double> p) {
-                        // (the queries without neighbours take the four-at-a-time box reads)
-                        const bool gm =
-                            nbr ? in_envelope_masked<true>(lst.data(), tri.data(), n, mk, p, eps2, sqrtT, hm)
-                                : in_envelope_masked<false, true>(lst.data(), tri.data(), n, mk, p, eps2, sqrtT,
-                                                                  hm);
-                        const bool gu =
-                            nbr ? in_envelope_list<true>(lst.data(), tri.data(), n, p, eps2, sqrtT, hu)
-                                : in_envelope_list(lst.data(), tri.data(), n, p, eps2, sqrtT, hu);
-                        double best = INFINITY;
-                        for (int f = 0; f < nf; ++f) best = std::min(best, facet_d2(W, f, p));
-                        CHECK(gm == gu && hm == hu && gm == (best <= eps2),
-                              "masked lists: %d facets, mode %d, query %d\n", nf, mode, q);
-                        masked++;
-                        return false;
-                    });
-                    // the whole decision of face_out_listed (masked scans)
-                    // against the per-sample tree walk
                     double t9[9];
                     for (int j = 0; j < 3; ++j) {
-                        t9[3 * j] = fv[j].x;
-                        t9[3 * j + 1] = fv[j].y;
-                        t9[3 * j + 2] = fv[j].z;
+                        t9[3 * j] = v[j].x;
+                        t9[3 * j + 1] = v[j].y;
+                        t9[3 * j + 2] = v[j].z;
                     }
+                    WaveFace G;
+                    G.t9 = t9;
+                    G.act = wave_face_first(v[0], v[1], v[2], d, G.first);
+                    face_mask_box(v[0], v[1], v[2], sqrtT, G.mlo, G.mhi);
+                    for (int j = 0; j < 3; ++j) G.q[j] = cert_local(F, v[(G.first + j) % 3]);
+                    face_list_mask(lst.data(), n, G.mlo, G.mhi, mk);
+                    int hm = -1;
+                    bool ref = false, first = true;
+                    for_each_sample(v[0], v[1], v[2], d, [&](V3<double> p) {
+                        if (first)
+                            CHECK(!memcmp(&p, &v[G.first], sizeof p), "first corner: query %d, triangle %d\n", q, r);
+                        first = false;
+                        const bool got = in_envelope_cert(W, lst.data(), cert.data(), n, mk, p, F, eps2, hm, sure);
+                        const bool in = brute(p);
+                        CHECK(got == in, "masked lists: %d facets, mode %d, query %d\n", nf, mode, q);
+                        ref = ref || !in;
+                        masked++;
+                        return masked % 64 == 0;  // (brute force is slow: some triangles end early)
+                    });
                     Stats st;
-                    const bool lo_ = face_out_listed<false>(W, t9, eps2, 0.004, Tt, sqrtT, lst.data(),
-                                                           tri.data(), n);
-                    const bool ref =
-                        face_out_sampled<false, false>(walk(T.view), t9, eps2, 0.004, Tt, sqrtT, st);
-                    CHECK(lo_ == ref, "face_out_listed: %d facets, mode %d, query %d\n", nf, mode, q);
+                    const bool walk_out =
+                        face_out_sampled<false, false>(walk(T.view), t9, eps2, d, Tt, sqrtT, st);
+                    CHECK(!ref || walk_out, "walk: %d facets, mode %d, query %d\n", nf, mode, q);
+                    const bool o = faces_wave_listed(W, G, eps2, d, lst.data(), cert.data(), n, F);
+                    CHECK(o == walk_out, "whole triangle: %d facets, mode %d, query %d\n", nf, mode, q);
                     listed_faces++;
+                    settled += !o;
                 }
             }
         }
     }
+    CHECK(word1 >= 100 && past >= 100 && settled >= 500 && settled < listed_faces, "lists: too few cases\n");
     printf("facet lists: %ld lists (%ld overflowed), %ld points against brute force, %ld face samples "
-           "through face masks, %ld face_out_listed decisions\n", lists, overflow, points, masked,
-           listed_faces);
+           "through face masks, %ld whole triangles (%ld in), %ld lists past 64 facets, %ld points held past them\n",
+           lists, overflow, points, masked, listed_faces, settled, word1, past);
 }
 
 // a grid of n x n squares over [0, 1]^2, each split into two triangles, on a

@@ -229,87 +229,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     if (STATS) flush_stats(st, stats);
 }
 
-// What a lane keeps of its triangle while the wave's list is made: its corners
-// in the list's frame, the one SampleGen::init rotates to the front first, and
-// the box face_list_mask compares the list with.  (The corners themselves,
-// 18 registers, are read again by the few lanes that need them.)
-struct WaveFace {
-    bool act;
-    int first;
-    const double* t9;
-    V3<float> q[3];
-    float mlo[3], mhi[3];
-};
-
-// face_out_sampled for the wave's triangles at once (a list of nl <= 128
-// facets, nl >= 0, with its certificates).  Every lane scans the facets near
-// its triangle for one that holds its first corner: none, and the triangle is
-// out; one that certifies all three corners, and it is in.  The few triangles
-// still open -- they straddle facets, or reach the limit -- are sampled by
-// their lanes, which pass over the samples between two that one facet
-// certifies on a row.  (Spreading the open triangles' samples over the wave
-// takes two more samplers per lane and their registers: 3 M triangles of 6-11
-// samples 1568 us against 1551, of ~20 samples 3205 against 3028.)  Returns the
-// lane's decision.
-__device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double eps2, double d,
-                                  LdsNode32W* lst, LdsF32* cert, int nl, const CertFrame& F)
-{
-    bool out = T.act, open_lane = false;
-    uint64_t mk[2] = {0ull, 0ull};
-    int hl = -1;
-    const double* t9 = T.t9;
-    if (T.act) {
-        face_list_mask(lst, nl, T.mlo, T.mhi, mk);
-        uint64_t unsure[2] = {0ull, 0ull};
-        bool all = false;
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            uint64_t mm = 64 * w < nl ? mk[w] : 0ull;
-            while (mm && !all) {
-                const int i = 64 * w + __builtin_ctzll(mm);
-                LdsF32* ci = cert + kCertFloats * i;
-                const int r = cert_class(ci, T.q[0], F);
-                if (r == 0) unsure[w] |= mm & (0ull - mm);
-                mm &= mm - 1;
-                if (r > 0) {
-                    hl = i;
-                    all = F.runs && cert_class(ci, T.q[1], F) > 0 && cert_class(ci, T.q[2], F) > 0;
-                }
-            }
-        }
-        if (hl < 0 && (unsure[0] | unsure[1])) {
-            const V3<double> p0 = ld3(t9 + 3 * T.first);
-#pragma unroll
-            for (int w = 0; w < 2; ++w)
-                for (uint64_t mm = unsure[w]; mm && hl < 0; mm &= mm - 1) {
-                    const int i = 64 * w + __builtin_ctzll(mm);
-                    if (facet_d2(W, lst[i].leaf, p0) <= eps2) hl = i;
-                }
-        }
-        out = hl < 0;
-        open_lane = hl >= 0 && !all;
-    }
-    if (open_lane) {
-        SampleGen g;
-        g.init(ld3(t9), ld3(t9 + 3), ld3(t9 + 6), d);
-        V3<double> s;
-        g.next(s);  // the first corner
-        while (g.next(s)) {
-            bool sure;
-            if (!in_envelope_cert(W, lst, cert, nl, mk, s, F, eps2, hl, sure)) {
-                out = true;
-                break;
-            }
-            if (sure && F.runs) {
-                const int64_t left = g.run_left(INT64_MAX);
-                if (left > 0 && cert_class(cert + kCertFloats * hl, cert_local(F, g.run_at(left)), F) > 0)
-                    g.k += (int)left;
-            }
-        }
-    }
-    return out;
-}
-
 // One triangle per lane, as faces_kernel, for batches walked in Morton
 // order: the wave's 64 consecutive triangles lie close together, so the wave
 // lists once (collect_facets, LDS) the facets whose boxes meet the box of its
@@ -364,11 +283,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
             unsigned k = atomicAdd(n_pending, 1u);
             pending[k] = i;
         } else {
-            const double l0 = len2(a - b), l1 = len2(b - c), l2 = len2(c - a);
-            const double N = __builtin_sqrt(fmax(l0, fmax(l1, l2))) / d;
-            T.act = N <= kMaxEdgeSamples;
+            T.act = wave_face_first(a, b, c, d, T.first);
             if (!T.act) out[i] = 1;
-            else if (N > 1) T.first = !(l2 < l0) && !(l2 < l1) ? 2 : (!(l1 < l0) ? 1 : 0);
         }
     }
     // The lanes [s, s + w) at a time: all 64, unless their facets do not fit the

@@ -404,7 +404,6 @@ __device__ __forceinline__ void put_lds(LdsNode32W* d, const BvhNode32& s)
         d->hi[k] = s.hi[k];
     }
     d->leaf = s.leaf;
-    d->pad = -1;  // no neighbours recorded
 }
 
 // The facets whose boxes meet the box [lo, hi], found by the G lanes of a
@@ -488,88 +487,10 @@ __device__ int collect_facets(const BvhWalk& W, const double lo[3], const double
 }
 
 typedef __attribute__((address_space(3))) double LdsF64;
-typedef __attribute__((address_space(3))) const double LdsF64c;
 
-// facet_d2 of a triangle held in LDS (9 doubles): the same computation on
-// the same values
-__device__ __forceinline__ double tri_d2(LdsF64c* t, V3<double> p)
-{
-    V3<double> cp;
-    return point_tri_d2<double, false>(p, mk3(t[0], t[1], t[2]), mk3(t[3], t[4], t[5]),
-                                       mk3(t[6], t[7], t[8]), cp);
-}
-
-// (in_envelope_list, face_list_mask's in_envelope_masked and face_out_listed are
-// the plain forms of in_envelope_cert's decision, without certificates; the
-// host checks reach them, no kernel does.)
-// in_envelope's decision for a point p of the box that a collect_facets list
-// was made for, with that box padded by at least sqrt(T) beyond every point
-// tested (then the list holds every facet the tree walk could accept): the
-// facet at list position hl first (the one that held the previous point, -1:
-// none), then the others, 64 positions at a time: the FP32 box tests of the
-// window first, into a bit mask, then the triangles of the boxes that pass.
-// (Box tests and triangle distances interleaved would make a wave pay a
-// triangle distance at every position where some lane's box passes.)  tri
-// holds the listed facets' triangles, 9 doubles per position.  On a hit hl
-// becomes the facet's position.
-template <bool NB = false>
-__device__ __forceinline__ bool in_envelope_list(LdsNode32W* lst, LdsF64c* tri, int nl,
-                                                 V3<double> p, double eps2, double sqrtT, int& hl)
-{
-    int nb[3] = {-1, -1, -1};
-    if (hl >= 0) {
-        if (tri_d2(tri + 9 * hl, p) <= eps2) return true;
-        // a sample that left its predecessor's facet is usually within eps of
-        // one of that facet's edge neighbours (NB: the list records them)
-        const uint32_t pk = NB ? (uint32_t)lst[hl].pad : 0xffffffffu;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const uint32_t q = (pk >> (8 * k)) & 0xffu;
-            if (q != 0xffu) {
-                if (tri_d2(tri + 9 * q, p) <= eps2) {
-                    hl = (int)q;
-                    return true;
-                }
-                nb[k] = (int)q;
-            }
-        }
-    }
-    const V3<float> pf = mk3((float)p.x, (float)p.y, (float)p.z);
-    const float Tf = f32_threshold(p, sqrtT);
-    for (int base = 0; base < nl; base += 64) {
-        const int n = nl - base < 64 ? nl - base : 64;
-        uint64_t m = 0;
-        for (int k0 = 0; k0 < n; k0 += 8) {  // eight records read before their tests
-            BvhNode32 e[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (k0 + u < n) e[u] = from_lds(lst + base + k0 + u);
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (k0 + u < n) m |= (uint64_t)(box_d2(pf, e[u].lo, e[u].hi) <= Tf) << (k0 + u);
-        }
-        if (hl >= base && hl < base + n) m &= ~(1ull << (hl - base));
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (nb[k] >= base && nb[k] < base + n) m &= ~(1ull << (nb[k] - base));
-        while (m) {
-            const int i = base + __builtin_ctzll(m);
-            m &= m - 1;
-            if (tri_d2(tri + 9 * i, p) <= eps2) {
-                hl = i;
-                return true;
-            }
-        }
-    }
-    return false;
-}
-
-// The positions of a collect_facets list (nl <= 128 entries) whose FP32 boxes
-// meet the box of triangle (a, b, c) padded as the list's own box is (by
-// 1.0001 sqrt(T) + 1e-9 max |coordinate|): every facet within sqrt(T) of a
-// point of the triangle -- or of a sample of it, up to its rounding -- is at
-// a set position.  mk: two 64-bit words.
-// the FP32 box face_list_mask compares the list's boxes with
+// the FP32 box face_list_mask compares a list's boxes with: that of triangle
+// (a, b, c) padded as the list's own box is (by 1.0001 sqrt(T) + 1e-9 max
+// |coordinate|)
 __device__ __forceinline__ void face_mask_box(V3<double> a, V3<double> b, V3<double> c,
                                               double sqrtT, float lof[3], float hif[3])
 {
@@ -591,6 +512,10 @@ __device__ __forceinline__ void face_mask_box(V3<double> a, V3<double> b, V3<dou
     }
 }
 
+// The positions of a collect_facets list (nl <= 128 entries) whose FP32 boxes
+// meet a triangle's face_mask_box: every facet within sqrt(T) of a point of the
+// triangle -- or of a sample of it, up to its rounding -- is at a set position.
+// mk: two 64-bit words.
 template <class L>
 __device__ __forceinline__ void face_list_mask(L lst, int nl, const float lof[3], const float hif[3],
                                                uint64_t mk[2])
@@ -619,96 +544,6 @@ __device__ __forceinline__ void face_list_mask(L lst, int nl, const float lof[3]
     mk[0] = w[0];
     mk[1] = w[1];
 }
-template <class L>
-__device__ __forceinline__ void face_list_mask(L lst, int nl, V3<double> a, V3<double> b,
-                                               V3<double> c, double sqrtT, uint64_t mk[2])
-{
-    float lof[3], hif[3];
-    face_mask_box(a, b, c, sqrtT, lof, hif);
-    face_list_mask(lst, nl, lof, hif, mk);
-}
-
-// in_envelope_list over the list positions set in mask (two 64-bit words;
-// lists of at most 128 entries), for a p whose caller guarantees that no
-// facet at an unset position lies within sqrt(T) of p: the facet at hl
-// first, then the set positions' FP32 box tests, then the triangles of the
-// boxes that pass, in ascending position as in_envelope_list.  Every facet
-// that could hold p is at a set position, so the decision and the facet left
-// in hl are in_envelope_list's.  BATCH: the set positions' boxes are read
-// four at a time before their tests (one LDS round trip per four; the
-// smoothing kernels gain from it, the envelope list kernel, short of
-// registers, loses).
-template <bool NB = false, bool BATCH = false, class M>
-__device__ __forceinline__ bool in_envelope_masked(LdsNode32W* lst, LdsF64c* tri, int nl, M mask,
-                                                   V3<double> p, double eps2, double sqrtT, int& hl)
-{
-    int nb[3] = {-1, -1, -1};
-    if (hl >= 0) {
-        if (tri_d2(tri + 9 * hl, p) <= eps2) return true;
-        // NB: the facet's edge neighbours next, as in_envelope_list<true>
-        const uint32_t pk = NB ? (uint32_t)lst[hl].pad : 0xffffffffu;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const uint32_t q = (pk >> (8 * k)) & 0xffu;
-            if (q != 0xffu) {
-                if (tri_d2(tri + 9 * q, p) <= eps2) {
-                    hl = (int)q;
-                    return true;
-                }
-                nb[k] = (int)q;
-            }
-        }
-    }
-    const V3<float> pf = mk3((float)p.x, (float)p.y, (float)p.z);
-    const float Tf = f32_threshold(p, sqrtT);
-    for (int w = 0; w < 2 && 64 * w < nl; ++w) {
-        uint64_t mm = mask[w];
-        if (hl >= 64 * w && hl < 64 * w + 64) mm &= ~(1ull << (hl - 64 * w));
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (nb[k] >= 64 * w && nb[k] < 64 * w + 64) mm &= ~(1ull << (nb[k] - 64 * w));
-        uint64_t m = 0;
-        while (!BATCH && mm) {
-            const int b = __builtin_ctzll(mm);
-            mm &= mm - 1;
-            const BvhNode32 e = from_lds(lst + 64 * w + b);
-            if (box_d2(pf, e.lo, e.hi) <= Tf) m |= 1ull << b;
-        }
-        while (BATCH && mm) {
-            // four set positions at a time, their boxes read before their
-            // tests (past the last set bit, the first is read again)
-            int bq[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                bq[u] = mm ? __builtin_ctzll(mm) : -1;
-                mm &= mm - 1;
-            }
-            float lo[4][3], hi[4][3];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const LdsNode32W* e = lst + 64 * w + (bq[u] >= 0 ? bq[u] : bq[0]);
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    lo[u][k] = e->lo[k];
-                    hi[u][k] = e->hi[k];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (bq[u] >= 0 && box_d2(pf, lo[u], hi[u]) <= Tf) m |= 1ull << bq[u];
-        }
-        while (m) {
-            const int i = 64 * w + __builtin_ctzll(m);
-            m &= m - 1;
-            if (tri_d2(tri + 9 * i, p) <= eps2) {
-                hl = i;
-                return true;
-            }
-        }
-    }
-    return false;
-}
-
 // The positions of a collect_facets list (nl <= 128 entries) whose FP32 boxes
 // can hold a facet within sqrt(T) of p (the tree walk's box test)
 template <class L>
@@ -893,11 +728,14 @@ __device__ __forceinline__ int cert_class(P c, V3<float> q, const CertFrame& F)
     return r;
 }
 
-// in_envelope_list / in_envelope_masked with the certificates: the facet at
-// hl first, then the positions set in mask, in
-// ascending order; positions no certificate decides go to FP64 at the end.
-// The decision is in_envelope_masked's; hl may become another facet that
-// holds p.  sure: set when the facet left in hl is certified.
+// in_envelope's decision for a point p of the box that a collect_facets list
+// was made for, with that box padded by at least sqrt(T) beyond every point
+// tested (then the list holds every facet the tree walk could accept) and every
+// facet within sqrt(T) of p at a position set in mask (two 64-bit words, lists of
+// at most 128 facets): the facet at list position hl first (the one that held the
+// previous point, -1: none), then the positions set in mask, in ascending order;
+// positions no certificate decides go to FP64 at the end.  On a hit hl becomes
+// the position of a facet that holds p.  sure: set when that is certified.
 template <class L, class P, class M>
 __device__ __forceinline__ bool in_envelope_cert(const BvhWalk& W, L lst, P cert, int nl, M mask,
                                                  V3<double> p, const CertFrame& F, double eps2,
@@ -1171,35 +1009,97 @@ __device__ bool face_out_sampled(const BvhWalk& B, const double* t9, double eps2
     });
 }
 
-// face_out_sampled's decision with the facets from a collect_facets list
-// (lst, tri; see in_envelope_list) whose box holds the triangle padded by
-// more than sqrt(T): every sample lies in that box, so the list holds every
-// facet the tree walk could accept.  nl < 0: the tree walk.
-template <bool F32>
-__device__ bool face_out_listed(const BvhWalk& B, const double* t9, double eps2, double d,
-                                double T, double sqrtT, LdsNode32W* lst, LdsF64c* tri, int nl)
+// What a lane keeps of its triangle while the wave's list is made: its corners
+// in the list's frame, the one SampleGen::init rotates to the front first, and
+// the box face_list_mask compares the list with.  (The corners themselves,
+// 18 registers, are read again by the few lanes that need them.)
+struct WaveFace {
+    bool act;
+    int first;
+    const double* t9;
+    V3<float> q[3];
+    float mlo[3], mhi[3];
+};
+
+// the corner SampleGen::init rotates to the front; false for a triangle that is
+// reported out without sampling
+__device__ __forceinline__ bool wave_face_first(V3<double> a, V3<double> b, V3<double> c, double d, int& first)
 {
-    if (nl < 0) {
-        Stats st;
-        return face_out_sampled<F32, false>(B, t9, eps2, d, T, sqrtT, st);
-    }
-    const V3<double> a = ld3(t9), b = ld3(t9 + 3), c = ld3(t9 + 6);
-    {
-        double l = fmax(len2(a - b), fmax(len2(b - c), len2(c - a)));
-        if (!(__builtin_sqrt(l) / d <= kMaxEdgeSamples)) return true;
-    }
+    const double l0 = len2(a - b), l1 = len2(b - c), l2 = len2(c - a);
+    const double N = __builtin_sqrt(fmax(l0, fmax(l1, l2))) / d;
+    first = 0;
+    if (!(N <= kMaxEdgeSamples)) return false;
+    if (N > 1) first = !(l2 < l0) && !(l2 < l1) ? 2 : (!(l1 < l0) ? 1 : 0);
+    return true;
+}
+
+// face_out_sampled for the wave's triangles at once (a list of nl <= 128
+// facets, nl >= 0, with its certificates).  Every lane scans the facets near
+// its triangle for one that holds its first corner: none, and the triangle is
+// out; one that certifies all three corners, and it is in.  The few triangles
+// still open -- they straddle facets, or reach the limit -- are sampled by
+// their lanes, which pass over the samples between two that one facet
+// certifies on a row.  (Spreading the open triangles' samples over the wave
+// takes two more samplers per lane and their registers: 3 M triangles of 6-11
+// samples 1568 us against 1551, of ~20 samples 3205 against 3028.)  Returns the
+// lane's decision.
+__device__ bool faces_wave_listed(const BvhWalk& W, const WaveFace& T, double eps2, double d,
+                                  LdsNode32W* lst, LdsF32* cert, int nl, const CertFrame& F)
+{
+    bool out = T.act, open_lane = false;
+    uint64_t mk[2] = {0ull, 0ull};
     int hl = -1;
-    if (nl <= 128) {
-        // only the listed facets that can lie near this triangle
-        uint64_t mk[2];
-        face_list_mask(lst, nl, a, b, c, sqrtT, mk);
-        return for_each_sample(a, b, c, d, [&](V3<double> s) {
-            return !in_envelope_masked<true>(lst, tri, nl, mk, s, eps2, sqrtT, hl);
-        });
+    const double* t9 = T.t9;
+    if (T.act) {
+        face_list_mask(lst, nl, T.mlo, T.mhi, mk);
+        uint64_t unsure[2] = {0ull, 0ull};
+        bool all = false;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            uint64_t mm = 64 * w < nl ? mk[w] : 0ull;
+            while (mm && !all) {
+                const int i = 64 * w + __builtin_ctzll(mm);
+                LdsF32* ci = cert + kCertFloats * i;
+                const int r = cert_class(ci, T.q[0], F);
+                if (r == 0) unsure[w] |= mm & (0ull - mm);
+                mm &= mm - 1;
+                if (r > 0) {
+                    hl = i;
+                    all = F.runs && cert_class(ci, T.q[1], F) > 0 && cert_class(ci, T.q[2], F) > 0;
+                }
+            }
+        }
+        if (hl < 0 && (unsure[0] | unsure[1])) {
+            const V3<double> p0 = ld3(t9 + 3 * T.first);
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+                for (uint64_t mm = unsure[w]; mm && hl < 0; mm &= mm - 1) {
+                    const int i = 64 * w + __builtin_ctzll(mm);
+                    if (facet_d2(W, lst[i].leaf, p0) <= eps2) hl = i;
+                }
+        }
+        out = hl < 0;
+        open_lane = hl >= 0 && !all;
     }
-    return for_each_sample(a, b, c, d, [&](V3<double> s) {
-        return !in_envelope_list<true>(lst, tri, nl, s, eps2, sqrtT, hl);
-    });
+    if (open_lane) {
+        SampleGen g;
+        g.init(ld3(t9), ld3(t9 + 3), ld3(t9 + 6), d);
+        V3<double> s;
+        g.next(s);  // the first corner
+        while (g.next(s)) {
+            bool sure;
+            if (!in_envelope_cert(W, lst, cert, nl, mk, s, F, eps2, hl, sure)) {
+                out = true;
+                break;
+            }
+            if (sure && F.runs) {
+                const int64_t left = g.run_left(INT64_MAX);
+                if (left > 0 && cert_class(cert + kCertFloats * hl, cert_local(F, g.run_at(left)), F) > 0)
+                    g.k += (int)left;
+            }
+        }
+    }
+    return out;
 }
 
 // LDS of face_out_wave per wave: a triangle's segment record and header
