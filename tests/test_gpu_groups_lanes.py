@@ -61,7 +61,8 @@ def test_group_sizes(size):
 
 
 @pytest.mark.parametrize("n,lo,hi", [(1, 1, 6), (63, 4, 4), (64, 4, 4), (65, 4, 4), (257, 0, 9), (900, 2, 6),
-                                     (70, 28, 36), (40, 60, 70)])
+                                     (64, 40, 40), (70, 36, 44), (40, 60, 70), (300000, 4, 4), (270001, 5, 5),
+                                     (300001, 0, 8)])
 @pytest.mark.parametrize("extra", [0, 1])
 def test_groups_of_a_wave(n, lo, hi, extra):
     """Waves whose groups just fill their LDS, miss it by one tet, straddle the
@@ -81,7 +82,7 @@ def test_groups_of_a_wave(n, lo, hi, extra):
     T = tets[r.integers(0, len(tets), off[-1])].copy()
     flip = r.random(len(T)) < 0.3 / max(hi, 1)
     T[flip] = T[flip][:, [0, 1, 3, 2]]
-    flat = r.random(len(T)) < 0.1 / max(hi, 1)
+    flat = r.random(len(T)) < min(0.1, 20 / n) / max(hi, 1)
     T[flat, 3] = T[flat, 2]
     dev = [torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0") for a in (T, off, x, y, z)]
     fl, mq, q = (t.cpu().numpy() for t in ctx.tet_groups(*dev))

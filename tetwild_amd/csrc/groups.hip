@@ -11,8 +11,8 @@
 // by FP64 arithmetic where neighbours share vertices.  One lane per group runs
 // the chain once per tet; eight lanes per group leave half of them idle on four
 // tets.  us a call with one lane, eight, and this: 150 k groups of 2..6 tets of a
-// lattice at random 54, 28, 29; 2.5 M of four 673, 360, 330; 2.5 M of four in the
-// lattice's order 115, 290, 118; 300 k of 20 1443, 258, 103.  (The next ids read
+// lattice at random 54, 28, 29; 2.5 M of four 673, 358, 327; 2.5 M of four in the
+// lattice's order 120, 298, 124; 300 k of 20 1450, 258, 97.  (The next ids read
 // before a tet's arithmetic: 133 -> 118 in order, 317 -> 330 at random.)
 // Orientation comes from the floating-point filter; a group with no tet certainly
 // flipped but some tet undecided is marked and finished by a second pass with the
@@ -127,8 +127,10 @@ __device__ __forceinline__ void group_out(const GroupArgs& A, int64_t g, uint8_t
 
 // lanes per group where groups are taken one by one
 constexpr int kGroupLanes = 8;
-// tets a wave takes at once
-constexpr int kWaveTets = 256;
+// tets a wave takes at once: four rounds and, with groups of mixed sizes, a fourth
+// more (64 groups of 2..6 pass 256 every other time, and those waves take three
+// times as long)
+constexpr int kWaveTets = 320;
 
 // group g by eight lanes, eight tets a round (g < 0: none); the wave calls it
 __device__ void group_by_lanes(const GroupArgs& A, int64_t g)
@@ -254,9 +256,12 @@ extern "C" int twg_tet_groups(twg_ctx* ctx, const int32_t* tets, const int32_t* 
     A.flipped = flipped;
     A.max_q = max_q;
     A.q = q;
-    // as many groups a wave as leave its tets, at the batch's mean, within its LDS
+    // as many groups a wave as leave four rounds of tets, at the batch's mean, and
+    // 16 waves a CU (which holds 20): 150 k groups of 2..6 22.4, 22.3, 21.5 us with
+    // 8, 16, 32 a wave; 2.5 M of 4 in order 169, 150, 140 with
+    // 16, 32, 64 (124 since)
     int gw = 8;
-    while (gw < 64 && 2 * gw * n_tets <= kWaveTets * n_groups) gw *= 2;
+    while (gw < 64 && 2 * gw * n_tets <= 256 * n_groups && n_groups >= (int64_t)32 * gw * ctx->num_cus) gw *= 2;
     const int64_t per = gw * (kBlock / 64);
     const unsigned gm = (unsigned)std::min<int64_t>((n_groups + per - 1) / per, 1 << 20);
     hipLaunchKernelGGL(groups_kernel, dim3(gm), dim3(kBlock), 0, ctx->cur, A, gw);
