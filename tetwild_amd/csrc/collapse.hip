@@ -323,19 +323,17 @@ __device__ void ring_candidate(const CollapseArgs& A, int64_t c, int tl, int wba
 // the better.  (Persistent tiles popping candidates from one atomic counter
 // ran at the counter's rate, ~6 ns per pop: 200k candidates of 24-tet rings,
 // chunk 1: 1446 us for the whole batch, 360 us this way.)  A launch holds fewer
-// than 2^32 threads, 2^26 candidates on 64-lane tiles: from kRingBlocks blocks on
-// a tile takes more than one chunk.
+// than 2^32 threads, 2^26 candidates on 64-lane tiles: larger batches take
+// several of kRingBlocks blocks, from block `base` on.
 constexpr int64_t kRingBlocks = 1 << 22;
 template <int TILE>
-__global__ __launch_bounds__(kBlock) void collapse_ring_kernel(CollapseArgs A)
+__global__ __launch_bounds__(kBlock) void collapse_ring_kernel(CollapseArgs A, int64_t base)
 {
     const int tl = threadIdx.x % TILE;
     const int wbase = (threadIdx.x % 64) - tl;
-    const int64_t step = (int64_t)gridDim.x * (kBlock / TILE) * A.chunk;
-    for (int64_t c0 = (xcd_block() * (int64_t)(kBlock / TILE) + threadIdx.x / TILE) * A.chunk; c0 < A.n; c0 += step) {
-        const int64_t c1 = c0 + A.chunk < A.n ? c0 + A.chunk : A.n;
-        for (int64_t c = c0; c < c1; ++c) ring_candidate<TILE, false>(A, c, tl, wbase);
-    }
+    const int64_t c0 = ((base + xcd_block()) * (int64_t)(kBlock / TILE) + threadIdx.x / TILE) * A.chunk;
+    const int64_t c1 = c0 + A.chunk < A.n ? c0 + A.chunk : A.n;
+    for (int64_t c = c0; c < c1; ++c) ring_candidate<TILE, false>(A, c, tl, wbase);
 }
 
 // the candidates the filter pass listed, with the exact predicate; a tile per
@@ -553,29 +551,35 @@ void bind_scratch(CollapseArgs& A, void* base)
     A.exact_list = reinterpret_cast<int32_t*>(b + w + t + 256);
 }
 
-using RingFn = void (*)(CollapseArgs);
+using RingFn = void (*)(CollapseArgs, int64_t);
+using RingExactFn = void (*)(CollapseArgs);
 
-RingFn ring_fn(int tile, bool exact)
+RingFn ring_fn(int tile)
 {
-    if (tile == 16) return exact ? collapse_ring_exact_kernel<16> : collapse_ring_kernel<16>;
-    if (tile == 32) return exact ? collapse_ring_exact_kernel<32> : collapse_ring_kernel<32>;
-    return exact ? collapse_ring_exact_kernel<64> : collapse_ring_kernel<64>;
+    return tile == 16 ? collapse_ring_kernel<16> : (tile == 32 ? collapse_ring_kernel<32> : collapse_ring_kernel<64>);
+}
+RingExactFn ring_exact_fn(int tile)
+{
+    return tile == 16 ? collapse_ring_exact_kernel<16>
+                      : (tile == 32 ? collapse_ring_exact_kernel<32> : collapse_ring_exact_kernel<64>);
 }
 
 // every launch of one batch, in order, on stream s (graph-capturable: the
 // list's length is cleared by a kernel)
 int enqueue(twg_ctx* ctx, const CollapseArgs& A, int tile, bool f32, hipStream_t s)
 {
-    RingFn ring = ring_fn(tile, false);
     const int64_t per = (int64_t)(kBlock / tile) * A.chunk;  // candidates per block
-    const unsigned gring = (unsigned)std::min<int64_t>((A.n + per - 1) / per, kRingBlocks);
+    const int64_t blocks = (A.n + per - 1) / per;
     const int64_t need = (A.n * tile + kBlock - 1) / kBlock;
     const unsigned gexact = (unsigned)std::min<int64_t>(std::max<int64_t>(need, 1), 2048);
     hipLaunchKernelGGL(reset_list, dim3(1), dim3(1), 0, s, A.counter);
     TWG_LAUNCHED();
-    hipLaunchKernelGGL(ring, dim3(gring), dim3(kBlock), 0, s, A);
-    TWG_LAUNCHED();
-    hipLaunchKernelGGL(ring_fn(tile, true), dim3(gexact), dim3(kBlock), 0, s, A);
+    for (int64_t at = 0; at < blocks; at += kRingBlocks) {
+        const dim3 g((unsigned)std::min<int64_t>(blocks - at, kRingBlocks));
+        hipLaunchKernelGGL(ring_fn(tile), g, dim3(kBlock), 0, s, A, at);
+        TWG_LAUNCHED();
+    }
+    hipLaunchKernelGGL(ring_exact_fn(tile), dim3(gexact), dim3(kBlock), 0, s, A);
     TWG_LAUNCHED();
     if (A.has_sf || A.has_bt) {
         if (f32) hipLaunchKernelGGL(collapse_point_kernel<true>, dim3(grid_for(A.n)), dim3(kBlock), 0, s, A);
