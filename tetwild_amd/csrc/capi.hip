@@ -31,18 +31,21 @@ int bind(twg_ctx* ctx)
     return TWG_OK;
 }
 
+bool capturing(twg_ctx* ctx)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->cur, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Memory of at least `bytes` in block m.  A block that a captured graph may
 // hold the address of is never freed while the context lives.
 static int ensure(twg_ctx* ctx, twg_ctx::Block& m, size_t bytes)
 {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->cur, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        cap = hipStreamCaptureStatusActive;  // the null stream beside a capturing one
-    }
-    const bool capturing = cap != hipStreamCaptureStatusNone;
+    const bool graph = capturing(ctx);
     if (bytes > m.bytes) {
-        if (m.p && (m.in_graph || capturing)) {
+        if (m.p && (m.in_graph || graph)) {
             twg_ctx::Retired* r = new (std::nothrow) twg_ctx::Retired{m.p, ctx->retired};
             if (!r) {
                 set_error("out of host memory");
@@ -58,7 +61,7 @@ static int ensure(twg_ctx* ctx, twg_ctx::Block& m, size_t bytes)
         TWG_HIP(hipMalloc(&m.p, want));
         m.bytes = want;
     }
-    m.in_graph = m.in_graph || capturing;
+    m.in_graph = m.in_graph || graph;
     return TWG_OK;
 }
 

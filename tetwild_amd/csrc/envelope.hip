@@ -491,8 +491,12 @@ constexpr int64_t kPointListDensity = 2;
 // sure of the walk's result -- far queries, ties -- the walk runs: in the group
 // itself for small batches, which have the lanes (4,096 far points 11 -> 2.2
 // ms, 65 k 10.5 -> 14.7), else by nearest_rest_kernel, a point per lane.
-// 4,096 points 2951 -> 37 us, 1 M 10.5 -> 3.7 ms.  (8, 16 and 64 lanes a
-// point: 65, 45 and 35 us for 4,096, 6.6, 4.7 and 5.7 ms for 1 M.)
+// Points near the surface, 4,096 of them 2850 -> 39 us, 1 M 10.5 -> 3.0 ms.  A
+// third of a radius off it (and seven tenths, deep inside) the group's lists are
+// in vain: 40 k 10.8 -> 11.0 ms (78 -> 80), 300 k on 512 k facets 21.6 -> 25.2 (171
+// -> 195), but 1 M in order 41.6 -> 31.8 (303 -> 234).  (8, 16 and 64 lanes a point
+// before the order: 65, 45 and 35 us for 4,096, 6.6, 4.7 and 5.7 ms for 1 M,
+// against 37 us and 3.7 ms.)
 constexpr int kNearestGroup = 32;
 constexpr int kNearestCap = 64;  // facets listed per group
 constexpr int64_t kNearestWalkMax = 1 << 15;
@@ -653,7 +657,8 @@ using namespace twg;
 
 // Surfaces from this size on are built on the device (build.hip), smaller ones
 // on the host: 64 facets take 59 us on the host and 169 on the device, 512 take
-// 187 and 180, 5,120 take 2.0 ms and 0.32, 246,420 take 121 ms and 0.96.
+// 187 and 180, 5,120 take 2.0 ms and 0.32, 246,420 take 121 ms and 0.96.  The host
+// also builds those whose working memory the device does not have.
 constexpr int64_t kDeviceBuildMin = 512;
 
 extern "C" {
@@ -664,17 +669,21 @@ int twg_bvh_build(twg_ctx* ctx, const double* V, int64_t nv, const int32_t* F, i
     TWG_REQUIRE(ctx && out, "twg_bvh_build: NULL argument");
     TWG_REQUIRE(nf >= 1 && nv >= 1 && V && F, "twg_bvh_build: empty surface");
     TWG_REQUIRE(nf < (int64_t(1) << 30), "twg_bvh_build: too many facets (%lld)", (long long)nf);
+    if (int r = bind(ctx)) return r;
     if (nf >= kDeviceBuildMin && nv < (int64_t(1) << 31)) {
-        if (int r = bind(ctx)) return r;
         std::unique_ptr<twg_bvh, int (*)(twg_bvh*)> B(new twg_bvh(), twg_bvh_destroy);
         B->device = ctx->device;
         B->nf = nf;
         int64_t bad = -1;
-        if (int r = bvh_build_device(ctx, V, nv, F, nf, B.get(), &bad)) return r;
-        TWG_REQUIRE(bad < 0, "twg_bvh_build: facet %lld has vertex id %d outside [0, %lld)",
-                    (long long)(bad / 3), F[bad], (long long)nv);
-        *out = B.release();
-        return TWG_OK;
+        const int r = bvh_build_device(ctx, V, nv, F, nf, B.get(), &bad);
+        if (r && r != TWG_ENOMEM) return r;
+        if (!r) {
+            TWG_REQUIRE(bad < 0, "twg_bvh_build: facet %lld has vertex id %d outside [0, %lld)",
+                        (long long)(bad / 3), F[bad], (long long)nv);
+            *out = B.release();
+            return TWG_OK;
+        }
+        (void)hipGetLastError();
     }
     for (int64_t f = 0; f < 3 * nf; ++f)
         TWG_REQUIRE(F[f] >= 0 && F[f] < nv, "twg_bvh_build: facet %lld has vertex id %d outside [0, %lld)",
@@ -952,14 +961,13 @@ int twg_nearest_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_t
     const dim3 b(kBlock);
     BvhView v = bvh_view(B);
     const int32_t* order = nullptr;
-    // (no ordering memory for a captured graph: it walks the points as they come)
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->cur, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        cap = hipStreamCaptureStatusActive;
+    // (a captured graph walks the points as they come, and so does a call that
+    // finds no memory for their order)
+    if (n >= kSortMin && n < (int64_t(1) << 31) && !capturing(ctx)) {
+        const int r = morton_order(ctx, 2, p3, n, 3, B, &order);
+        if (r && r != TWG_ENOMEM) return r;
+        if (r) (void)hipGetLastError();
     }
-    if (cap == hipStreamCaptureStatusNone && n >= kSortMin && n < (int64_t(1) << 31))
-        if (int r = morton_order(ctx, 2, p3, n, 3, B, &order)) return r;
     constexpr int64_t kPart = 1 << 26;  // a launch holds fewer than 2^32 threads
     for (int64_t at = 0; at < n; at += kPart) {
         const dim3 g(grid_for(std::min(n - at, kPart) * kNearestGroup));
@@ -971,7 +979,9 @@ int twg_nearest_points(twg_ctx* ctx, const twg_bvh* B, const double* p3, int64_t
     }
     if (n < kNearestWalkMax) return TWG_OK;
     // (walks far from the surface gain nothing from the order below some 250 k
-    // points: 65 k 10.5 ms without and 12.1 with it, 1 M 41 and 30)
+    // points: 65 k 10.5 ms without and 12.1 with it, 1 M 44 and 31.  At 300 k it
+    // depends: a third of a radius outside 246 k facets 15.9 and 16.3, a tenth
+    // inside 11.2 and 9.1, outside 5 k facets 3.1 and 2.2)
     hipLaunchKernelGGL(nearest_rest_kernel, dim3(grid_for(n)), b, 0, ctx->cur, v, p3, n, cp3, d2, facet,
                        n < (1 << 18) ? nullptr : order);
     TWG_LAUNCHED();

@@ -1160,9 +1160,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 // instead of 35, which 96 % of the benchmark's rings fit against 73 %; 5.89
 // -> 5.79 ms on its 200k batch.)  The 32-lane pass leaves the envelope stage
 // out of its code, which spares the whole kernel 96 spilled registers: 60 k
-// problems, a fifth of them surface, 1921 -> 1588 us.  Two launches, one per
-// kind, lose more in the tail between them than the others gain from three or
-// four waves a SIMD (1945 us at two waves, 2035 and 2242 at three and four).
+// problems, a fifth of them surface, took 1745 us before the face test's
+// certificates, 1921 with them and the stage in both passes, and take 1645 this
+// way.  Two launches, one per kind, lose more in the tail between them than the
+// others gain from three or four waves a SIMD (1945 us at two waves, 2035 and
+// 2242 at three and four; this, timed with them, 1588).
 __device__ __forceinline__ bool surface_kind(const SmoothArgs& A, int64_t p)
 {
     const int k = A.kind ? A.kind[p] : 0;

@@ -60,6 +60,10 @@ void set_error(const char* fmt, ...);
 // returns nonzero (TWG_EDEVICE) and records the message on failure
 int hip_fail(hipError_t e, const char* what, const char* file, int line);
 
+// Whether the context's stream captures a graph (or cannot be asked: the null
+// stream beside a capturing one).
+bool capturing(twg_ctx* ctx);
+
 int ensure_scratch(twg_ctx* ctx, size_t bytes);
 int ensure_slot(twg_ctx* ctx, int i, size_t bytes);
 
