@@ -453,9 +453,9 @@ def bench_envelope(ctx, args, result, surf_cache):
     # counted traffic over the HIP-event time of the whole call (Morton
     # ordering included); its FP64 lane-FLOP rate
     kern64 = rates["fp64"][1]
-    rl = {"bound": "latency (dependent box / facet reads)", "kernel": "faces_list_kernel<80>",
+    rl = {"bound": "latency (dependent box / facet reads)", "kernel": "faces_list_kernel<false, 80>",
           "avg_launch_ms": kern64 * 1e3, "unit": "GB/s", "peak": HBM_PEAK_GBS}
-    rl.update(counted_roofline(counters("faces_list_kernel<80>"), kern64))
+    rl.update(counted_roofline(counters("faces_list_kernel<false, 80>"), kern64))
     if "hbm_side_gbs" in rl:
         rl["achieved"] = rl["hbm_side_gbs"]
         rl["frac"] = rl["achieved"] / HBM_PEAK_GBS
