@@ -474,9 +474,12 @@ constexpr int64_t kWaveMax = 1 << 16;
 // 2153, so sparser batches keep faces_kernel.  So do wide envelopes (reach_wide),
 // and below kWideDensity queries a facet those 2.5 times less wide: eps two facets,
 // 2 M triangles (8 a facet) 4156 us without lists and 4356 with them; eps one
-// facet, 560 k (2.3) 1372 and 1779, 2 M (8) 3509 and 3478.
+// facet, 560 k (2.3) 1372 and 1779, 2 M (8) 3509 and 3478.  On graded surfaces
+// (morton_refined) a wave's queries lie further apart in facets: 72 k facets
+// shrinking tenfold, 160 k triangles (2.2) 464 and 558, 290 k (4) 591 and 503, so
+// those start at kGradedDensity.
 constexpr int kFaceListCap = 80;
-constexpr int64_t kFaceListDensity = 2, kWideDensity = 8;
+constexpr int64_t kFaceListDensity = 2, kGradedDensity = 3, kWideDensity = 8;
 // the same for points_list_kernel: 1 M points on 246 k facets (4 a facet) 593
 // -> 576 us, 4 M on 72 k (56) 980 -> 829, but 300 k on 512 k (0.6) 418 -> 822;
 // eps three facets, 1 M points (4 a facet) 1562 us without lists and 1774 with
@@ -905,7 +908,8 @@ int twg_envelope_faces(twg_ctx* ctx, const twg_bvh* B, const double* tri9, int64
     hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, ctx->cur, n_pending);
     TWG_LAUNCHED();
     const bool wide = reach_wide(B, (n < kWideDensity * B->nf ? 5.0 : 2.0) * sT);
-    if (order && !stats && !wide && n >= kFaceListDensity * B->nf) {
+    const int64_t density = morton_refined(B, n) ? kGradedDensity : kFaceListDensity;
+    if (order && !stats && !wide && n >= density * B->nf) {
         if (precision == TWG_FP64)
             hipLaunchKernelGGL((faces_list_kernel<false, kFaceListCap>), dim3(4 * grid_for(n)), dim3(64), 0, ctx->cur, v, tri9, n, eps2, sampling_dist, T, sT, out, n_pending, pending, order, ctx->list_stats_on ? ctx->list_stats : nullptr);
         else

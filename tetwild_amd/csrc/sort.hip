@@ -279,13 +279,16 @@ int sort_pairs(ulonglong2* kv[2], int64_t n, int bits, void* work, hipStream_t s
 // wave's queries overflow its list, 8452 and 10780 us a call, with 36 and 45 bits
 // 1414 and 1484.)
 constexpr int64_t kCrowdShare = 64;
+static int default_passes(int64_t n) { return n < kTwoPassMax ? 2 : 3; }
 static int morton_bits(const twg_bvh* B, int64_t n)
 {
     constexpr int kLevels = kDigitBits / 3;  // a pass
-    int passes = n < kTwoPassMax ? 2 : 3;
+    int passes = default_passes(n);
     while (passes * kLevels < kCrowdLevels - 1 && B->crowded[0][passes * kLevels] * kCrowdShare > B->nf) ++passes;
     return passes * kDigitBits;
 }
+
+bool morton_refined(const twg_bvh* B, int64_t n) { return morton_bits(B, n) > default_passes(n) * kDigitBits; }
 
 // KV: a (key, item) pair that holds the key's bits
 template <class KV>

@@ -74,6 +74,9 @@ int ensure_slot(twg_ctx* ctx, int i, size_t bytes);
 int morton_order(twg_ctx* ctx, int slot, const double* items, int64_t n, int stride, const twg_bvh* B,
                  const int32_t** order);
 
+// Whether that order takes more bits than its size asks for: the surface is graded.
+bool morton_refined(const twg_bvh* B, int64_t n);
+
 // Stable sort of n (key, value) pairs by the low `bits` bits of their keys:
 // kv[0] in and, after the call, out; kv[1] as large; work: sort_pairs_bytes(n).
 size_t sort_pairs_bytes(int64_t n);
